@@ -11,7 +11,7 @@
 // big kernel when the output allows 16-byte stores, a transpose through LDS into
 // whole 128-byte lines per row.
 //
-// Two kernels:
+// Three kernels:
 //  * gemm_bf16_nt_big_kernel<TM, TN> (K >= 64; a last partial k-slab is zero-filled): (64 TM) x (128 TN) x 64 tiles,
 //    8 waves (2 x 4, two per SIMD), each wave (32 TM) x (32 TN): 128/192/256/320 x 256
 //    (TN = 2) chosen per problem so that the tile count wastes the fewest workgroup
@@ -26,14 +26,17 @@
 //    operand's size, so tile rows past M or N read as zeros.  Fragments are
 //    double-buffered in registers; the next k-step's LDS reads are issued
 //    between the two halves of the current step's MFMAs.
-//  * gemm_bf16_nt_kernel (any K % 8 == 0): 128 x 128 x 64 tiles, 4 waves,
-//    register-staged loads into padded LDS; the general fallback.
+//  * gemm_bf16_nt_ksplit_kernel<MT, NT> (at most 256 rows, or too few columns for the big
+//    tiles): (32 MT) x (32 NT) tiles whose four waves share the inner dimension.
+//  * gemm_bf16_nt_kernel (K > 2^24, where a tile's rows outgrow 32-bit offsets): 128 x 128 x 64
+//    tiles, 4 waves, register-staged loads into padded LDS, 64-bit addresses.
 // Workgroups walk the tile list with stride gridDim.x (grid cap = compute-unit
 // budget of the weave schedule), and tile ids are remapped so that the
 // workgroups of one XCD (blockIdx % 8) share operand panels in that XCD's L2.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "tw_common.h"
@@ -192,13 +195,202 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_bf16_nt_kernel(
   }
 }
 
+// `count` independent products of one shape in one launch: out[p] = a[p] * b[p]^T.  The
+// token-weave producer uses it for the P row-parallel partial sums of a token split,
+// each written into its rank's staging slot; a plain GEMM is count = 1.
+struct GemmBatch {
+  uint16_t* out[TW_MAX_PARTIALS];
+  const uint16_t* a[TW_MAX_PARTIALS];
+  const uint16_t* b[TW_MAX_PARTIALS];
+  const uint16_t* bias[TW_MAX_PARTIALS];  // [N] bf16 or null: added to that product only
+};
+
+// ---------------------------------------------------------------------------
+// K-split kernel: few rows (a decode step, a short prefill chunk).  The product is bound by
+// reading b once, so what counts is how many compute units stream it and how evenly.
+//
+// A workgroup owns (32 MT) x (at most 32 NT) of the output and its four waves share the inner
+// dimension: wave w takes the 64-wide k-slabs w, w + 4, ... .  Each wave brings its slabs of
+// both operands from global memory straight into LDS of its own, STAGES slabs deep, and
+// reads its fragments back from there: no barrier in the k loop, a wave only waits for its own
+// loads.  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
+// Every load covers whole 128-byte lines of eight rows.  The sum of an output element does not
+// depend on the tile it lies in (nor on MT, NT, the grid or the number of products).
+//
+// The launcher makes the tiles just wide enough for one (or a whole number of) workgroups per
+// compute unit: 32 columns at N = 8192, 24 at N = 6144.  Measured on 256 units, operands
+// rotated through 2 GB / through three sets: [32, 3584] x [8192, 3584]^T 13.9 / 10.6 us
+// (59 MB: 4.3 / 5.6 TB/s) against 65 / 47 us with 64 workgroups of 128 x 128; K = 1024: 6.0 / 5.0 us
+// against 16 us; [128, 3584]: 21 / 15 us against 69 / 50 us.
+// ---------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+constexpr int KS_WAVES = 4;
+constexpr int KS_THREADS = KS_WAVES * 64;
+constexpr int KS_ROWB = 128;                      // bytes of a slab row: 64 elements
+constexpr uint32_t KS_OUT_OF_RANGE = 0x80000000u; // a tile's rows span at most 2 GiB (KS_MAX_K)
+constexpr int64_t KS_MAX_K = 1 << 24;
+
+constexpr int ks_lds_bytes(int mt, int nt, int stages) {
+  const int slabs = KS_WAVES * stages * 32 * (mt + nt) * KS_ROWB;
+  const int sums = KS_WAVES * 32 * mt * (32 * nt * 4 + 16);
+  return slabs > sums ? slabs : sums;
+}
+
+// One operand's share of a slab, 8 rows per wave instruction; `tail`: the last slab of an inner
+// dimension that is no multiple of 64, whose chunks past K must arrive as zeros (`even` / `odd`
+// say whether this lane's chunk of an even / odd 8-row block is inside).
+template <int L>
+__device__ __forceinline__ void ks_issue(__amdgpu_buffer_rsrc_t d, const uint32_t (&v)[L], uint8_t* s, uint32_t koff,
+                                         bool tail, bool even, bool odd) {
+  if (tail) {
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_void_t*)(s + j * 1024), 16,
+                                               ((j & 1) ? odd : even) ? v[j] : KS_OUT_OF_RANGE, koff, 0, 0);
+  } else {
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_void_t*)(s + j * 1024), 16, v[j], koff, 0, 0);
+  }
+}
+
+template <int MT, int NT, int STAGES>
+__global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
+    GemmBatch batch, int count, int M, int N, int K, int64_t ldc, int tiles_m, int tiles_n, int cols) {
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass only needs the stub, and cannot instantiate the device builtins
+  constexpr int RA = 32 * MT, RB = 32 * NT, LA = RA / 8, LB = RB / 8;
+  constexpr int STAGE = (RA + RB) * KS_ROWB;
+  static_assert(STAGES == 2, "the k loop waits for one slab beside the one in use");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds_ks[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, lhi = lane >> 5;
+  const int nk = (K + BK - 1) / BK;
+  const int tail_chunks = (K % BK) / 8;
+  const bool even = ((lane & 7) ^ (lane >> 4)) < tail_chunks;
+  const bool odd = ((lane & 7) ^ (lane >> 4) ^ 4) < tail_chunks;
+  // Row r of a slab keeps its 16-byte chunk c at position c ^ ((r >> 1) & 7) (see the file
+  // comment).  Offsets are inside the tile: its descriptors begin at its first row and end
+  // behind its last one, so that rows past M, N or the tile's columns read as zeros.
+  uint32_t va[LA], vb[LB], roff[4];
+#pragma unroll
+  for (int j = 0; j < (LA > LB ? LA : LB); ++j) {
+    const int chunk = (lane & 7) ^ (((j & 1) << 2) | (lane >> 4));
+    const uint32_t v = (uint32_t)((j * 8 + (lane >> 3)) * (int64_t)K + chunk * 8) * 2u;
+    if (j < LA) va[j] = v;
+    if (j < LB) vb[j] = v;
+  }
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) roff[kk] = l32 * KS_ROWB + ((((kk << 1) | lhi) ^ ((l32 >> 1) & 7)) << 4);
+  uint8_t* const mine = lds_ks + wave * (STAGES * STAGE);
+
+  const int tiles_per_product = tiles_m * tiles_n;
+  const int num_tiles = count * tiles_per_product;
+  for (int t = blockIdx.x; t < num_tiles; t += gridDim.x) {
+    // Every XCD a contiguous range of tiles, the row tiles of one column range next to each other:
+    // they read the same rows of b through one L2.
+    int pid = t;
+    const int per_xcd = num_tiles / 8;
+    if (t < per_xcd * 8) pid = (t & 7) * per_xcd + (t >> 3);
+    const int product = pid / tiles_per_product;
+    pid -= product * tiles_per_product;
+    const int m0 = (pid % tiles_m) * RA, n0 = (pid / tiles_m) * cols;
+    const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(batch.a[product]) + (size_t)m0 * K, 0, (uint32_t)min(M - m0, RA) * (uint32_t)K * 2u, 0x00020000);
+    const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(batch.b[product]) + (size_t)n0 * K, 0, (uint32_t)min(N - n0, cols) * (uint32_t)K * 2u, 0x00020000);
+
+    f32x16_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+    // slabs `wave`, wave + 4, ...; b first: it is the operand that comes from far
+    int slab = wave;
+    if (slab < nk) {
+      const bool tail = tail_chunks && slab == nk - 1;
+      ks_issue<LB>(db, vb, mine + RA * KS_ROWB, (uint32_t)slab * KS_ROWB, tail, even, odd);
+      ks_issue<LA>(da, va, mine, (uint32_t)slab * KS_ROWB, tail, even, odd);
+    }
+    for (int stage = 0; slab < nk; slab += KS_WAVES, stage ^= 1) {
+      const int next = slab + KS_WAVES;
+      if (next < nk) {
+        uint8_t* s = mine + (stage ^ 1) * STAGE;
+        const bool tail = tail_chunks && next == nk - 1;
+        ks_issue<LB>(db, vb, s + RA * KS_ROWB, (uint32_t)next * KS_ROWB, tail, even, odd);
+        ks_issue<LA>(da, va, s, (uint32_t)next * KS_ROWB, tail, even, odd);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + LB) : "memory");  // all but the loads just issued
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      const uint8_t* pa = mine + stage * STAGE;
+      const uint8_t* pb = pa + RA * KS_ROWB;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        bf16x8_t fa[MT], fb[NT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          fa[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(pa + i * 32 * KS_ROWB + roff[kk]));
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          fb[j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(pb + j * 32 * KS_ROWB + roff[kk]));
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+      }
+      // the fragments are in registers: the loads issued next may overwrite this stage
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+
+    // acc[i][j][4 q + e] = partial sum of out[m0 + i*32 + l32][n0 + j*32 + 8 q + 4 lhi + e].
+    // The slab stages become the four waves' fp32 tiles (rows padded by 16 bytes).
+    constexpr int PITCH = RB * 4 + 16;
+    __syncthreads();
+    uint8_t* const sums = lds_ks + wave * (RA * PITCH);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<f32x4_t*>(sums + (i * 32 + l32) * PITCH + (j * 32 + 8 * q + 4 * lhi) * 4) =
+              f32x4_t{acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    __syncthreads();
+    uint16_t* __restrict__ out = batch.out[product];
+    const uint16_t* __restrict__ bias = batch.bias[product];
+    for (int g = tid; g < RA * RB / 4; g += KS_THREADS) {
+      const int m = g / (RB / 4), c = (g % (RB / 4)) * 4;
+      if (m0 + m < M && c < cols && n0 + c < N) {  // N and cols are multiples of 4
+        const uint8_t* p = lds_ks + m * PITCH + c * 4;
+        f32x4_t s = *reinterpret_cast<const f32x4_t*>(p);
+#pragma unroll
+        for (int w = 1; w < KS_WAVES; ++w) s += *reinterpret_cast<const f32x4_t*>(p + w * (RA * PITCH));
+        uint2 v = {pack2(s.x, s.y), pack2(s.z, s.w)};
+        if (bias) {
+          const uint2 bv = *reinterpret_cast<const uint2*>(bias + n0 + c);
+          v.x = add_bias2(v.x, bv.x);
+          v.y = add_bias2(v.y, bv.y);
+        }
+        *reinterpret_cast<uint2*>(out + (size_t)(m0 + m) * ldc + n0 + c) = v;
+      }
+    }
+    __syncthreads();  // the next tile's slabs overwrite the sums
+  }
+#endif
+}
+
 // ---------------------------------------------------------------------------
 // (32 TM x 2) x 256 x 64 tiles, direct-to-LDS operand slabs (see the file
 // comment).  TM = 32-row MFMA tiles per wave along M: 4 -> 256-row tiles,
 // 5 -> 320-row tiles, 3 -> 192-row tiles.  The launcher picks the height that
 // wastes the fewest workgroup rounds for the given M.
 // ---------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void lds_void_t;
 constexpr int BIG_BK = 64;
 constexpr int BIG_THREADS = 512;
 constexpr int BIG_ROWB = BIG_BK * 2;             // bytes per LDS row
@@ -246,16 +438,6 @@ __device__ __forceinline__ void big_issue_slab_tail(__amdgpu_buffer_rsrc_t da, _
                                              0, 0);
   }
 }
-
-// `count` independent products of one shape in one launch: out[p] = a[p] * b[p]^T.  The
-// token-weave producer uses it for the P row-parallel partial sums of a token split,
-// each written into its rank's staging slot; a plain GEMM is count = 1.
-struct GemmBatch {
-  uint16_t* out[TW_MAX_PARTIALS];
-  const uint16_t* a[TW_MAX_PARTIALS];
-  const uint16_t* b[TW_MAX_PARTIALS];
-  const uint16_t* bias[TW_MAX_PARTIALS];  // [N] bf16 or null: added to that product only
-};
 
 template <int TM, int TN>
 __global__ __launch_bounds__(BIG_THREADS) void gemm_bf16_nt_big_kernel(
@@ -526,23 +708,61 @@ __global__ __launch_bounds__(BIG_THREADS) void gemm_bf16_nt_big_kernel(
   }
 }
 
+// More than 64 KiB of dynamic LDS must be allowed once per function and device.
+static int allow_lds(const void* kernel, std::atomic<bool>* ok, int max_devices, int bytes) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= max_devices)
+    return set_error(TW_ERR_LAUNCH, "gemm_bf16_nt: no current device");
+  if (!ok[dev].load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
+      return set_error(TW_ERR_LAUNCH, "gemm_bf16_nt: the device refused %d bytes of LDS", bytes);
+    ok[dev].store(true, std::memory_order_release);
+  }
+  return TW_OK;
+}
+constexpr int kMaxDevices = 64;
+
+template <int MT, int NT>
+static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc, int max_cus,
+                         hipStream_t hs) {
+  constexpr int STAGES = 2, LDS = ks_lds_bytes(MT, NT, STAGES);
+  static std::atomic<bool> lds_ok[kMaxDevices];
+  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES>), lds_ok, kMaxDevices,
+                         LDS))
+    return rc;
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  // Columns per workgroup: as few rounds of one workgroup per unit as full-width tiles need, and
+  // then tiles no wider than that many rounds require, so that every unit streams its share of b.
+  const int64_t tiles_m = (M + 32 * MT - 1) / (32 * MT), full = (N + 32 * NT - 1) / (32 * NT);
+  const int64_t rounds = (tiles_m * full + cus - 1) / cus;
+  const int64_t per_row_tile = std::max(full, cus * rounds / tiles_m);  // column tiles those rounds have room for
+  const int cols = (int)std::min<int64_t>(32 * NT, ((N + per_row_tile - 1) / per_row_tile + 3) / 4 * 4);
+  const int64_t tiles_n = (N + cols - 1) / cols;
+  int64_t grid = count * tiles_m * tiles_n;
+  if (max_cus > 0 && grid > max_cus) grid = max_cus;
+  launch_kernel(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES>, dim3((unsigned)grid), dim3(KS_THREADS), LDS, hs, batch, count,
+                (int)M, (int)N, (int)K, ldc, (int)tiles_m, (int)tiles_n, cols);
+  return TW_OK;
+}
+
+// The rule looks at M, N and K alone: a product has the same bits under every grid cap and in
+// every batch.
+static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
+                             int max_cus, hipStream_t hs) {
+  if (M <= 32) return launch_ksplit<1, 1>(batch, count, M, N, K, ldc, max_cus, hs);
+  if (M <= 64) return launch_ksplit<2, 1>(batch, count, M, N, K, ldc, max_cus, hs);
+  return launch_ksplit<2, 2>(batch, count, M, N, K, ldc, max_cus, hs);
+}
+
 template <int TM, int TN>
 static int launch_big(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
                       int max_cus, hipStream_t hs) {
   constexpr int BM = 64 * TM, BN = 128 * TN;
   constexpr int LDS = big_lds_bytes(TM, TN);
-  // the attribute belongs to the function on one device: set it once per device
-  constexpr int kMaxDevices = 64;
   static std::atomic<bool> lds_ok[kMaxDevices];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
-    return set_error(TW_ERR_LAUNCH, "gemm_bf16_nt: no current device");
-  if (!lds_ok[dev].load(std::memory_order_acquire)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_nt_big_kernel<TM, TN>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
-      return set_error(TW_ERR_LAUNCH, "gemm_bf16_nt: the device refused %d bytes of LDS", LDS);
-    lds_ok[dev].store(true, std::memory_order_release);
-  }
+  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_big_kernel<TM, TN>), lds_ok, kMaxDevices, LDS))
+    return rc;
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
   int64_t grid = (int64_t)count * tiles_m * tiles_n;
   if (max_cus > 0 && grid > max_cus) grid = max_cus;
@@ -591,7 +811,7 @@ static bool big_kernel_fits(int64_t M, int64_t N, int64_t K) {
   // out-of-range marker when a last partial slab has to be zero-filled), and enough rows and
   // columns to be worth the larger prologue
   const uint64_t limit = (K % BIG_BK == 0) ? (1ull << 31) : (1ull << 30);  // elements per operand
-  return K >= BIG_BK && (uint64_t)M * K < limit && (uint64_t)N * K < limit && M >= 192 && N >= 192;
+  return K >= BIG_BK && (uint64_t)M * K < limit && (uint64_t)N * K < limit && M > 256 && N >= 192;
 }
 
 static int launch_big_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
@@ -624,35 +844,43 @@ static int check_gemm_pointers(const char* what, const void* out, const void* a,
   return TW_OK;
 }
 
+static int run_products(const char* what, const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K,
+                        int64_t ldc, int max_cus, hipStream_t hs) {
+  if (big_kernel_fits(M, N, K)) {
+    if (int rc = launch_big_for(batch, count, M, N, K, ldc, max_cus, hs)) return rc;
+    return finish_launch(what);
+  }
+  if (K <= KS_MAX_K) {
+    if (int rc = launch_ksplit_for(batch, count, M, N, K, ldc, max_cus, hs)) return rc;
+    return finish_launch(what);
+  }
+  const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
+  int64_t grid = (int64_t)tiles_m * tiles_n;
+  if (max_cus > 0 && grid > max_cus) grid = max_cus;
+  if (grid > INT32_MAX) grid = INT32_MAX;
+  for (int p = 0; p < count; ++p) {
+    launch_kernel(gemm_bf16_nt_kernel, dim3((unsigned)grid), dim3(GEMM_THREADS), 0, hs, batch.out[p], batch.a[p],
+                  batch.b[p], batch.bias[p], (int)M, (int)N, (int)K, ldc, tiles_m, tiles_n);
+    if (int rc = finish_launch(what)) return rc;
+  }
+  return TW_OK;
+}
+
 int run_gemm_bf16_nt(void* out, const void* a, const void* b, const void* bias, int64_t M, int64_t N,
                      int64_t K, int64_t ldc, int max_cus, void* stream) {
   if (int rc = check_gemm_shape("gemm_bf16_nt", M, N, K, ldc)) return rc;
   if (M == 0) return TW_OK;
   if (int rc = check_gemm_pointers("gemm_bf16_nt", out, a, b, bias)) return rc;
-  hipStream_t hs = static_cast<hipStream_t>(stream);
-  if (big_kernel_fits(M, N, K)) {
-    GemmBatch batch = {};
-    batch.out[0] = static_cast<uint16_t*>(out);
-    batch.a[0] = static_cast<const uint16_t*>(a);
-    batch.b[0] = static_cast<const uint16_t*>(b);
-    batch.bias[0] = static_cast<const uint16_t*>(bias);
-    if (int rc = launch_big_for(batch, 1, M, N, K, ldc, max_cus, hs)) return rc;
-  } else {
-    const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
-    int64_t grid = (int64_t)tiles_m * tiles_n;
-    if (max_cus > 0 && grid > max_cus) grid = max_cus;
-    if (grid > INT32_MAX) grid = INT32_MAX;
-    launch_kernel(gemm_bf16_nt_kernel, dim3((unsigned)grid), dim3(GEMM_THREADS), 0, hs,
-                  static_cast<uint16_t*>(out), static_cast<const uint16_t*>(a),
-                  static_cast<const uint16_t*>(b), static_cast<const uint16_t*>(bias), (int)M, (int)N, (int)K, ldc,
-                  tiles_m, tiles_n);
-  }
-  return finish_launch("gemm_bf16_nt");
+  GemmBatch batch = {};
+  batch.out[0] = static_cast<uint16_t*>(out);
+  batch.a[0] = static_cast<const uint16_t*>(a);
+  batch.b[0] = static_cast<const uint16_t*>(b);
+  batch.bias[0] = static_cast<const uint16_t*>(bias);
+  return run_products("gemm_bf16_nt", batch, 1, M, N, K, ldc, max_cus, static_cast<hipStream_t>(stream));
 }
 
 // outs[p][M, N] (row stride ldc) = as[p][M, K] * bs[p][N, K]^T (+ biases[p] when `biases` and
-// that entry are non-null) for p < count: one launch over count x tiles when the shape fits
-// the big kernel, one launch per product otherwise.
+// that entry are non-null) for p < count, in one launch over count x tiles.
 int run_gemm_bf16_nt_partials(void* const* outs, const void* const* as, const void* const* bs,
                               const void* const* biases, int count, int64_t M, int64_t N, int64_t K,
                               int64_t ldc, int max_cus, void* stream) {
@@ -672,13 +900,7 @@ int run_gemm_bf16_nt_partials(void* const* outs, const void* const* as, const vo
     batch.a[p] = static_cast<const uint16_t*>(as[p]);
     batch.b[p] = static_cast<const uint16_t*>(bs[p]);
   }
-  if (big_kernel_fits(M, N, K)) {
-    if (int rc = launch_big_for(batch, count, M, N, K, ldc, max_cus, static_cast<hipStream_t>(stream))) return rc;
-    return finish_launch(what);
-  }
-  for (int p = 0; p < count; ++p)
-    if (int rc = run_gemm_bf16_nt(outs[p], as[p], bs[p], batch.bias[p], M, N, K, ldc, max_cus, stream)) return rc;
-  return TW_OK;
+  return run_products(what, batch, count, M, N, K, ldc, max_cus, static_cast<hipStream_t>(stream));
 }
 
 }  // namespace tw
