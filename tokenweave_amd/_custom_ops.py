@@ -47,6 +47,20 @@ if os.path.exists(BINDING_PATH) and os.environ.get("TOKENWEAVE_AMD_NO_COMPILED_B
                       "from Python and calls the HIP library through ctypes instead", RuntimeWarning)
 _T = torch.ops.tokenweave_amd
 
+# The same functions as direct Python calls (csrc/tw_hostpath.cpp): 0.3 us on top of a launch
+# instead of 1.5 us through torch.ops or 5 us through ctypes.  Each answers False (or
+# NotImplemented) where the ordinary route has something to do: an argument it does not take,
+# an error to word, autograd, a dispatch mode.  None without the compiled binding.
+_fast = None
+if COMPILED_BINDING:
+    try:
+        from . import _hostpath as _fast
+    except ImportError as e:
+        warnings.warn(f"the direct calls could not be loaded ({e}); tokenweave_amd calls its ops through "
+                      "torch.ops instead", RuntimeWarning)
+# Under torch.compile the registered op must be traced, not the direct call.
+_tracing = torch.compiler.is_dynamo_compiling
+
 # Message of the reference's launchers (csrc/tokenweave_fused_kernels.cu:259).
 ALIGNMENT_MESSAGE = ("Input, residual, and weight tensors must be 16-byte aligned and "
                      "hidden_size must be divisible by 8 for optimized kernel.")
@@ -619,6 +633,10 @@ def rms_norm_dynamic_per_token_quant(input: torch.Tensor, weight: torch.Tensor, 
                                      residual: Optional[torch.Tensor] = None):
     """vllm/_custom_ops.py:256-272: allocates the outputs, returns (output, scales);
     residual (if given) is updated in place."""
+    if _fast is not None and not _tracing():
+        done = _fast.rms_norm_dynamic_per_token_quant(input, weight, epsilon, quant_dtype, scale_ub, residual)
+        if done is not NotImplemented:
+            return done
     output = torch.empty_like(input, dtype=quant_dtype)
     scales = torch.empty((input.numel() // input.shape[-1], 1), device=input.device, dtype=torch.float32)
     rms_norm_dynamic_per_token_quant_out(output, input, weight, scales, epsilon, scale_ub, residual)
@@ -693,7 +711,8 @@ def gemm_bf16_nt(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor,
     reference does it (on the rounded product, rounded again).  `out` may be a row slice of
     a wider buffer (row stride >= N).  The in-place row-parallel linear of
     vllm/model_executor/layers/linear.py:203-228."""
-    BoundOp(*_prepare_gemm_bf16_nt(out, a, b, max_cus, bias))()
+    if _fast is None or not _fast.gemm_bf16_nt(out, a, b, max_cus, bias):
+        BoundOp(*_prepare_gemm_bf16_nt(out, a, b, max_cus, bias))()
 
 
 def bind_gemm_bf16_nt(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor,
@@ -737,7 +756,8 @@ def gemm_bf16_nt_partials(outs: Sequence[torch.Tensor], a: Sequence[torch.Tensor
     rank's staging rows (`outs[p]` = `PartialsBuffer.slot(p)[first_row:first_row + M]`).  The
     producer side of the fused op: vllm/model_executor/layers/linear.py:203-228, 1310-1321
     (only rank 0 adds its bias, :1306-1308: pass it as biases[0], None elsewhere)."""
-    BoundOp(*_prepare_gemm_bf16_nt_partials(outs, a, b, max_cus, biases))()
+    if _fast is None or not _fast.gemm_bf16_nt_partials(outs, a, b, max_cus, biases):
+        BoundOp(*_prepare_gemm_bf16_nt_partials(outs, a, b, max_cus, biases))()
 
 
 def bind_gemm_bf16_nt_partials(outs: Sequence[torch.Tensor], a: Sequence[torch.Tensor],
@@ -829,40 +849,50 @@ if COMPILED_BINDING:
 
     def rms_norm(out: torch.Tensor, input: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                  epsilon: float) -> None:
-        _op_rms_norm(out, input, weight, epsilon)
+        if _fast is None or _tracing() or not _fast.rms_norm(out, input, weight, epsilon):
+            _op_rms_norm(out, input, weight, epsilon)
 
     def fused_add_rms_norm(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                            epsilon: float) -> None:
-        _op_fused_add_rms_norm(input, residual, weight, epsilon)
+        if _fast is None or _tracing() or not _fast.fused_add_rms_norm(input, residual, weight, epsilon):
+            _op_fused_add_rms_norm(input, residual, weight, epsilon)
 
     def rms_norm_inplace(out: torch.Tensor, input: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                          epsilon: float) -> None:
-        _op_rms_norm_inplace(out, input, weight, epsilon)
+        if _fast is None or _tracing() or not _fast.rms_norm_inplace(out, input, weight, epsilon):
+            _op_rms_norm_inplace(out, input, weight, epsilon)
 
     def fused_add_rms_norm_cta(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                                MAX_CTAS: int, epsilon: float) -> None:
-        _op_fused_add_rms_norm_cta(input, residual, weight, 0 if MAX_CTAS is None else MAX_CTAS, epsilon)
+        if _fast is None or _tracing() or not _fast.fused_add_rms_norm_cta(input, residual, weight, MAX_CTAS, epsilon):
+            _op_fused_add_rms_norm_cta(input, residual, weight, 0 if MAX_CTAS is None else MAX_CTAS, epsilon)
 
     def fused_rs_ln_ag_cta(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                            mcptr: int, signal_pads: int, rank: int, world_size: int, MAX_CTAS: int,
                            epsilon: float) -> None:
-        _op_fused_rs_ln_ag_cta(input, residual, weight, mcptr, signal_pads, rank, world_size,
-                               0 if MAX_CTAS is None else MAX_CTAS, epsilon)
+        if _fast is None or _tracing() or not _fast.fused_rs_ln_ag_cta(input, residual, weight, mcptr, rank, world_size,
+                                                                          MAX_CTAS, epsilon):
+            _op_fused_rs_ln_ag_cta(input, residual, weight, mcptr, signal_pads, rank, world_size,
+                                   0 if MAX_CTAS is None else MAX_CTAS, epsilon)
 
     def fused_rs_ln_cta(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                         mcptr: int, signal_pads: int, rank: int, world_size: int, MAX_CTAS: int,
                         epsilon: float) -> None:
-        _op_fused_rs_ln_cta(input, residual, weight, mcptr, signal_pads, rank, world_size,
-                            0 if MAX_CTAS is None else MAX_CTAS, epsilon)
+        if _fast is None or _tracing() or not _fast.fused_rs_ln_cta(input, residual, weight, mcptr, rank, world_size,
+                                                                       MAX_CTAS, epsilon):
+            _op_fused_rs_ln_cta(input, residual, weight, mcptr, signal_pads, rank, world_size,
+                                0 if MAX_CTAS is None else MAX_CTAS, epsilon)
 
     def rms_norm_static_fp8_quant(result: torch.Tensor, input: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                                   scale: torch.Tensor, epsilon: float) -> None:
-        _op_rms_norm_static_fp8_quant(result, input, weight, scale, epsilon)
+        if _fast is None or _tracing() or not _fast.rms_norm_static_fp8_quant(result, input, weight, scale, epsilon):
+            _op_rms_norm_static_fp8_quant(result, input, weight, scale, epsilon)
 
     def fused_add_rms_norm_static_fp8_quant(result: torch.Tensor, input: torch.Tensor,  # noqa: F811
                                             residual: torch.Tensor, weight: torch.Tensor,
                                             scale: torch.Tensor, epsilon: float) -> None:
-        _op_fused_add_rms_norm_static_fp8_quant(result, input, residual, weight, scale, epsilon)
+        if _fast is None or _tracing() or not _fast.fused_add_rms_norm_static_fp8_quant(result, input, residual, weight, scale, epsilon):
+            _op_fused_add_rms_norm_static_fp8_quant(result, input, residual, weight, scale, epsilon)
 
     def rms_norm_dynamic_per_token_quant_out(result: torch.Tensor, input: torch.Tensor,  # noqa: F811
                                              weight: torch.Tensor, scale: torch.Tensor, epsilon: float,
@@ -870,7 +900,9 @@ if COMPILED_BINDING:
                                              residual: Optional[torch.Tensor] = None) -> None:
         """The registered op (schema csrc/torch_bindings.cpp:216-219): result, scale and
         residual are written in place."""
-        _op_rms_norm_dynamic_per_token_quant(result, input, weight, scale, epsilon, scale_ub, residual)
+        if _fast is None or _tracing() or not _fast.rms_norm_dynamic_per_token_quant_out(result, input, weight, scale, epsilon, scale_ub,
+                                                                       residual):
+            _op_rms_norm_dynamic_per_token_quant(result, input, weight, scale, epsilon, scale_ub, residual)
 else:
     _library = torch.library.Library("tokenweave_amd", "DEF")
     for _name, _schema in SCHEMAS.items():

@@ -20,6 +20,7 @@
 #include <unordered_map>
 
 #include "../../include/tokenweave_amd.h"
+#include "tw_torch_ops.h"
 
 namespace {
 
@@ -183,9 +184,13 @@ void prepare_split_workspace(int64_t device_index) {
               "prepare_split_workspace: the current stream is being captured; call it before the capture begins");
 }
 
+}  // namespace
+
 // ---------------------------------------------------------------------------
 // layer norm ops (vllm/_custom_ops.py:176-207 -> csrc/torch_bindings.cpp:135-171)
 // ---------------------------------------------------------------------------
+namespace tw_torch {
+
 void rms_norm(Tensor& out, Tensor& input, Tensor& weight, double epsilon) {
   const int code = dtype_code("rms_norm_kernel", input);
   const auto dt = input.scalar_type();
@@ -241,49 +246,55 @@ void fused_add_rms_norm_cta(Tensor& input, Tensor& residual, Tensor& weight, int
                                      (int)max_ctas, (float)epsilon, l.stream));
 }
 
-void fused_rs_ln(bool all_gather, const char* kernel, Tensor& input, Tensor& residual, Tensor& weight,
-                 int64_t mcptr, int64_t rank, int64_t world_size, int64_t max_ctas, double epsilon) {
-  require_bf16(kernel, input);
+void fused_rs_ln_rows(bool all_gather, const Tensor& input, const Tensor& residual, const Tensor& weight, int64_t row0,
+                      int64_t rows, int64_t mcptr, int64_t rank, int64_t world_size, int64_t max_ctas, double epsilon) {
+  require_bf16(all_gather ? "fused_rs_ln_ag_cta_kernel" : "fused_rs_ln_cta_kernel", input);
   const auto dev = input.device();
   check_tensor("input", input, at::kBFloat16, dev);
   check_tensor("residual", residual, at::kBFloat16, dev);
   const Rows r = rows_of(input);
   TORCH_CHECK(residual.sizes() == input.sizes(), "input and residual must have the same shape");
+  TORCH_CHECK(row0 >= 0 && rows >= 0 && row0 + rows <= r.T, "rows [", row0, ", ", row0 + rows, ") outside [0, ", r.T, ")");
   check_weight(weight, r.H, at::kBFloat16, dev);
   TORCH_CHECK(rank >= 0 && rank < world_size, "Invalid rank ", rank, ", must be in [0, ", world_size - 1, "]");
-  const int64_t stride = peer_stride((uint64_t)mcptr, world_size, r.T * r.H * 2);
+  const int64_t stride = peer_stride((uint64_t)mcptr, world_size, rows * r.H * 2);
   Launch l(input);
-  if (max_ctas <= 0 && r.T > 0 && r.T <= 2 * TW_SPLIT_MAX_TOKENS) {
+  char* in = static_cast<char*>(input.data_ptr()) + row0 * r.H * 2;
+  char* res = static_cast<char*>(residual.data_ptr()) + row0 * r.H * 2;
+  if (max_ctas <= 0 && rows > 0 && rows <= 2 * TW_SPLIT_MAX_TOKENS) {
     // decode-size batch, or a few more rows than compute units: the workspace entry point
     // cuts rows into several workgroups where that pays
     if (void* ws = split_workspace(dev, l.stream)) {
-      check_rc(tw_fused_rs_ln_ag_cta_ws(input.data_ptr(), residual.data_ptr(), weight.data_ptr(), (uint64_t)mcptr,
-                                        stride, (int)rank, (int)world_size, 0, (float)epsilon, r.T, r.H, ws,
-                                        TW_SPLIT_WORKSPACE_BYTES, l.stream));
+      check_rc(tw_fused_rs_ln_ag_cta_ws(in, res, weight.data_ptr(), (uint64_t)mcptr, stride, (int)rank, (int)world_size,
+                                        0, (float)epsilon, rows, r.H, ws, TW_SPLIT_WORKSPACE_BYTES, l.stream));
       return;
     }
   }
   auto fn = all_gather ? tw_fused_rs_ln_ag_cta : tw_fused_rs_ln_cta;
-  check_rc(fn(input.data_ptr(), residual.data_ptr(), weight.data_ptr(), (uint64_t)mcptr, stride, (int)rank,
-              (int)world_size, (int)max_ctas, (float)epsilon, r.T, r.H, l.stream));
+  check_rc(fn(in, res, weight.data_ptr(), (uint64_t)mcptr, stride, (int)rank, (int)world_size, (int)max_ctas,
+              (float)epsilon, rows, r.H, l.stream));
 }
 
-void fused_rs_ln_ag_cta(Tensor& input, Tensor& residual, Tensor& weight, int64_t mcptr, int64_t /*signal_pads*/,
+static void fused_rs_ln(bool all_gather, const Tensor& input, const Tensor& residual, const Tensor& weight,
+                        int64_t mcptr, int64_t rank, int64_t world_size, int64_t max_ctas, double epsilon) {
+  fused_rs_ln_rows(all_gather, input, residual, weight, 0, rows_of(input).T, mcptr, rank, world_size, max_ctas,
+                   epsilon);
+}
+
+static void fused_rs_ln_ag_cta(Tensor& input, Tensor& residual, Tensor& weight, int64_t mcptr, int64_t /*signal_pads*/,
                         int64_t rank, int64_t world_size, int64_t max_ctas, double epsilon) {
-  fused_rs_ln(true, "fused_rs_ln_ag_cta_kernel", input, residual, weight, mcptr, rank, world_size, max_ctas,
-              epsilon);
+  fused_rs_ln(true, input, residual, weight, mcptr, rank, world_size, max_ctas, epsilon);
 }
 
-void fused_rs_ln_cta(Tensor& input, Tensor& residual, Tensor& weight, int64_t mcptr, int64_t /*signal_pads*/,
+static void fused_rs_ln_cta(Tensor& input, Tensor& residual, Tensor& weight, int64_t mcptr, int64_t /*signal_pads*/,
                      int64_t rank, int64_t world_size, int64_t max_ctas, double epsilon) {
-  fused_rs_ln(false, "fused_rs_ln_cta_kernel", input, residual, weight, mcptr, rank, world_size, max_ctas,
-              epsilon);
+  fused_rs_ln(false, input, residual, weight, mcptr, rank, world_size, max_ctas, epsilon);
 }
 
 // ---------------------------------------------------------------------------
 // norm + quantisation (csrc/torch_bindings.cpp:199-219)
 // ---------------------------------------------------------------------------
-void check_fp8_out(const Tensor& out, const Tensor& like) {
+static void check_fp8_out(const Tensor& out, const Tensor& like) {
   TORCH_CHECK(out.is_cuda() && out.device() == like.device(), "result is on ", out.device(), ", expected ",
               like.device());
   TORCH_CHECK_NOT_IMPLEMENTED(out.scalar_type() == at::kFloat8_e4m3fn,
@@ -293,7 +304,7 @@ void check_fp8_out(const Tensor& out, const Tensor& like) {
               "result must be a contiguous fp8 tensor with the input's shape");
 }
 
-void check_scale(const Tensor& scale, const c10::Device& dev) {
+static void check_scale(const Tensor& scale, const c10::Device& dev) {
   TORCH_CHECK(scale.is_cuda() && scale.device() == dev, "scale must be a tensor on the input's device");
   TORCH_CHECK(scale.scalar_type() == at::kFloat && scale.numel() == 1, "scale must hold one float32 value");
 }
@@ -367,6 +378,79 @@ void rms_norm_dynamic_per_token_quant(Tensor& out, const Tensor& input, const Te
                                                fp8 ? TW_QUANT_FP8_E4M3FN : TW_QUANT_INT8, l.stream));
 }
 
+// ---------------------------------------------------------------------------
+// the row-parallel projection (vllm/model_executor/layers/linear.py:203-228)
+// ---------------------------------------------------------------------------
+namespace {
+struct GemmShape {
+  int64_t M, N, K, ldc;
+  bool operator==(const GemmShape& o) const { return M == o.M && N == o.N && K == o.K && ldc == o.ldc; }
+};
+}  // namespace
+
+static GemmShape check_gemm(const Tensor& out, const Tensor& a, const Tensor& b, const Tensor* bias) {
+  require_bf16("gemm_bf16_nt_kernel", a);
+  const auto dev = a.device();
+  check_tensor("a", a, at::kBFloat16, dev);
+  check_tensor("b", b, at::kBFloat16, dev);
+  TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && out.dim() == 2, "gemm operands must be 2-D");
+  TORCH_CHECK(out.is_cuda() && out.device() == dev && out.scalar_type() == at::kBFloat16,
+              "out must be a bf16 tensor on the same device");
+  const int64_t M = a.size(0), K = a.size(1), N = b.size(0);
+  TORCH_CHECK(b.size(1) == K, "inner dimensions differ: a is ", a.sizes(), ", b is ", b.sizes());
+  TORCH_CHECK(out.size(0) == M && out.size(1) == N, "out has shape ", out.sizes(), ", expected (", M, ", ", N, ")");
+  TORCH_CHECK(out.stride(1) == 1 && (M <= 1 || out.stride(0) >= N), "out rows must be contiguous");
+  if (bias) {
+    check_tensor("bias", *bias, at::kBFloat16, dev);
+    TORCH_CHECK(bias->dim() == 1 && bias->numel() == N, "bias has shape ", bias->sizes(), ", expected (", N, ",)");
+  }
+  return {M, N, K, M > 1 ? out.stride(0) : std::max(N, out.stride(0))};
+}
+
+void gemm_bf16_nt(const Tensor& out, const Tensor& a, const Tensor& b, int64_t max_cus, const Tensor* bias) {
+  const GemmShape s = check_gemm(out, a, b, bias);
+  Launch l(a);
+  if (bias)
+    check_rc(tw_gemm_bf16_nt_bias(out.data_ptr(), a.data_ptr(), b.data_ptr(), bias->data_ptr(), s.M, s.N, s.K, s.ldc,
+                                  (int)max_cus, l.stream));
+  else
+    check_rc(tw_gemm_bf16_nt(out.data_ptr(), a.data_ptr(), b.data_ptr(), s.M, s.N, s.K, s.ldc, (int)max_cus, l.stream));
+}
+
+void gemm_bf16_nt_partials(const std::vector<const Tensor*>& outs, const std::vector<const Tensor*>& a,
+                           const std::vector<const Tensor*>& b, int64_t max_cus,
+                           const std::vector<const Tensor*>& biases) {
+  const size_t P = outs.size();
+  TORCH_CHECK(P >= 1 && P <= TW_MAX_PARTIALS, "number of partials ", P, " not in [1, ", TW_MAX_PARTIALS, "]");
+  TORCH_CHECK(a.size() == P && b.size() == P, "outs, a and b must have one entry per partial");
+  TORCH_CHECK(biases.empty() || biases.size() == P, "biases must have one entry (a tensor or None) per partial");
+  void* o[TW_MAX_PARTIALS];
+  const void *pa[TW_MAX_PARTIALS], *pb[TW_MAX_PARTIALS], *pbias[TW_MAX_PARTIALS];
+  GemmShape shape{};
+  bool any_bias = false;
+  for (size_t p = 0; p < P; ++p) {
+    const Tensor* bias = biases.empty() ? nullptr : biases[p];
+    const GemmShape s = check_gemm(*outs[p], *a[p], *b[p], bias);
+    if (p == 0) shape = s;
+    TORCH_CHECK(s == shape && a[p]->device() == a[0]->device(), "partial ", p, " has another shape than partial 0");
+    o[p] = outs[p]->data_ptr();
+    pa[p] = a[p]->data_ptr();
+    pb[p] = b[p]->data_ptr();
+    pbias[p] = bias ? bias->data_ptr() : nullptr;
+    any_bias = any_bias || bias;
+  }
+  Launch l(*a[0]);
+  if (any_bias)
+    check_rc(tw_gemm_bf16_nt_partials_bias(o, pa, pb, pbias, (int)P, shape.M, shape.N, shape.K, shape.ldc, (int)max_cus,
+                                           l.stream));
+  else
+    check_rc(tw_gemm_bf16_nt_partials(o, pa, pb, (int)P, shape.M, shape.N, shape.K, shape.ldc, (int)max_cus, l.stream));
+}
+
+}  // namespace tw_torch
+
+namespace {
+
 [[noreturn]] void no_cpu(const char* name) {
   TORCH_CHECK(false, "tokenweave_amd::", name,
               " has no CPU implementation: tokenweave_amd ops run on the GPU only; pass tensors that live on "
@@ -376,6 +460,8 @@ void rms_norm_dynamic_per_token_quant(Tensor& out, const Tensor& input, const Te
 }  // namespace
 
 // Schema strings of the reference (csrc/torch_bindings.cpp:135-171, 199-219).
+using namespace tw_torch;
+
 TORCH_LIBRARY(tokenweave_amd, m) {
   m.def("rms_norm(Tensor! result, Tensor input, Tensor weight, float epsilon) -> ()");
   m.def("fused_add_rms_norm(Tensor! input, Tensor! residual, Tensor weight, float epsilon) -> ()");

@@ -90,6 +90,11 @@ class RowParallelLinear(nn.Module):
     def forward(self, input_: torch.Tensor, output_: Optional[torch.Tensor] = None,
                 is_tokenweave: Optional[bool] = False, gemm_cus: Optional[int] = None
                 ) -> Tuple[torch.Tensor, Optional[Parameter]]:
+        if (is_tokenweave and ops._fast is not None and type(self.quant_method) is UnquantizedLinearMethod
+                and ops._fast.row_parallel_inplace(self, input_, output_, gemm_cus)):
+            if not self.return_bias:
+                return output_
+            return output_, (self.bias if self.skip_bias_add else None)
         if self.input_is_parallel:
             input_parallel = input_
         else:

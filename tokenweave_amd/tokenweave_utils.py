@@ -169,6 +169,12 @@ def fused_allreduce_layernorm(
     (tokenweave_utils.py:24-92).  `row_range=(start, end)` overrides the even
     split for ragged token counts (the reference pads instead, llama.py:536).
     """
+    # one native call for the usual case; it takes no other than a plain RMSNorm on plain tensors
+    if (ops._fast is not None and type(layernorm) is RMSNorm and not ops._tracing()
+            and ops._fast.fused_allreduce_layernorm(layernorm, hidden_states, residual, symm_mem_hdl,
+                                                    num_tokens_per_rank, rank, world_size, MAX_CTAS,
+                                                    offset_symm_mem, row_range)):
+        return
     assert hidden_states.shape == residual.shape, \
         "hidden_states and residual must have the same shape"
     assert 0 <= rank < world_size, f"Invalid rank {rank}, must be in [0, {world_size - 1}]"
