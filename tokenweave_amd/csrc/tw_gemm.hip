@@ -4,35 +4,25 @@
 // runs it as torch.matmul(x, W.t(), out=) (vllm/model_executor/layers/
 // linear.py:203-228).
 //
-// Both operands are K-contiguous, so the 8 consecutive k a lane feeds to
-// v_mfma_f32_32x32x16_bf16 are one 16-byte chunk of a row of `a` or `b`.  The
-// MFMA is issued with `b` rows as its first operand, which leaves every lane
-// with 4 consecutive n per accumulator quad: 8-byte row-major stores, or, in the
-// big kernel when the output allows 16-byte stores, a transpose through LDS into
-// whole 128-byte lines per row.
+// Both operands are K-contiguous, so the 8 consecutive k a lane feeds to an MFMA are one
+// 16-byte chunk of a row of `a` or `b`.  The MFMAs are issued with `b` rows as their first
+// operand, which leaves every lane with 4 consecutive n per accumulator quad.
 //
 // Three kernels:
-//  * gemm_bf16_nt_big_kernel<TM, TN> (K >= 64; a last partial k-slab is zero-filled): (64 TM) x (128 TN) x 64 tiles,
-//    8 waves (2 x 4, two per SIMD), each wave (32 TM) x (32 TN): 128/192/256/320 x 256
-//    (TN = 2) chosen per problem so that the tile count wastes the fewest workgroup
-//    rounds (M = 2458: 320-row tiles make exactly 256 tiles; M = 1024: 128-row tiles
-//    give every compute unit one), or 256 x 384.
-//    Operand slabs go from global memory straight into LDS (buffer_load ... lds:
-//    no staging registers, no LDS store instructions), two LDS stages.
-//    A wave instruction fills 1 KiB = 8 LDS rows of 128 bytes; row r keeps its
-//    16-byte chunk c at position c ^ ((r >> 1) & 7), which makes the 16-byte
-//    fragment reads of 16 consecutive rows conflict-free on the 64-bank LDS
-//    (counter-verified) without padding.  The descriptor's extent is the
-//    operand's size, so tile rows past M or N read as zeros.  Fragments are
-//    double-buffered in registers; the next k-step's LDS reads are issued
-//    between the two halves of the current step's MFMAs.
-//  * gemm_bf16_nt_ksplit_kernel<MT, NT> (at most 256 rows, or too few columns for the big
-//    tiles): (32 MT) x (32 NT) tiles whose four waves share the inner dimension.
+//  * gemm_bf16_nt_ksplit_kernel<MT, NT> (at most 128 rows): (32 MT) x (32 NT) tiles whose four
+//    waves share the inner dimension;
+//  * gemm_bf16_nt_tile_kernel<TM, TN> (more rows): (32 TM) x (32 TN) tiles, 64 x 128 to 256 x 256,
+//    picked per problem so that the tile count wastes the fewest workgroup rounds;
 //  * gemm_bf16_nt_kernel (K > 2^24, where a tile's rows outgrow 32-bit offsets): 128 x 128 x 64
 //    tiles, 4 waves, register-staged loads into padded LDS, 64-bit addresses.
-// Workgroups walk the tile list with stride gridDim.x (grid cap = compute-unit
-// budget of the weave schedule), and tile ids are remapped so that the
-// workgroups of one XCD (blockIdx % 8) share operand panels in that XCD's L2.
+// The first two bring operand slabs from global memory straight into LDS (buffer_load ... lds: no
+// staging registers, no LDS store instructions).  A wave instruction fills 1 KiB = 8 LDS rows of
+// 128 bytes with whole lines of eight operand rows; the 16-byte chunks of a row are permuted by the
+// row number so that fragment reads are conflict-free without padding.  A last partial k-slab is
+// zero-filled, and the descriptors end with the operand, so that tile rows past M or N read as zeros.
+// Workgroups walk the tile list with stride gridDim.x (grid cap = compute-unit budget of the weave
+// schedule), and tile ids are remapped so that the workgroups of one XCD (blockIdx % 8) share operand
+// panels in that XCD's L2.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -47,6 +37,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 128, BN = 128, BK = 64;
@@ -386,326 +377,327 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// (32 TM x 2) x 256 x 64 tiles, direct-to-LDS operand slabs (see the file
-// comment).  TM = 32-row MFMA tiles per wave along M: 4 -> 256-row tiles,
-// 5 -> 320-row tiles, 3 -> 192-row tiles.  The launcher picks the height that
-// wastes the fewest workgroup rounds for the given M.
+// Tile kernel: (32 TM) x (32 TN) x 64 tiles for everything with more rows.
+//
+// Four waves (2 x 2, one per SIMD), each (16 TM) x (16 TN) of the output in 16 x 16 accumulators
+// held in accumulation registers (256 of them for the 256 x 256 tile), v_mfma_f32_16x16x32_bf16:
+// its 4-register accumulators cost less register traffic than 32 x 32 ones, and a 128 x 128 wave
+// tile reads a third fewer fragment bytes from LDS per flop than the 64 x 128 one of eight waves.
+//
+// One wave per SIMD hides nothing behind other waves, so everything is placed by hand between the
+// MFMAs of the k loop and pinned there by scheduling barriers:
+//  * A slab (64 of the inner dimension) is two phases of TM * TN MFMAs, one per 32 of it.  While a
+//    phase runs on one set of fragments the other set is read from LDS for the next one: no MFMA
+//    waits for LDS, also not across slabs or tiles.
+//  * Between the phases lies the slab's one barrier.  It says that this slab's LDS is free and
+//    that the next slab has arrived: a wave waits for its own loads before it, D - 1 slabs after
+//    it issued them.
+//  * Operand slabs go from global memory straight into LDS, D slabs ahead, one load per several
+//    MFMAs: the compute unit's path to memory takes 64 bytes per cycle, half of the 256 x 256
+//    tile's loop, and loads issued in a burst stall the waves behind it (all 16 loads of a wave in
+//    half a phase: 786 us for 8192^3, spread over a phase 749, over the slab 714).
+//  * The slab sequence runs on across tiles: a workgroup keeps its compute unit and walks the tile
+//    list with stride gridDim.x, the first D slabs of the next tile are under way while the
+//    accumulators of the last one are stored, and its first barrier does not wait for those stores
+//    (vmcnt counts in order: they are younger than the loads it needs).
+//  * Results leave by 16-byte stores from the registers.  The columns a lane holds are made
+//    adjacent by the row order in which b's fragments are read: MFMA row r of the tile pair
+//    (2 p, 2 p + 1) is column 32 p + 8 (r / 4) + 4 (tile & 1) + r % 4 of the wave's columns.  They are
+//    written through (nt sc0 sc1): all compute units store 33 MB at the same moment, and what
+//    stays dirty in the L2s is in the way of the next tile's loads (8192 x 8192 x 1024: 107 us, default
+//    policy 112, nt 116).
+// LDS: rows of 128 bytes, 16-byte chunk c of row r at position c ^ key(r), key(r) = (r >> 1) & 7 for
+// a and bits 1, 3, 4 of r for b: the 16 rows that a fragment read touches at once are
+// conflict-free (counter-verified).  256 x 256: three a panels and two b panels, exactly 160 KiB.
+//
+// The MFMAs are written as inline assembly with the accumulators tied to accumulation registers:
+// left to choose, the register allocator moves accumulators between the two files and spills
+// (112 against 107 us, 8192 x 8192 x 1024).
+//
+// Measured against the 8-wave kernel this replaces, same box: 8192^3 874 -> 714 us (1 253 -> 1 539
+// TFLOP/s; matrix cores busy 65 -> 84 % of the cycles while the clock, under the board's power limit,
+// falls from 1.91 to 1.84 GHz), 8192 x 8192 x 3584 406 -> 325, 8192 x 8192 x 1024 127 -> 107,
+// 1024 x 8192 x 3712 59 -> 48, 512 x 8192 x 3584 49 -> 28 us.
 // ---------------------------------------------------------------------------
-constexpr int BIG_BK = 64;
-constexpr int BIG_THREADS = 512;
-constexpr int BIG_ROWB = BIG_BK * 2;             // bytes per LDS row
-constexpr int BIG_GROUP_M = 4;
-constexpr int big_lds_bytes(int tm, int tn) { return 2 * (tm * 64 + tn * 128) * BIG_ROWB; }
+typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
+typedef __attribute__((address_space(3))) const bf16x8_t lds_frag_t;
+constexpr int TILE_THREADS = 256;
+constexpr int64_t TILE_MAX_K = 1 << 21;    // a tile's rows span less than 2 GiB: the out-of-range marker below
+constexpr int64_t TILE_MAX_LDC = 1 << 21;
+[[maybe_unused]] constexpr uint32_t TILE_OUT_OF_RANGE = 0x80000000u;
 
-// One k-slab of both operands, global memory -> LDS: this wave's LA + LB wave
-// instructions of 1 KiB each.  (A free function, not a lambda: the kernel is a
-// template, and the host pass must be able to instantiate its stub without
-// compiling device builtins.)
-template <int LA, int LB>
-__device__ __forceinline__ void big_issue_slab(__amdgpu_buffer_rsrc_t da, __amdgpu_buffer_rsrc_t db,
-                                               const uint32_t (&va)[LA], const uint32_t (&vb)[LB],
-                                               uint8_t* sa, uint8_t* sb, uint32_t koff) {
-#pragma unroll
-  for (int j = 0; j < LA; ++j)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(da, (lds_void_t*)(sa + j * 1024), 16, va[j], koff, 0, 0);
-#pragma unroll
-  for (int j = 0; j < LB; ++j)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(db, (lds_void_t*)(sb + j * 1024), 16, vb[j], koff, 0, 0);
+// How a tile shape uses LDS and where in a slab (slots: its 2 TM TN MFMAs) its loads go out.
+template <int TM, int TN>
+struct TileShape {
+  static constexpr int BM = 32 * TM, BN = 32 * TN, SLOTS = TM * TN;
+  static constexpr int LA = TM, LB = TN, L = LA + LB;  // wave loads (8 rows each) per slab and operand
+  static constexpr int PA = BM * 128, PB = BN * 128;   // panel bytes
+  static constexpr int STAGES = 160 * 1024 / (PA + PB);
+  // Two whole stages only: a third a panel, so that a's loads can go out in the phase before the
+  // barrier, b's in the one behind it.
+  static constexpr bool TIGHT = STAGES == 2;
+  static constexpr int D = TIGHT ? 2 : (STAGES - 1 < 3 ? STAGES - 1 : 3);  // slabs ahead
+  static constexpr int SA = D + 1, SB = TIGHT ? D : D + 1;
+  static constexpr int LDS = SA * PA + SB * PB;
+  static constexpr int SPREAD = 2 * SLOTS / L;
+  static constexpr int A0 = TIGHT ? 1 : 0, A_STEP = TIGHT ? SLOTS / LA : SPREAD;
+  static constexpr int B0 = TIGHT ? SLOTS + 1 : LA * SPREAD, B_STEP = TIGHT ? SLOTS / LB : SPREAD;
+  static constexpr int READ_STEP = SLOTS / L / 2 < 1 ? 1 : SLOTS / L / 2;
+  // loads that go out before the barrier
+  static constexpr int before(int first, int step, int n) {
+    int c = 0;
+    for (int l = 0; l < n; ++l) c += first + l * step < SLOTS ? 1 : 0;
+    return c;
+  }
+  static constexpr int EARLY = before(A0, A_STEP, LA) + before(B0, B_STEP, LB);
+  // may be outstanding at a slab's barrier: slabs 2 .. D - 1 ahead and the early part of slab D
+  static constexpr int IN_FLIGHT = (D - 2) * L + EARLY;
+  static constexpr int STORES = SLOTS / 2;
+  static_assert(SPREAD >= 1 && D >= 2 && LDS <= 160 * 1024 && IN_FLIGHT + STORES <= 63, "tile shape");
+  static_assert(A0 + (LA - 1) * A_STEP < 2 * SLOTS && B0 + (LB - 1) * B_STEP < 2 * SLOTS, "every load has a slot");
+  static_assert((L - 1) * READ_STEP < SLOTS, "every fragment read has a slot");
+};
+
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass only needs the kernels' stubs
+__device__ __forceinline__ void tile_mfma_first(f32x4_t& c, const bf16x8_t& x, const bf16x8_t& y) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(x), "v"(y));
+}
+__device__ __forceinline__ void tile_mfma(f32x4_t& c, const bf16x8_t& x, const bf16x8_t& y) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));
+}
+__device__ __forceinline__ uint32_t tile_pack2(float lo, float hi) {
+  float x, y;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(lo));
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(y) : "a"(hi));
+  return pack2(x, y);
 }
 
-// The last k-slab of an inner dimension that is not a multiple of 64 (but of 8): the 16-byte
-// chunks that lie past K must land in LDS as zeros.  A lane's chunk is c ^ 4 in odd 8-row
-// blocks and c in even ones (the swizzle above), so two flags per lane say whether its chunk
-// is inside; a chunk outside is requested at an offset past the descriptor's extent, which
-// the hardware answers with zeros.
-constexpr uint32_t BIG_OUT_OF_RANGE = 0x80000000u;  // operands are smaller than 2 GiB
-
-template <int LA, int LB>
-__device__ __forceinline__ void big_issue_slab_tail(__amdgpu_buffer_rsrc_t da, __amdgpu_buffer_rsrc_t db,
-                                                    const uint32_t (&va)[LA], const uint32_t (&vb)[LB],
-                                                    uint8_t* sa, uint8_t* sb, uint32_t koff, int blk_a, int blk_b,
-                                                    bool in_even, bool in_odd) {
+// One phase: acc += fb x fa, and between the MFMAs the next phase's fragments (na, nb from pa, pb)
+// and this half's share of the loads of the slab D ahead.
+template <int TM, int TN, bool FIRST, int HALF>
+__device__ __forceinline__ void tile_phase(f32x4_t (&acc)[TM][TN], const bf16x8_t (&fa)[TM], const bf16x8_t (&fb)[TN],
+                                           bf16x8_t (&na)[TM], bf16x8_t (&nb)[TN], const lds_u8_t* pa,
+                                           const lds_u8_t* pb, __amdgpu_buffer_rsrc_t da, __amdgpu_buffer_rsrc_t db,
+                                           const uint32_t (&va)[TM], const uint32_t (&vb)[TN], lds_u8_t* sa,
+                                           lds_u8_t* sb, uint32_t koff) {
+  using S = TileShape<TM, TN>;
 #pragma unroll
-  for (int j = 0; j < LA; ++j) {
-    const bool in = ((blk_a + j) & 1) ? in_odd : in_even;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(da, (lds_void_t*)(sa + j * 1024), 16, in ? va[j] : BIG_OUT_OF_RANGE, koff,
-                                             0, 0);
-  }
-#pragma unroll
-  for (int j = 0; j < LB; ++j) {
-    const bool in = ((blk_b + j) & 1) ? in_odd : in_even;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(db, (lds_void_t*)(sb + j * 1024), 16, in ? vb[j] : BIG_OUT_OF_RANGE, koff,
-                                             0, 0);
+  for (int n = 0; n < S::SLOTS; ++n) {
+    const int i = n / TN, j = n % TN, slot = n + HALF * S::SLOTS;
+    if (FIRST) tile_mfma_first(acc[i][j], fb[j], fa[i]);
+    else tile_mfma(acc[i][j], fb[j], fa[i]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (n % S::READ_STEP == 0 && n / S::READ_STEP < S::L) {
+      const int r = n / S::READ_STEP;
+      if (r < TN) nb[r] = *(lds_frag_t*)(pb + (r >> 1) * 4096 + (r & 1) * 512);
+      else na[r - TN] = *(lds_frag_t*)(pa + (r - TN) * 2048);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (slot >= S::A0 && (slot - S::A0) % S::A_STEP == 0 && (slot - S::A0) / S::A_STEP < S::LA) {
+      const int l = (slot - S::A0) / S::A_STEP;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(da, (lds_void_t*)(sa + l * 1024), 16, va[l], koff, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (slot >= S::B0 && (slot - S::B0) % S::B_STEP == 0 && (slot - S::B0) / S::B_STEP < S::LB) {
+      const int l = (slot - S::B0) / S::B_STEP;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(db, (lds_void_t*)(sb + l * 1024), 16, vb[l], koff, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 }
+
+constexpr int kStoreThrough = 19;  // nt sc0 sc1
+
+// The wave's accumulators: row 16 i of `dc` at voffset + i * row_step.  WIDE: eight columns per
+// store, else four (rows that are only 8-byte aligned, or N % 8 != 0).
+template <int TM, int TN, bool WIDE, bool BIAS>
+__device__ __forceinline__ void tile_store(const f32x4_t (&acc)[TM][TN], __amdgpu_buffer_rsrc_t dc, uint32_t row_off,
+                                           uint32_t row_step, int n, int N, const uint16_t* bias) {
+  uint32_t off[TN];  // of four columns each, out of range when they lie past N
+  uint2 bv[BIAS ? TN : 1];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int c = n + (j >> 1) * 32 + (j & 1) * 4;
+    off[j] = c < N ? row_off + (uint32_t)((j >> 1) * 64 + (j & 1) * 8) : TILE_OUT_OF_RANGE;
+    if (BIAS) bv[j] = c < N ? *reinterpret_cast<const uint2*>(bias + c) : make_uint2(0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int j = 0; j < TN; j += 2) {
+      u32x4_t v = {tile_pack2(acc[i][j][0], acc[i][j][1]), tile_pack2(acc[i][j][2], acc[i][j][3]),
+                   tile_pack2(acc[i][j + 1][0], acc[i][j + 1][1]), tile_pack2(acc[i][j + 1][2], acc[i][j + 1][3])};
+      if (BIAS)
+        v = u32x4_t{add_bias2(v.x, bv[j].x), add_bias2(v.y, bv[j].y), add_bias2(v.z, bv[j + 1].x),
+                    add_bias2(v.w, bv[j + 1].y)};
+      if (WIDE) {
+        __builtin_amdgcn_raw_buffer_store_b128(v, dc, off[j] + (uint32_t)i * row_step, 0, kStoreThrough);
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{v.x, v.y}, dc, off[j] + (uint32_t)i * row_step, 0, kStoreThrough);
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{v.z, v.w}, dc, off[j + 1] + (uint32_t)i * row_step, 0,
+                                              kStoreThrough);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// Where the loader stands: product, tile and slab of the next slab to request.
+struct TilePlace {
+  int product, m0, n0;
+};
 
 template <int TM, int TN>
-__global__ __launch_bounds__(BIG_THREADS) void gemm_bf16_nt_big_kernel(
+__device__ __forceinline__ TilePlace tile_place(int t, int num_tiles, int tiles_m, int tiles_n) {
+  using S = TileShape<TM, TN>;
+  // Tile rows per sweep over the columns: the 32 tiles an XCD works on at a time then form a block
+  // that needs the fewest operand bytes through that XCD's L2.
+  constexpr int GROUP = S::BN >= 2 * S::BM ? 8 : 4;
+  // Every XCD (workgroup ids congruent mod 8) gets a contiguous range of the tile order: with
+  // eight products, one product each.
+  int pid = t;
+  const int per_xcd = num_tiles / 8;
+  if (t < per_xcd * 8) pid = (t & 7) * per_xcd + (t >> 3);
+  const int per_product = tiles_m * tiles_n;
+  const int product = pid / per_product;
+  pid -= product * per_product;
+  const int sweep = GROUP * tiles_n, group = pid / sweep, first = group * GROUP, rows = min(tiles_m - first, GROUP);
+  return {product, (first + (pid % sweep) % rows) * S::BM, ((pid % sweep) / rows) * S::BN};
+}
+#endif
+
+template <int TM, int TN>
+__global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THREADS) void gemm_bf16_nt_tile_kernel(
     GemmBatch batch, int count, int M, int N, int K, int64_t ldc, int tiles_m, int tiles_n, int wide_store) {
-  constexpr int WM = 32 * TM, WN = 32 * TN;  // wave tile
-  constexpr int BM = 2 * WM, BN = 4 * WN;    // workgroup tile: the 8 waves as 2 x 4
-  constexpr int PANEL_A = BM * BIG_ROWB;
-  constexpr int STAGE = PANEL_A + BN * BIG_ROWB;  // a-panel then b-panel
-  constexpr int LA = BM / 64;           // a-panel loads per wave per slab (8 rows x 8 waves each)
-  constexpr int LB = BN / 64;           // b-panel loads per wave per slab
-  constexpr int H1 = (TM + 1) / 2;      // MFMA rows issued before the next fragments are fetched
-  extern __shared__ __attribute__((aligned(1024))) uint8_t lds_big[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2, wn = wave & 3, l32 = lane & 31, lhi = lane >> 5;
-  const int tiles_per_product = tiles_m * tiles_n;
-  const int num_tiles = count * tiles_per_product;
-  const int nk = (K + BIG_BK - 1) / BIG_BK;
-  const int tail_chunks = (K % BIG_BK) / 8;  // 16-byte chunks of the last slab that lie inside K (0: all eight)
-  // Loader: wave instruction j of wave w fills the 8-row LDS block w * L + j; lane l
-  // lands at row l / 8, position l % 8 of that block, so it must fetch the chunk
-  // (l % 8) ^ key(row), key(r) = (r >> 1) & 7 = ((block & 1) << 2) | (l >> 4).
-  const int ld_row = lane >> 3;
-  const int ld_key = lane >> 4;
-  const bool tail_in_even = ((lane & 7) ^ ld_key) < tail_chunks;
-  const bool tail_in_odd = ((lane & 7) ^ ld_key ^ 4) < tail_chunks;
-  // Reader: lane row l32 (+ 32 i; wave offsets are multiples of 16 rows, which do not
-  // change the key), chunk 2 kk + lhi.
-  uint32_t roff[4];
+#ifdef __HIP_DEVICE_COMPILE__
+  using S = TileShape<TM, TN>;
+  constexpr int LA = S::LA, LB = S::LB, PA = S::PA, PB = S::PB, D = S::D;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds_tile[];
+  lds_u8_t* const lds_a = (lds_u8_t*)lds_tile;
+  lds_u8_t* const lds_b = lds_a + S::SA * PA;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, quad = lane >> 4;
+  const int nk = (K + BK - 1) / BK;
+  const int tail_chunks = (K % BK) / 8;  // 16-byte chunks of the last slab that lie inside K (0: all eight)
+  const int num_tiles = count * tiles_m * tiles_n;
+
+  // Reader: the two 32-wide halves of a slab.
+  const uint32_t row_a = (wm * 16 * TM + r16) * 128, row_b = (wn * 16 * TN + (r16 >> 2) * 8 + (r16 & 3)) * 128;
+  const uint32_t chunk0 = (quad ^ (r16 >> 1)) << 4, chunk1 = ((4 + quad) ^ (r16 >> 1)) << 4;
+  const lds_u8_t *const a0 = lds_a + row_a + chunk0, *const a1 = lds_a + row_a + chunk1;
+  const lds_u8_t *const b0 = lds_b + row_b + chunk0, *const b1 = lds_b + row_b + chunk1;
+  // Loader: wave instruction l fills the 8-row block wave * L + l; lane l lands at row l / 8,
+  // position l % 8 of it and fetches the chunk that belongs there.  Offsets are inside the tile,
+  // whose descriptors end with the last row of the operand: rows past it read as zeros.
+  lds_u8_t* const wa = lds_a + wave * LA * 1024;
+  lds_u8_t* const wb = lds_b + wave * LB * 1024;
+  uint32_t va[LA], vb[LB];
+  // `chunks`: how many of a row's chunks exist in the slab; the others must arrive as zeros
+#define TW_TILE_OFFSETS(chunks)                                                                              \
+  do {                                                                                                       \
+    _Pragma("unroll") for (int l = 0; l < LA; ++l) {                                                         \
+      const int blk = wave * LA + l, c = (lane & 7) ^ (((blk & 1) << 2) | (lane >> 4));                      \
+      va[l] = c < (chunks) ? (uint32_t)((blk * 8 + (lane >> 3)) * K + c * 8) * 2u : TILE_OUT_OF_RANGE;       \
+    }                                                                                                        \
+    _Pragma("unroll") for (int l = 0; l < LB; ++l) {                                                         \
+      const int blk = wave * LB + l, c = (lane & 7) ^ (((lane >> 4) & 1) | ((blk & 3) << 1));                \
+      vb[l] = c < (chunks) ? (uint32_t)((blk * 8 + (lane >> 3)) * K + c * 8) * 2u : TILE_OUT_OF_RANGE;       \
+    }                                                                                                        \
+  } while (0)
+  // Load cursor: slab lk of tile lt.  Past the last tile the descriptors are empty and the loads
+  // ask memory for nothing.
+  int lt = blockIdx.x, lk = 0;
+  __amdgpu_buffer_rsrc_t da, db;
+#define TW_TILE_DESCRIPTORS()                                                                                \
+  do {                                                                                                       \
+    const bool in = lt < num_tiles;                                                                          \
+    const TilePlace p = tile_place<TM, TN>(in ? lt : 0, num_tiles, tiles_m, tiles_n);                        \
+    da = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(batch.a[p.product]) + (size_t)p.m0 * K, 0,  \
+                                           in ? (uint32_t)min(M - p.m0, S::BM) * (uint32_t)K * 2u : 0u,      \
+                                           0x00020000);                                                      \
+    db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(batch.b[p.product]) + (size_t)p.n0 * K, 0,  \
+                                           in ? (uint32_t)min(N - p.n0, S::BN) * (uint32_t)K * 2u : 0u,      \
+                                           0x00020000);                                                      \
+  } while (0)
+#define TW_TILE_ADVANCE()                                                                                    \
+  do {                                                                                                       \
+    ++lk;                                                                                                    \
+    if (lk == nk) {                                                                                          \
+      lk = 0;                                                                                                \
+      lt += gridDim.x;                                                                                       \
+      TW_TILE_DESCRIPTORS();                                                                                 \
+      if (tail_chunks) TW_TILE_OFFSETS(nk == 1 ? tail_chunks : 8);                                           \
+    } else if (tail_chunks && lk == nk - 1) {                                                                \
+      TW_TILE_OFFSETS(tail_chunks);                                                                          \
+    }                                                                                                        \
+  } while (0)
+  TW_TILE_DESCRIPTORS();
+  TW_TILE_OFFSETS(tail_chunks && nk == 1 ? tail_chunks : 8);
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk)
-    roff[kk] = l32 * BIG_ROWB + ((((kk << 1) | lhi) ^ ((l32 >> 1) & 7)) << 4);
+  for (int s = 0; s < D; ++s) {
+#pragma unroll
+    for (int l = 0; l < LA; ++l)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(da, (lds_void_t*)(wa + s * PA + l * 1024), 16, va[l], lk * 128u, 0, 0);
+#pragma unroll
+    for (int l = 0; l < LB; ++l)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(db, (lds_void_t*)(wb + s * PB + l * 1024), 16, vb[l], lk * 128u, 0, 0);
+    TW_TILE_ADVANCE();
+  }
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 1) * S::L) : "memory");
+  f32x4_t acc[TM][TN];
+  bf16x8_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
+#pragma unroll
+  for (int r = 0; r < TN; ++r) fb0[r] = *(lds_frag_t*)(b0 + (r >> 1) * 4096 + (r & 1) * 512);
+#pragma unroll
+  for (int r = 0; r < TM; ++r) fa0[r] = *(lds_frag_t*)(a0 + r * 2048);
+
+  // ring positions: the slab in use and the one being filled
+  uint32_t use_a = 0, use_b = 0, fill_a = (D % S::SA) * PA, fill_b = (D % S::SB) * PB;
+#define TW_RING(x, panel, n) x = (x) + (panel) == (n) * (panel) ? 0u : (x) + (panel)
+#define TW_TILE_SLAB(FIRST, AFTER_STORE)                                                                         \
+  do {                                                                                                       \
+    tile_phase<TM, TN, FIRST, 0>(acc, fa0, fb0, fa1, fb1, a1 + use_a, b1 + use_b, da, db, va, vb, wa + fill_a, \
+                                 wb + fill_b, lk * 128u);                                                    \
+    if (AFTER_STORE)                                                                                         \
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S::IN_FLIGHT + S::STORES) : "memory"); \
+    else                                                                                                     \
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S::IN_FLIGHT) : "memory");            \
+    TW_RING(use_a, PA, S::SA);                                                                               \
+    TW_RING(use_b, PB, S::SB);                                                                               \
+    tile_phase<TM, TN, false, 1>(acc, fa1, fb1, fa0, fb0, a0 + use_a, b0 + use_b, da, db, va, vb, wa + fill_a, \
+                                 wb + fill_b, lk * 128u);                                                    \
+    TW_TILE_ADVANCE();                                                                                       \
+    TW_RING(fill_a, PA, S::SA);                                                                              \
+    TW_RING(fill_b, PB, S::SB);                                                                              \
+  } while (0)
 
   for (int t = blockIdx.x; t < num_tiles; t += gridDim.x) {
-    // Every XCD (workgroup ids congruent mod 8) gets a contiguous range of the tile order:
-    // with eight products, one product each.
-    int pid = t;
-    {
-      const int per_xcd = num_tiles / 8;
-      const int body = per_xcd * 8;
-      if (t < body) pid = (t & 7) * per_xcd + (t >> 3);
-    }
-    const int product = pid / tiles_per_product;
-    pid -= product * tiles_per_product;
-    uint16_t* __restrict__ out = batch.out[product];
-    const uint16_t* __restrict__ bias = batch.bias[product];
-    const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(batch.a[product]), 0, (uint32_t)((size_t)M * K * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(batch.b[product]), 0, (uint32_t)((size_t)N * K * 2), 0x00020000);
-    const int group_size = BIG_GROUP_M * tiles_n;
-    const int group = pid / group_size;
-    const int first_m = group * BIG_GROUP_M;
-    const int rows_in_group = min(tiles_m - first_m, BIG_GROUP_M);
-    const int tm_idx = first_m + (pid % group_size) % rows_in_group;
-    const int tn_idx = (pid % group_size) / rows_in_group;
-    const int m0 = tm_idx * BM, n0 = tn_idx * BN;
+    TW_TILE_SLAB(true, t != (int)blockIdx.x);
+    for (int kt = 1; kt < nk; ++kt) TW_TILE_SLAB(false, false);
 
-    uint32_t va[LA], vb[LB];
-#pragma unroll
-    for (int j = 0; j < LA; ++j) {
-      const int blk = wave * LA + j;
-      const int chunk = (lane & 7) ^ (((blk & 1) << 2) | ld_key);
-      va[j] = (uint32_t)(((size_t)(m0 + blk * 8 + ld_row) * K + chunk * 8) * 2);
-    }
-#pragma unroll
-    for (int j = 0; j < LB; ++j) {
-      const int blk = wave * LB + j;
-      const int chunk = (lane & 7) ^ (((blk & 1) << 2) | ld_key);
-      vb[j] = (uint32_t)(((size_t)(n0 + blk * 8 + ld_row) * K + chunk * 8) * 2);
-    }
-    f32x16_t acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-    __syncthreads();  // the previous tile's fragment reads are finished
-    big_issue_slab<LA, LB>(da, db, va, vb, lds_big + (wave * LA) * 1024,
-                           lds_big + PANEL_A + (wave * LB) * 1024, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-
-    for (int kt = 0; kt < nk; ++kt) {
-      const int stage = kt & 1;
-      if (kt + 2 < nk || (kt + 2 == nk && tail_chunks == 0))
-        big_issue_slab<LA, LB>(da, db, va, vb, lds_big + (stage ^ 1) * STAGE + (wave * LA) * 1024,
-                               lds_big + (stage ^ 1) * STAGE + PANEL_A + (wave * LB) * 1024,
-                               (uint32_t)(kt + 1) * BIG_ROWB);
-      else if (kt + 2 == nk)
-        big_issue_slab_tail<LA, LB>(da, db, va, vb, lds_big + (stage ^ 1) * STAGE + (wave * LA) * 1024,
-                                    lds_big + (stage ^ 1) * STAGE + PANEL_A + (wave * LB) * 1024,
-                                    (uint32_t)(kt + 1) * BIG_ROWB, wave * LA, wave * LB, tail_in_even, tail_in_odd);
-      const uint8_t* pa = lds_big + stage * STAGE + (wm * WM) * BIG_ROWB;
-      const uint8_t* pb = lds_big + stage * STAGE + PANEL_A + (wn * WN) * BIG_ROWB;
-      if constexpr (TN == 3) {
-        // 192 accumulators leave no room for two copies of both fragment sets: `a`
-        // fragments are single-buffered and refilled for the next step right after
-        // their last use in this one (half of them in the middle of the step, half
-        // at its end); only the `b` fragments are double-buffered.
-        bf16x8_t fa[TM], fb[2][TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-          fa[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(pa + i * 32 * BIG_ROWB + roff[0]));
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          fb[0][j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(pb + j * 32 * BIG_ROWB + roff[0]));
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const int cur = kk & 1, nxt = cur ^ 1;
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = 0; i < H1; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][j], fa[i], acc[i][j], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          if (kk < 3) {
-#pragma unroll
-            for (int i = 0; i < H1; ++i)
-              fa[i] = __builtin_bit_cast(
-                  bf16x8_t, *reinterpret_cast<const uint4*>(pa + i * 32 * BIG_ROWB + roff[kk + 1]));
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              fb[nxt][j] = __builtin_bit_cast(
-                  bf16x8_t, *reinterpret_cast<const uint4*>(pb + j * 32 * BIG_ROWB + roff[kk + 1]));
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = H1; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][j], fa[i], acc[i][j], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          if (kk < 3) {
-#pragma unroll
-            for (int i = H1; i < TM; ++i)
-              fa[i] = __builtin_bit_cast(
-                  bf16x8_t, *reinterpret_cast<const uint4*>(pa + i * 32 * BIG_ROWB + roff[kk + 1]));
-          }
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        continue;
-      }
-      bf16x8_t fa[2][TM], fb[2][TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        fa[0][i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(pa + i * 32 * BIG_ROWB + roff[0]));
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        fb[0][j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(pb + j * 32 * BIG_ROWB + roff[0]));
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const int cur = kk & 1, nxt = cur ^ 1;
-        // First part of this step's MFMAs, the next step's fragment reads, the rest:
-        // the reads complete in the shadow of the rest.  The scheduling barriers keep
-        // the compiler from sinking the reads to their use.
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < H1; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][j], fa[cur][i], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (kk < 3) {
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-            fa[nxt][i] = __builtin_bit_cast(
-                bf16x8_t, *reinterpret_cast<const uint4*>(pa + i * 32 * BIG_ROWB + roff[kk + 1]));
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            fb[nxt][j] = __builtin_bit_cast(
-                bf16x8_t, *reinterpret_cast<const uint4*>(pb + j * 32 * BIG_ROWB + roff[kk + 1]));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = H1; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][j], fa[cur][i], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // the next slab has landed (this wave's share), and after the barrier every
-      // wave's share has; nobody still reads the stage that gets overwritten next
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-    }
-
-    // acc[i][j][4 q + e] = out[m0 + wm*WM + i*32 + l32][n0 + wn*WN + j*32 + 8 q + 4 lhi + e]
-    if (wide_store) {
-      // Through LDS, 32 rows of the wave tile at a time (a wave-private 32 x WN patch,
-      // rows padded by 8 bytes): lanes write their 4-element groups, then read the patch
-      // back row-contiguously, 16 bytes per lane, so that a wave store covers whole
-      // 128-byte lines of 8 output rows instead of 16-byte pieces of 32 rows.  The slab
-      // stages are free: every wave passed the barrier that ends the k loop.
-      constexpr int PATCH_ROW = WN * 2 + 8;            // bytes
-      constexpr int CHUNKS = WN / 8;                   // 16-byte chunks per patch row
-      constexpr int ROWS_PER_PASS = 64 / CHUNKS;       // 8 (WN = 64) or 5 (WN = 96: 4 lanes idle)
-      uint8_t* patch = lds_big + wave * (32 * PATCH_ROW);
-      const int rd_row = lane / CHUNKS, rd_chunk = lane % CHUNKS;
-      const bool rd_lane = rd_row < ROWS_PER_PASS;
-      const int n = n0 + wn * WN + rd_chunk * 8;
-      // this lane's eight columns are the same in every pass: their bias is fetched once
-      uint4 bv = make_uint4(0, 0, 0, 0);
-      if (bias && rd_lane && n < N) bv = *reinterpret_cast<const uint4*>(bias + n);
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            uint2 v;
-            v.x = pack2(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1]);
-            v.y = pack2(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-            *reinterpret_cast<uint2*>(patch + l32 * PATCH_ROW + (j * 32 + 8 * q + 4 * lhi) * 2) = v;
-          }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int r = 0; r < 32; r += ROWS_PER_PASS) {
-          const int row = min(r + rd_row, 31);
-          const int m = m0 + wm * WM + i * 32 + row;
-          // 8-byte LDS reads: the padded row pitch keeps rows 8-byte, not 16-byte, aligned
-          const uint2 lo = *reinterpret_cast<const uint2*>(patch + row * PATCH_ROW + rd_chunk * 16);
-          const uint2 hi = *reinterpret_cast<const uint2*>(patch + row * PATCH_ROW + rd_chunk * 16 + 8);
-          // streaming stores: the tile is not read again by this kernel, and whoever reads
-          // it next (the norm kernel) runs on other XCDs; 1 - 3.5 % faster than default stores
-          if (rd_lane && r + rd_row < 32 && m < M && n < N) {
-            u32x4_t v = {lo.x, lo.y, hi.x, hi.y};
-            if (bias) v = u32x4_t{add_bias2(lo.x, bv.x), add_bias2(lo.y, bv.y), add_bias2(hi.x, bv.z),
-                                  add_bias2(hi.y, bv.w)};
-            __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(out + (size_t)m * ldc + n));
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
-      continue;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int m = m0 + wm * WM + i * 32 + l32;
-      if (m >= M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n0 + wn * WN + j * 32 + 8 * q + 4 * lhi;
-          if (n < N) {
-            uint2 v;
-            v.x = pack2(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1]);
-            v.y = pack2(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-            if (bias) {
-              const uint2 bv = *reinterpret_cast<const uint2*>(bias + n);
-              v.x = add_bias2(v.x, bv.x);
-              v.y = add_bias2(v.y, bv.y);
-            }
-            *reinterpret_cast<uint2*>(out + (size_t)m * ldc + n) = v;
-          }
-        }
-      }
+    const TilePlace p = tile_place<TM, TN>(t, num_tiles, tiles_m, tiles_n);
+    const uint16_t* __restrict__ bias = batch.bias[p.product];
+    const __amdgpu_buffer_rsrc_t dc = __builtin_amdgcn_make_buffer_rsrc(
+        batch.out[p.product] + (size_t)p.m0 * ldc + p.n0, 0, (uint32_t)min(M - p.m0, S::BM) * (uint32_t)ldc * 2u,
+        0x00020000);
+    const int col = wn * 16 * TN + quad * 8;
+    const uint32_t row_off = (uint32_t)((wm * 16 * TM + r16) * (int)ldc + col) * 2u, row_step = (uint32_t)ldc * 32u;
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result is written
+    if (bias) {
+      if (wide_store) tile_store<TM, TN, true, true>(acc, dc, row_off, row_step, p.n0 + col, N, bias);
+      else tile_store<TM, TN, false, true>(acc, dc, row_off, row_step, p.n0 + col, N, bias);
+    } else {
+      if (wide_store) tile_store<TM, TN, true, false>(acc, dc, row_off, row_step, p.n0 + col, N, bias);
+      else tile_store<TM, TN, false, false>(acc, dc, row_off, row_step, p.n0 + col, N, bias);
     }
   }
+#undef TW_TILE_SLAB
+#undef TW_RING
+#undef TW_TILE_ADVANCE
+#undef TW_TILE_DESCRIPTORS
+#undef TW_TILE_OFFSETS
+#endif
 }
 
 // More than 64 KiB of dynamic LDS must be allowed once per function and device.
@@ -756,74 +748,78 @@ static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64
 }
 
 template <int TM, int TN>
-static int launch_big(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
-                      int max_cus, hipStream_t hs) {
-  constexpr int BM = 64 * TM, BN = 128 * TN;
-  constexpr int LDS = big_lds_bytes(TM, TN);
+static int launch_tile(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
+                       int max_cus, hipStream_t hs) {
+  using S = TileShape<TM, TN>;
   static std::atomic<bool> lds_ok[kMaxDevices];
-  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_big_kernel<TM, TN>), lds_ok, kMaxDevices, LDS))
+  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<TM, TN>), lds_ok, kMaxDevices, S::LDS))
     return rc;
-  const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
-  int64_t grid = (int64_t)count * tiles_m * tiles_n;
-  if (max_cus > 0 && grid > max_cus) grid = max_cus;
+  const int tiles_m = (int)((M + S::BM - 1) / S::BM), tiles_n = (int)((N + S::BN - 1) / S::BN);
+  // a workgroup per compute unit at most: it fills the unit and walks its share of the tiles
+  int cus = max_cus > 0 ? max_cus : device_compute_units();
+  if (cus <= 0) cus = 256;
+  const int64_t grid = std::min<int64_t>((int64_t)count * tiles_m * tiles_n, cus);
   // 16-byte stores need 16-byte aligned row segments that end inside the row
   int wide_store = (N % 8 == 0 && ldc % 8 == 0) ? 1 : 0;
   for (int p = 0; p < count; ++p)
-    if ((reinterpret_cast<uintptr_t>(batch.out[p]) | reinterpret_cast<uintptr_t>(batch.bias[p])) & 15u) wide_store = 0;
-  launch_kernel(gemm_bf16_nt_big_kernel<TM, TN>, dim3((unsigned)grid), dim3(BIG_THREADS), LDS, hs, batch, count,
+    if (reinterpret_cast<uintptr_t>(batch.out[p]) & 15u) wide_store = 0;
+  launch_kernel(gemm_bf16_nt_tile_kernel<TM, TN>, dim3((unsigned)grid), dim3(TILE_THREADS), S::LDS, hs, batch, count,
                 (int)M, (int)N, (int)K, ldc, tiles_m, tiles_n, wide_store);
   return TW_OK;
 }
 
-// Workgroup tile for the problem, (64 TM) x (128 TN).  Cost = rounds x (tile area /
-// relative throughput + a fixed part per round); ties go to the earlier entry.  The
-// 64-wide wave tiles come in four heights so that a tile count can be made to fit the
-// compute units exactly (M = 2458: 320-row tiles make 256 tiles; the 128-row tile loads
-// 30 % more operand bytes per flop than the 192-row one and is rated 0.85); 256 x 384 (96-wide
-// wave tiles, 192 accumulators, exactly 160 KiB of LDS) wins where its fewer, larger
-// rounds fit.  96 x 96 wave tiles (192 x 384) were measured no faster per area than
-// 256 x 256 and are not offered.
-struct BigTile { int tm, tn; };
+// The tile shapes, in 32-row and 32-column units, with the time a round of them takes on all
+// compute units relative to 256 x 256 tiles, measured at K = 3584 with one tile per unit.  The
+// heights and widths are there to make a tile count fit the units: 192 x 256 (M = 1500), 160 x 256
+// (M = 2458: 512 tiles) and the 192-wide ones for N = 6144, whose 24 columns of 256 leave a quarter
+// of the units idle; the small ones for M <= 512 at N = 8192 (64 x 128, 96 x 128, 128 x 128: 256
+// tiles for 256, 384 and 512 rows).
+struct TileChoice { int tm, tn; double cost; };
+#define TW_TILES(X)                                                                                            \
+  X(8, 8, 1.0) X(6, 8, 0.79) X(8, 6, 0.77) X(5, 8, 0.69) X(6, 6, 0.65) X(4, 8, 0.58) X(3, 8, 0.48) X(4, 6, 0.46) \
+  X(3, 6, 0.41) X(4, 4, 0.365) X(3, 4, 0.315) X(2, 4, 0.25)
+#define TW_TILE_CHOICE(TM, TN, COST) {TM, TN, COST},
+constexpr TileChoice kTiles[] = {TW_TILES(TW_TILE_CHOICE)};
+#undef TW_TILE_CHOICE
 
-static BigTile pick_big_tile(int64_t M, int64_t N, int count, int cus) {
-  // Relative throughput per tile area, measured: the 256 x 384 tile loads a fifth fewer
-  // operand bytes per flop and runs a round in 1.35x the time of a 256 x 256 round.
-  static const struct { int tm, tn; double eff; } kTiles[] = {
-      {2, 2, 0.85}, {3, 2, 1.0}, {4, 2, 1.0}, {5, 2, 1.0}, {4, 3, 1.1}};
-  BigTile best = {4, 2};
+static int launch_tile_shape(int tm, int tn, const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K,
+                             int64_t ldc, int max_cus, hipStream_t hs) {
+#define TW_TILE_LAUNCH(TM, TN, COST) \
+  if (tm == TM && tn == TN) return launch_tile<TM, TN>(batch, count, M, N, K, ldc, max_cus, hs);
+  TW_TILES(TW_TILE_LAUNCH)
+#undef TW_TILE_LAUNCH
+  return set_error(TW_ERR_INVALID_ARGUMENT, "gemm_bf16_nt: no %d x %d tile", 32 * tm, 32 * tn);
+}
+
+// The shape whose rounds over the available units take the least time; ties go to the earlier
+// (larger) one.  The shape never changes a result bit: every output element is the same sequence
+// of MFMA k-steps whatever tile it lies in.
+static const TileChoice& pick_tile(int64_t M, int64_t N, int count, int cus) {
+  const TileChoice* best = &kTiles[0];
   double best_cost = 1e300;
-  for (const auto& t : kTiles) {
-    const int64_t tiles = count * ((M + 64 * t.tm - 1) / (64 * t.tm)) * ((N + 128 * t.tn - 1) / (128 * t.tn));
-    const int64_t rounds = (tiles + cus - 1) / cus;
-    const double cost = (double)rounds * (64.0 * t.tm * 128.0 * t.tn / t.eff + 2048.0);
+  for (const TileChoice& t : kTiles) {
+    const int64_t tiles = count * ((M + 32 * t.tm - 1) / (32 * t.tm)) * ((N + 32 * t.tn - 1) / (32 * t.tn));
+    const double cost = (double)((tiles + cus - 1) / cus) * t.cost;
     if (cost < best_cost) {
       best_cost = cost;
-      best = BigTile{t.tm, t.tn};
+      best = &t;
     }
   }
-  return best;
+  return *best;
 }
 
-// The tile shape never changes a result bit: every output element is the same sequence of
-// MFMA k-steps whatever tile it lies in.
-static bool big_kernel_fits(int64_t M, int64_t N, int64_t K) {
-  // at least one whole 64-wide k-slab, 32-bit byte offsets into both operands (below the
-  // out-of-range marker when a last partial slab has to be zero-filled), and enough rows and
-  // columns to be worth the larger prologue
-  const uint64_t limit = (K % BIG_BK == 0) ? (1ull << 31) : (1ull << 30);  // elements per operand
-  return K >= BIG_BK && (uint64_t)M * K < limit && (uint64_t)N * K < limit && M > 256 && N >= 192;
+// Which of the two families runs is decided by M, N and K alone (their sums differ in the order of
+// the additions): a product has the same bits under every grid cap and in every batch.
+static bool tile_kernel_fits(int64_t M, int64_t N, int64_t K, int64_t ldc) {
+  return K <= TILE_MAX_K && ldc <= TILE_MAX_LDC && M > 128 && N >= 64;
 }
 
-static int launch_big_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
-                          int max_cus, hipStream_t hs) {
+static int launch_tile_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
+                           int max_cus, hipStream_t hs) {
   int cus = max_cus > 0 ? max_cus : device_compute_units();
   if (cus <= 0) cus = 256;
-  const BigTile bt = pick_big_tile(M, N, count, cus);
-  if (bt.tn == 3) return launch_big<4, 3>(batch, count, M, N, K, ldc, max_cus, hs);
-  if (bt.tm == 2) return launch_big<2, 2>(batch, count, M, N, K, ldc, max_cus, hs);
-  if (bt.tm == 3) return launch_big<3, 2>(batch, count, M, N, K, ldc, max_cus, hs);
-  if (bt.tm == 5) return launch_big<5, 2>(batch, count, M, N, K, ldc, max_cus, hs);
-  return launch_big<4, 2>(batch, count, M, N, K, ldc, max_cus, hs);
+  const TileChoice& t = pick_tile(M, N, count, cus);
+  return launch_tile_shape(t.tm, t.tn, batch, count, M, N, K, ldc, max_cus, hs);
 }
 
 static int check_gemm_shape(const char* what, int64_t M, int64_t N, int64_t K, int64_t ldc) {
@@ -846,8 +842,8 @@ static int check_gemm_pointers(const char* what, const void* out, const void* a,
 
 static int run_products(const char* what, const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K,
                         int64_t ldc, int max_cus, hipStream_t hs) {
-  if (big_kernel_fits(M, N, K)) {
-    if (int rc = launch_big_for(batch, count, M, N, K, ldc, max_cus, hs)) return rc;
+  if (tile_kernel_fits(M, N, K, ldc)) {
+    if (int rc = launch_tile_for(batch, count, M, N, K, ldc, max_cus, hs)) return rc;
     return finish_launch(what);
   }
   if (K <= KS_MAX_K) {
