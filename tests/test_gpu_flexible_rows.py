@@ -1,0 +1,83 @@
+"""The flexible vector norm kernel: fp32, hidden sizes and addresses that are not 16-byte aligned, at the
+edges of its vectors, lanes and registers.
+
+The reference is float64 arithmetic with the op's rounding points.  In 16-bit types the residual is one
+rounding of an exact sum of two (bit-exact) and y may be one unit in the last place off where the fp32
+value lies next to a rounding boundary; in fp32 the residual is exact and y carries the error of a
+sum of H squares and a handful of operations: 2^-24 (H / 64 + 16) relative (the longest chain of additions
+is H / 64 / 8 vectors deep, with room)."""
+import pytest
+import torch
+
+from tokenweave_amd import _custom_ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+EPS = 1e-5
+# one element .. whole vectors +- 1, one wave +- 1 vector, two vectors per lane full (2048 vectors)
+# and one more, four per lane full (4096) and one more: the element-wise kernel
+SIZES_16 = [1, 7, 8, 9, 511, 513, 1025, 5125, 8199, 16383, 16385, 32767, 32769]
+SIZES_32 = [1, 3, 4, 5, 255, 257, 2051, 5120, 8191, 8193, 16383, 16384, 16385]
+
+
+def offset_rows(T, H, dtype, g, shift):
+    """[T, H] that begins `shift` elements behind an aligned address, in a buffer whose other
+    elements must survive."""
+    flat = torch.full((T * H + 32,), 7.0, device=DEV, dtype=dtype)
+    flat[shift:shift + T * H].copy_(torch.randn(T * H, generator=g, device=DEV))
+    return flat, flat[shift:shift + T * H].view(T, H)
+
+
+def untouched(flat, shift, n):
+    return bool((flat[:shift] == 7).all() and (flat[shift + n:] == 7).all())
+
+
+@pytest.mark.parametrize("dtype,H", [(d, h) for d in (torch.bfloat16, torch.float16) for h in SIZES_16]
+                         + [(torch.float32, h) for h in SIZES_32])
+@pytest.mark.parametrize("T,shift", [(3, 0), (2, 1)])
+def test_add_norm(dtype, H, T, shift):
+    print(f"[case] flex {dtype} T={T} H={H} shift={shift}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(H * 3 + shift)
+    fx, x = offset_rows(T, H, dtype, g, shift)
+    fr, r = offset_rows(T, H, dtype, g, shift)
+    _, w = offset_rows(1, H, dtype, g, shift)
+    s = x.double() + r.double()
+    want_r = s.to(dtype)
+    ref = (want_r.double() / torch.sqrt(s.pow(2).mean(-1, keepdim=True) + EPS) * w.double())
+    ops.fused_add_rms_norm(x, r, w.view(-1), EPS)
+    torch.cuda.synchronize()
+    assert torch.equal(r, want_r)
+    if dtype == torch.float32:
+        bound = ref.abs() * (2.0 ** -24 * (H / 64 + 16))
+    else:
+        bound = ref.abs() * (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10) + 1e-7
+    assert bool(((x.double() - ref).abs() <= bound).all())
+    assert untouched(fx, shift, T * H) and untouched(fr, shift, T * H)
+
+
+@pytest.mark.parametrize("H", [9, 1025, 4104])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_every_output_kind_equals_the_plain_result(dtype, H):
+    """rms_norm, the in-place form, both static fp8 ops: the same normalised values, copied or
+    quantised; capped grids walk the same rows."""
+    T = 5
+    g = torch.Generator(device=DEV).manual_seed(H)
+    x, r = (torch.randn(T, H, generator=g, device=DEV).to(dtype) for _ in range(2))
+    w = torch.randn(H, generator=g, device=DEV).to(dtype)
+    y = torch.empty_like(x)
+    ops.rms_norm(y, x, w, EPS)
+    x2, copy = x.clone(), torch.empty_like(x)
+    ops.rms_norm_inplace(copy, x2, w, EPS)
+    assert torch.equal(x2, y) and torch.equal(copy, x)
+    scale = torch.tensor([0.03], device=DEV)
+    code = torch.empty(T, H, device=DEV, dtype=torch.float8_e4m3fn)
+
+    def quantised(t):
+        return (t.float() * (1.0 / scale)).clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8)
+    ops.rms_norm_static_fp8_quant(code, x, w, scale, EPS)
+    assert torch.equal(code.view(torch.uint8), quantised(y))
+    xa, ra = x.clone(), r.clone()
+    ops.fused_add_rms_norm(xa, ra, w, EPS)
+    rb = r.clone()
+    ops.fused_add_rms_norm_static_fp8_quant(code, x, rb, w, scale, EPS)
+    assert torch.equal(code.view(torch.uint8), quantised(xa)) and torch.equal(ra, rb)
