@@ -310,6 +310,28 @@ __device__ __forceinline__ uint32_t quant4_fp8_div(float a, float b, float c, fl
   return (uint32_t)r;
 }
 
+// The same quotients from the row's reciprocal y = RN(1 / scale): one product and one
+// correction from its exact remainder give the correctly rounded x / scale in three
+// operations, the division takes eleven.  For 16-bit x and a scale that is a 16-bit
+// maximum over 448 (or the floor) that was checked over every pair of significands.  The
+// remainder is taken with the sign that keeps -0.  row_scale_plain() says where it may
+// be used: no quotient then passes 448 by more than an ulp, which rounds to the code
+// of 448, so of the clamp only the half that turns NaN into 448 is left.
+__device__ __forceinline__ float quotient(float x, float scale, float y) {
+  const float q = x * y;
+  return fminf(__builtin_fmaf(-__builtin_fmaf(q, scale, -x), y, q), kFp8Max);
+}
+
+__device__ __forceinline__ bool row_scale_plain(float amax, float ub, float scale) {
+  return amax <= ub && scale < 1e36f;
+}
+
+__device__ __forceinline__ uint32_t quant4_fp8_plain(float a, float b, float c, float d, float scale, float y) {
+  int r = __builtin_amdgcn_cvt_pk_fp8_f32(quotient(a, scale, y), quotient(b, scale, y), 0, false);
+  r = __builtin_amdgcn_cvt_pk_fp8_f32(quotient(c, scale, y), quotient(d, scale, y), r, true);
+  return (uint32_t)r;
+}
+
 // Round to nearest even, saturate (quant_conversions.cuh:14-32).
 __device__ __forceinline__ uint32_t quant1_int8(float x, float scale_inv) {
   float q = fmaxf(-128.0f, fminf(__builtin_rintf(x * scale_inv), 127.0f));
@@ -502,6 +524,7 @@ __device__ __forceinline__ void row_norm_vec_body(
       const float scale = dyn_scale(fminf(amax, qparam), nullptr, Q == kQDynInt8);
       if (threadIdx.x == 0) row_scales[row] = scale;
       const float sinv = 1.0f / scale;
+      const bool plain = row_scale_plain(amax, qparam, scale);
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
         float n[8];
@@ -509,6 +532,9 @@ __device__ __forceinline__ void row_norm_vec_body(
         if (Q == kQDynInt8)
           store8(dy, off[k] / 2, quant4_int8(n[0], n[1], n[2], n[3], sinv),
                  quant4_int8(n[4], n[5], n[6], n[7], sinv));
+        else if (plain)
+          store8(dy, off[k] / 2, quant4_fp8_plain(n[0], n[1], n[2], n[3], scale, sinv),
+                 quant4_fp8_plain(n[4], n[5], n[6], n[7], scale, sinv));
         else
           store8(dy, off[k] / 2, quant4_fp8_div(n[0], n[1], n[2], n[3], scale),
                  quant4_fp8_div(n[4], n[5], n[6], n[7], scale));
@@ -971,13 +997,17 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
       const float scale = dyn_scale(fminf(amax, qparam), nullptr, Q == kQDynInt8);
       if (threadIdx.x == 0) row_scales[row] = scale;
       const float sinv = 1.0f / scale;
+      const bool plain = sizeof(T) == 2 && row_scale_plain(amax, qparam, scale);
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
         uint32_t c[NE / 4];
 #pragma unroll
-        for (int g = 0; g < NE / 4; ++g)
-          c[g] = Q == kQDynInt8 ? quant4_int8(s[k][4 * g], s[k][4 * g + 1], s[k][4 * g + 2], s[k][4 * g + 3], sinv)
-                                : quant4_fp8_div(s[k][4 * g], s[k][4 * g + 1], s[k][4 * g + 2], s[k][4 * g + 3], scale);
+        for (int g = 0; g < NE / 4; ++g) {
+          const float *v = &s[k][4 * g];
+          c[g] = Q == kQDynInt8 ? quant4_int8(v[0], v[1], v[2], v[3], sinv)
+                 : plain        ? quant4_fp8_plain(v[0], v[1], v[2], v[3], scale, sinv)
+                                : quant4_fp8_div(v[0], v[1], v[2], v[3], scale);
+        }
         flex_store_codes<NE>(static_cast<uint8_t*>(y_out) + base + first[k], c, n[k]);
       }
     } else {
