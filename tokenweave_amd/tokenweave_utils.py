@@ -324,8 +324,13 @@ def tokenweave_overlap(
     the tokens are cut at `split_size`; while one split computes (attention, MLP) on
     `current_stream`, the fused reduce + add + norm of the other runs on
     `copy_stream`.  Every compute step ends with `current_stream.wait_stream(copy_stream)`
-    and every norm starts with `copy_stream.wait_stream(current_stream)`, exactly as
+    and every norm waits for what `current_stream` held before that step, exactly as
     in the reference, so the result equals the unsplit schedule's.
+
+    Within a stage the compute is enqueued first and the norm second; the reference does it
+    the other way round.  A projection's workgroup needs a whole compute unit, and while
+    a norm of thousands of one-row workgroups is being handed out no unit ever falls
+    empty: enqueued second, the projection starts when the norm ends.
 
     Layer 0 (reference :203-226): split 0 has nothing to reduce and takes
     `input_layernorm(x, out=residual)`; for split 1 the reference reduce-scatters,
@@ -369,41 +374,37 @@ def tokenweave_overlap(
             num_tokens_per_rank=blpr, rank=rank, world_size=world_size, MAX_CTAS=max_ctas,
             offset_symm_mem=off, row_range=rows)
 
+    def attention(split):
+        hs, rows = (hidden_states_1, positions[:split_size]) if split == 0 else (hidden_states_2, positions[split_size:])
+        self.self_attn(positions=rows, hidden_states=hs, split_id=split, split_size=split_size,
+                       num_actual_tokens=split_size if split == 0 else actual_tokens - split_size, **budget)
+
+    def mlp(split):
+        mlp_fn(hidden_states_1 if split == 0 else hidden_states_2, **mlp_budget)
+
+    def stage(compute, split, *norm_args):
+        """`compute` of one split beside the norm of the other: the norm waits for what was queued
+        before the stage, the next stage for both."""
+        before = current_stream.record_event()
+        with torch.cuda.stream(current_stream):
+            compute(split)
+        copy_stream.wait_event(before)
+        with torch.cuda.stream(copy_stream):
+            norm(*norm_args)
+        current_stream.wait_stream(copy_stream)
+
     if layer_id == 0:
         self.input_layernorm(hidden_states_1, out=residual_1)
         residual_2.zero_()
         norm(self.input_layernorm, 1, 0)
+        with torch.cuda.stream(current_stream):
+            attention(0)
+            current_stream.wait_stream(copy_stream)
     else:
-        with torch.cuda.stream(copy_stream):
-            copy_stream.wait_stream(current_stream)
-            norm(self.input_layernorm, 1, MAX_CTAS_ATTN)
-
-    with torch.cuda.stream(current_stream):
-        self.self_attn(positions=positions[:split_size], hidden_states=hidden_states_1, split_id=0,
-                       split_size=split_size, num_actual_tokens=split_size, **budget)
-        current_stream.wait_stream(copy_stream)
-    with torch.cuda.stream(copy_stream):
-        copy_stream.wait_stream(current_stream)
-        norm(self.post_attention_layernorm, 0, MAX_CTAS_ATTN)
-
-    with torch.cuda.stream(current_stream):
-        self.self_attn(positions=positions[split_size:], hidden_states=hidden_states_2, split_id=1,
-                       split_size=split_size, num_actual_tokens=actual_tokens - split_size, **budget)
-        current_stream.wait_stream(copy_stream)
-    with torch.cuda.stream(copy_stream):
-        copy_stream.wait_stream(current_stream)
-        norm(self.post_attention_layernorm, 1, MAX_CTAS_MLP)
-
-    with torch.cuda.stream(current_stream):
-        mlp_fn(hidden_states_1, **mlp_budget)
-        current_stream.wait_stream(copy_stream)
-    with torch.cuda.stream(copy_stream):
-        copy_stream.wait_stream(current_stream)
-        norm(next_layer_norm, 0, MAX_CTAS_MLP)
-
-    with torch.cuda.stream(current_stream):
-        mlp_fn(hidden_states_2, **mlp_budget)
-        current_stream.wait_stream(copy_stream)
+        stage(attention, 0, self.input_layernorm, 1, MAX_CTAS_ATTN)
+    stage(attention, 1, self.post_attention_layernorm, 0, MAX_CTAS_ATTN)
+    stage(mlp, 0, self.post_attention_layernorm, 1, MAX_CTAS_MLP)
+    stage(mlp, 1, next_layer_norm, 0, MAX_CTAS_MLP)
 
     if layer_id == end_layer - 1:
         with torch.cuda.stream(current_stream):
