@@ -607,8 +607,9 @@ __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THR
       vb[l] = c < (chunks) ? (uint32_t)((blk * 8 + (lane >> 3)) * K + c * 8) * 2u : TILE_OUT_OF_RANGE;       \
     }                                                                                                        \
   } while (0)
-  // Load cursor: slab lk of tile lt.  Past the last tile the descriptors are empty and the loads
-  // ask memory for nothing.
+  // Load cursor: slab lk of tile lt.  Past the last tile it stays at slab 0 of an empty descriptor:
+  // its loads ask memory for nothing.  (The hardware compares with the extent less the slab's offset,
+  // which for an extent of 0 must not go below 0.)
   int lt = blockIdx.x, lk = 0;
   __amdgpu_buffer_rsrc_t da, db;
 #define TW_TILE_DESCRIPTORS()                                                                                \
@@ -624,7 +625,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THR
   } while (0)
 #define TW_TILE_ADVANCE()                                                                                    \
   do {                                                                                                       \
-    ++lk;                                                                                                    \
+    if (lt < num_tiles) ++lk;                                                                                \
     if (lk == nk) {                                                                                          \
       lk = 0;                                                                                                \
       lt += gridDim.x;                                                                                       \
