@@ -898,7 +898,7 @@ def time_gemm_only(device, steps=200):
 
 
 def time_gemm_limits(device):
-    """What the big GEMM kernel's k loop can reach by itself on this GPU: the loop of the 320 x 256 tile
+    """What the k loop of an eight-wave GEMM can reach by itself on this GPU: the loop of the 320 x 256 tile
     put together from its parts, every compute unit busy, operands served by the L2s, no tile prologue
     or epilogue.  TFLOP/s from HIP events around the launch; cycles and clock from the kernel's own stamps.
     Also the rate at which 1 .. 16 waves of a compute unit get the loop's 16-byte LDS reads through."""

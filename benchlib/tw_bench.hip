@@ -213,7 +213,7 @@ __global__ __launch_bounds__(64) void clock_probe_kernel(long long* out, long lo
 }
 
 
-// The k loop of gemm_bf16_nt_big_kernel<5, 2> (eight waves, 160 x 64 wave tiles, 320 x 256 x 64
+// The k loop of an eight-wave GEMM (2 x 4 waves, 160 x 64 wave tiles, 320 x 256 x 64
 // slabs, two LDS stages) assembled from switchable parts; the arithmetic result is
 // meaningless.  parts bit 0: fragment reads from LDS (else the MFMAs reuse their first
 // operands); bit 1: the slab loads global -> LDS (from a `window`-byte region per XCD, so

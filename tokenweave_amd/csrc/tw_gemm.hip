@@ -436,7 +436,9 @@ struct TileShape {
   // Two whole stages only: a third a panel, so that a's loads can go out in the phase before the
   // barrier, b's in the one behind it.
   static constexpr bool TIGHT = STAGES == 2;
-  static constexpr int D = TIGHT ? 2 : (STAGES - 1 < 3 ? STAGES - 1 : 3);  // slabs ahead
+  // slabs ahead; three at most: with four or five the 64- to 128-row tiles take longer to start than they
+  // gain ([256, 1024] x [8192, 1024]^T 8.3 -> 8.8 us, [160, 3584] x [8192, 3584]^T 18.2 -> 18.8)
+  static constexpr int D = TIGHT ? 2 : (STAGES - 1 < 3 ? STAGES - 1 : 3);
   static constexpr int SA = D + 1, SB = TIGHT ? D : D + 1;
   static constexpr int LDS = SA * PA + SB * PB;
   static constexpr int SPREAD = 2 * SLOTS / L;
@@ -567,7 +569,9 @@ __device__ __forceinline__ TilePlace tile_place(int t, int num_tiles, int tiles_
 #endif
 
 // TAIL: the last slab is a partial one.  (Apart from the others because switching the offsets costs
-// the k loop a register move per load and slab: 341 against 324 us for 8192 x 8192 x 3584.)
+// the k loop a register move per load and slab: 341 against 324 us for 8192 x 8192 x 3584.  Zeroing the
+// fragments instead needs no moves and is no faster, 227 against 230 us for 16384 x 8192 x 1000: what such
+// a K costs is that its rows are not whole lines, 46 against 58 us for 1000 rows at K = 3584 and 3696.)
 template <int TM, int TN, bool TAIL>
 __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THREADS) void gemm_bf16_nt_tile_kernel(
     GemmBatch batch, int count, int M, int N, int K, int64_t ldc, int tiles_m, int tiles_n, int wide_store) {
