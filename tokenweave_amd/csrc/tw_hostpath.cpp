@@ -399,22 +399,38 @@ PyObject* row_parallel_inplace(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return yes_no(enqueue([&] { tw_torch::gemm_bf16_nt(*o, *x, weight, cus, bias ? &bias_held : nullptr); }));
 }
 
-#define TW_FAST(name, fn) {name, (PyCFunction)(void (*)(void))(fn), METH_FASTCALL, nullptr}
+// What Python calls.  Some tensors throw when they are asked for a size (nested ones have none), and
+// no C++ exception may leave through C frames: it would end the process.  Nothing is enqueued
+// then, so the answer is that the call was not made: NotImplemented where a call has a RESULT,
+// False where it only says whether it was made.
+typedef PyObject* (*Fast)(PyObject*, PyObject* const*, Py_ssize_t);
+template <Fast FN, bool RESULT>
+PyObject* entry(PyObject* self, PyObject* const* a, Py_ssize_t n) noexcept {
+  try {
+    return FN(self, a, n);
+  } catch (...) {
+    return RESULT ? not_handled() : yes_no(false);
+  }
+}
+
+#define TW_ENTRY(name, fn, result) {name, (PyCFunction)(void (*)(void))(entry<fn, result>), METH_FASTCALL, nullptr}
+#define TW_FAST(name, fn) TW_ENTRY(name, (fn), false)
+#define TW_FAST_RESULT(name, fn) TW_ENTRY(name, (fn), true)
 PyMethodDef g_methods[] = {
-    TW_FAST("rms_norm", (norm3<tw_torch::rms_norm>)),
-    TW_FAST("fused_add_rms_norm", (norm3<tw_torch::fused_add_rms_norm>)),
-    TW_FAST("rms_norm_inplace", (norm3<tw_torch::rms_norm_inplace>)),
+    TW_FAST("rms_norm", norm3<tw_torch::rms_norm>),
+    TW_FAST("fused_add_rms_norm", norm3<tw_torch::fused_add_rms_norm>),
+    TW_FAST("rms_norm_inplace", norm3<tw_torch::rms_norm_inplace>),
     TW_FAST("fused_add_rms_norm_cta", fused_add_rms_norm_cta),
-    TW_FAST("fused_rs_ln_ag_cta", (fused_rs_ln<true>)),
-    TW_FAST("fused_rs_ln_cta", (fused_rs_ln<false>)),
+    TW_FAST("fused_rs_ln_ag_cta", fused_rs_ln<true>),
+    TW_FAST("fused_rs_ln_cta", fused_rs_ln<false>),
     TW_FAST("rms_norm_static_fp8_quant", rms_norm_static_fp8_quant),
     TW_FAST("fused_add_rms_norm_static_fp8_quant", fused_add_rms_norm_static_fp8_quant),
     TW_FAST("rms_norm_dynamic_per_token_quant_out", rms_norm_dynamic_per_token_quant_out),
-    TW_FAST("rms_norm_dynamic_per_token_quant", rms_norm_dynamic_per_token_quant),
+    TW_FAST_RESULT("rms_norm_dynamic_per_token_quant", rms_norm_dynamic_per_token_quant),
     TW_FAST("gemm_bf16_nt", gemm_bf16_nt),
     TW_FAST("gemm_bf16_nt_partials", gemm_bf16_nt_partials),
-    TW_FAST("rms_norm_forward", rms_norm_forward),
-    TW_FAST("rms_norm_call", rms_norm_call),
+    TW_FAST_RESULT("rms_norm_forward", rms_norm_forward),
+    TW_FAST_RESULT("rms_norm_call", rms_norm_call),
     TW_FAST("fused_allreduce_layernorm", fused_allreduce_layernorm),
     TW_FAST("row_parallel_inplace", row_parallel_inplace),
     {nullptr, nullptr, 0, nullptr}};
