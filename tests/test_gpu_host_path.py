@@ -131,6 +131,32 @@ def test_hooks_autograd_and_dispatch_modes_take_the_ordinary_route(counted):
     assert counted["rms_norm"] == 1
 
 
+def test_a_lazily_negated_tensor_is_read_with_its_sign(counted):
+    """`torch._neg_view` only marks a tensor as negated; the dispatcher resolves the mark before an op
+    sees the storage, so such a tensor takes that route, whichever argument it is."""
+    x, r, layer = tensors(dtype=torch.float32)
+    w = layer.weight.data
+    want = torch.empty_like(x)
+    ops.rms_norm(want, torch.neg(x), w, 1e-6)
+    assert counted.pop("rms_norm") == 1
+    neg = torch._neg_view(x)
+    assert neg.is_neg() and neg.is_contiguous() and neg.data_ptr() == x.data_ptr()
+    got = torch.empty_like(x)
+    ops.rms_norm(got, neg, w, 1e-6)
+    assert torch.equal(got, want) and torch.equal(layer(neg), want)
+    sum_, res = torch.neg(x), r.clone()
+    ops.fused_add_rms_norm(sum_, res, w, 1e-6)
+    written, res2 = torch._neg_view(x.clone()), r.clone()
+    ops.fused_add_rms_norm(written, res2, w, 1e-6)      # an output: written back with its sign
+    assert torch.equal(written, sum_) and torch.equal(res, res2)
+    ops.rms_norm(got, x, torch._neg_view(w), 1e-6)
+    assert torch.equal(got, want)                        # -(x w) = (-x) w
+    codes, scales = ops.rms_norm_dynamic_per_token_quant(neg, w, 1e-6, torch.int8)
+    want_codes, want_scales = ops.rms_norm_dynamic_per_token_quant(torch.neg(x), w, 1e-6, torch.int8)
+    assert torch.equal(codes, want_codes) and torch.equal(scales, want_scales)
+    assert counted == {"fused_add_rms_norm": 1, "rms_norm_dynamic_per_token_quant": 1}   # of plain tensors
+
+
 def test_errors_are_those_of_the_ordinary_route():
     x, r, layer = tensors()
     with pytest.raises(RuntimeError, match="same shape"):

@@ -42,12 +42,19 @@ bool direct_allowed() {
          !at::hasCallbacks() && !torch::jit::tracer::isTracing();
 }
 
-// The tensor behind a plain torch.Tensor; `data`: one the op reads or writes as data (a weight is
-// taken by its values alone, as `.data` is).
+// The keys of a strided tensor whose storage on the GPU holds its values.  With any other key (a lazy
+// sign or conjugation, a tensor of zeros without storage, a nested, sparse or wrapped one) the
+// dispatcher has work to do before the op may read it.
+const c10::DispatchKeySet g_own_data({c10::DispatchKey::Dense, c10::DispatchKey::AutogradFunctionality,
+                                      c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutocastCUDA});
+
+// The tensor behind a plain torch.Tensor on the GPU; `data`: one the op reads or writes as data (a weight
+// is taken by its values alone, as `.data` is).
 const Tensor* plain(PyObject* o, bool data = true) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
-  if (!t.defined() || t.key_set().has(c10::DispatchKey::Python)) return nullptr;
+  if (!t.defined() || !t.is_cuda() || (t.key_set() - g_own_data).highestFunctionalityKey() != c10::DispatchKey::Undefined)
+    return nullptr;
   if (data && t.requires_grad() && at::GradMode::is_enabled()) return nullptr;
   return &t;
 }
