@@ -167,3 +167,22 @@ def test_errors_are_those_of_the_ordinary_route():
         tw.fused_allreduce_layernorm(layer, x, r, tw.PartialsBuffer(2, 5, H, device=DEV), 3, 0, 2, 0)
     with pytest.raises(RuntimeError, match="inner dimensions differ"):
         ops.gemm_bf16_nt(r, x, x[:, :8].contiguous())
+
+
+def test_the_handles_signal_pads_are_wanted_as_by_the_registered_op(counted):
+    """One GPU has no peers to signal, but a handle that cannot name its pads is refused."""
+    x, r, layer = tensors()
+    buf = tw.PartialsBuffer(1, 5, H, device=DEV)
+    with pytest.raises(RuntimeError, match="signal_pads"):
+        ops.fused_rs_ln_ag_cta(x, r, layer.weight.data, buf.multicast_ptr, "pads", 0, 1, 0, 1e-6)
+    with pytest.raises(RuntimeError, match="signal_pads"):
+        ops.fused_rs_ln_cta(x, r, layer.weight.data, buf.multicast_ptr, None, 0, 1, 0, 1e-6)
+
+    class Half:
+        multicast_ptr = buf.multicast_ptr
+    with pytest.raises(AttributeError, match="signal_pad_ptrs_dev"):
+        tw.fused_allreduce_layernorm(layer, x, r, Half(), 5, 0, 1, 0)
+    assert counted == {}
+    ops.fused_rs_ln_ag_cta(x, r, layer.weight.data, buf.multicast_ptr, 0, 0, 1, 0, 1e-6)
+    tw.fused_allreduce_layernorm(layer, x, r, buf, 5, 0, 1, 0)
+    assert counted == {"fused_rs_ln_ag_cta": 1, "fused_allreduce_layernorm": 1}

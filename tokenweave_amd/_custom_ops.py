@@ -870,16 +870,16 @@ if COMPILED_BINDING:
     def fused_rs_ln_ag_cta(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                            mcptr: int, signal_pads: int, rank: int, world_size: int, MAX_CTAS: int,
                            epsilon: float) -> None:
-        if _fast is None or _tracing() or not _fast.fused_rs_ln_ag_cta(input, residual, weight, mcptr, rank, world_size,
-                                                                          MAX_CTAS, epsilon):
+        if _fast is None or _tracing() or not _fast.fused_rs_ln_ag_cta(
+                input, residual, weight, mcptr, signal_pads, rank, world_size, MAX_CTAS, epsilon):
             _op_fused_rs_ln_ag_cta(input, residual, weight, mcptr, signal_pads, rank, world_size,
                                    0 if MAX_CTAS is None else MAX_CTAS, epsilon)
 
     def fused_rs_ln_cta(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,  # noqa: F811
                         mcptr: int, signal_pads: int, rank: int, world_size: int, MAX_CTAS: int,
                         epsilon: float) -> None:
-        if _fast is None or _tracing() or not _fast.fused_rs_ln_cta(input, residual, weight, mcptr, rank, world_size,
-                                                                       MAX_CTAS, epsilon):
+        if _fast is None or _tracing() or not _fast.fused_rs_ln_cta(
+                input, residual, weight, mcptr, signal_pads, rank, world_size, MAX_CTAS, epsilon):
             _op_fused_rs_ln_cta(input, residual, weight, mcptr, signal_pads, rank, world_size,
                                 0 if MAX_CTAS is None else MAX_CTAS, epsilon)
 

@@ -33,7 +33,7 @@ using at::Tensor;
 
 // Interned attribute names and torch.nn's global hook tables, looked up once.
 PyObject *s_parameters, *s_weight, *s_bias, *s_epsilon, *s_var_override, *s_forward, *s_compiled, *s_multicast,
-    *s_hooks[4], *s_tp_rank, *s_skip_bias, *s_input_parallel, *s_residual, *s_out;
+    *s_signal_pads, *s_hooks[4], *s_tp_rank, *s_skip_bias, *s_input_parallel, *s_residual, *s_out;
 PyObject* g_global_hooks[4];
 
 bool direct_allowed() {
@@ -69,6 +69,14 @@ bool as_int(PyObject* o, int64_t* v) {
 bool as_cap(PyObject* o, int64_t* v) {  // None: no cap
   *v = 0;
   return o == Py_None || as_int(o, v);
+}
+
+bool int_attribute(PyObject* o, PyObject* name, int64_t* v) {
+  PyObject* value = PyObject_GetAttr(o, name);
+  if (!value) PyErr_Clear();  // the ordinary route raises it
+  const bool got = value && as_int(value, v);
+  Py_XDECREF(value);
+  return got;
 }
 
 bool as_double(PyObject* o, double* v) {
@@ -136,15 +144,16 @@ PyObject* fused_add_rms_norm_cta(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return yes_no(enqueue([&] { tw_torch::fused_add_rms_norm_cta(mut(x), mut(r), mut(w), cap, eps); }));
 }
 
-// (input, residual, weight, mcptr, rank, world_size, MAX_CTAS, epsilon)
+// (input, residual, weight, mcptr, signal_pads, rank, world_size, MAX_CTAS, epsilon); the signal pads are
+// for peers, of which there are none: an integer, as the registered op wants it
 template <bool ALL_GATHER>
 PyObject* fused_rs_ln(PyObject*, PyObject* const* a, Py_ssize_t n) {
   double eps;
-  int64_t mcptr, rank, ws, cap;
-  if (n != 8 || !direct_allowed()) Py_RETURN_FALSE;
+  int64_t mcptr, pads, rank, ws, cap;
+  if (n != 9 || !direct_allowed()) Py_RETURN_FALSE;
   const Tensor *x = plain(a[0]), *r = plain(a[1]), *w = plain(a[2]);
-  if (!x || !r || !w || !as_int(a[3], &mcptr) || !as_int(a[4], &rank) || !as_int(a[5], &ws) || !as_cap(a[6], &cap) ||
-      !as_double(a[7], &eps) || x->dim() < 1 || x->size(-1) == 0)
+  if (!x || !r || !w || !as_int(a[3], &mcptr) || !as_int(a[4], &pads) || !as_int(a[5], &rank) || !as_int(a[6], &ws) ||
+      !as_cap(a[7], &cap) || !as_double(a[8], &eps) || x->dim() < 1 || x->size(-1) == 0)
     Py_RETURN_FALSE;
   const int64_t rows = x->numel() / x->size(-1);
   return yes_no(enqueue([&] { tw_torch::fused_rs_ln_rows(ALL_GATHER, *x, *r, *w, 0, rows, mcptr, rank, ws, cap, eps); }));
@@ -367,16 +376,11 @@ PyObject* fused_allreduce_layernorm(PyObject*, PyObject* const* a, Py_ssize_t n)
       Py_RETURN_FALSE;
   }
   if (rank < 0 || rank >= ws || start < 0 || start >= end || end > T) Py_RETURN_FALSE;
-  PyObject* base = PyObject_GetAttr(a[3], s_multicast);
-  int64_t mcptr;
-  const bool got = base && as_int(base, &mcptr);
-  Py_XDECREF(base);
-  if (!got) {
-    PyErr_Clear();
-    Py_RETURN_FALSE;
-  }
-  const int64_t rows = end - start;
+  // copied before the handle is asked, which may run Python code
   const Tensor weight = *w;
+  int64_t mcptr, pads;
+  if (!int_attribute(a[3], s_multicast, &mcptr) || !int_attribute(a[3], s_signal_pads, &pads)) Py_RETURN_FALSE;
+  const int64_t rows = end - start;
   return yes_no(enqueue([&] {
     tw_torch::fused_rs_ln_rows(true, *x, *r, weight, start, rows, mcptr + offset + start * H * 2, rank, ws,
                                std::min(cap, rows), eps);
@@ -448,8 +452,8 @@ bool init_names() {
   const struct { PyObject** at; const char* name; } names[] = {
       {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_bias, "bias"}, {&s_epsilon, "variance_epsilon"},
       {&s_var_override, "variance_size_override"}, {&s_forward, "forward"}, {&s_compiled, "_compiled_call_impl"},
-      {&s_multicast, "multicast_ptr"}, {&s_hooks[0], "_forward_hooks"}, {&s_hooks[1], "_forward_pre_hooks"},
-      {&s_hooks[2], "_backward_hooks"}, {&s_hooks[3], "_backward_pre_hooks"}, {&s_tp_rank, "tp_rank"},
+      {&s_multicast, "multicast_ptr"}, {&s_signal_pads, "signal_pad_ptrs_dev"}, {&s_hooks[0], "_forward_hooks"},
+      {&s_hooks[1], "_forward_pre_hooks"}, {&s_hooks[2], "_backward_hooks"}, {&s_hooks[3], "_backward_pre_hooks"}, {&s_tp_rank, "tp_rank"},
       {&s_skip_bias, "skip_bias_add"}, {&s_input_parallel, "input_is_parallel"},
       {&s_residual, "residual"}, {&s_out, "out"}};
   for (const auto& n : names)
