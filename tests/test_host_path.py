@@ -5,7 +5,9 @@ import subprocess
 import sys
 
 import pytest
+import torch
 
+import tokenweave_amd as tw
 from tokenweave_amd import _custom_ops as ops
 
 pytestmark = pytest.mark.skipif(ops._fast is None, reason="no compiled binding")
@@ -32,3 +34,34 @@ def test_a_tensor_without_sizes_is_refused_and_does_not_end_the_process():
     done = subprocess.run([sys.executable, "-c", NESTED], cwd=ROOT, capture_output=True, text=True, timeout=300,
                           env=dict(os.environ, PYTHONPATH=ROOT))
     assert done.returncode == 0 and "refused:" in done.stdout, done.stderr[-2000:]
+
+
+class AnsweredDirectly:
+    """In place of the direct calls: says of every call that it was made."""
+
+    def __getattr__(self, name):
+        return lambda *args: "direct"
+
+
+@pytest.fixture
+def layer(monkeypatch):
+    monkeypatch.setattr(ops, "_fast", AnsweredDirectly())
+    return tw.RMSNorm(8, dtype=torch.bfloat16)
+
+
+def fused(layer):
+    x = torch.zeros(4, 8, dtype=torch.bfloat16)
+    handle = tw.PartialsBuffer(1, 4, 8, device="cpu")
+    return tw.fused_allreduce_layernorm(layer, x, x.clone(), handle, 4, 0, 1, 0)
+
+
+@pytest.mark.parametrize("owner,name", [(tw.RMSNorm, "forward"), (tw.RMSNorm, "__call__"),
+                                        (torch.nn.Module, "__call__")])
+def test_a_replaced_forward_of_the_class_is_called(layer, monkeypatch, owner, name):
+    x = torch.zeros(4, 8, dtype=torch.bfloat16)
+    assert layer(x) == "direct" and fused(layer) is None
+    calls = []
+    monkeypatch.setattr(owner, name, lambda self, *args, **kwargs: calls.append(self) or "replaced")
+    assert layer(x) == "replaced" and calls == [layer]
+    fused(layer)
+    assert calls == [layer, layer]

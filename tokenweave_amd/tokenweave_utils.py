@@ -19,7 +19,7 @@ from typing import Any, Callable, Dict, Optional, Tuple
 import torch
 
 from . import _custom_ops as ops
-from .layernorm import RMSNorm
+from .layernorm import RMSNorm, _as_defined
 
 
 @lru_cache(maxsize=None)
@@ -170,7 +170,7 @@ def fused_allreduce_layernorm(
     split for ragged token counts (the reference pads instead, llama.py:536).
     """
     # one native call for the usual case; it takes no other than a plain RMSNorm on plain tensors
-    if (ops._fast is not None and type(layernorm) is RMSNorm and not ops._tracing()
+    if (ops._fast is not None and _as_defined(layernorm) and not ops._tracing()
             and ops._fast.fused_allreduce_layernorm(layernorm, hidden_states, residual, symm_mem_hdl,
                                                     num_tokens_per_rank, rank, world_size, MAX_CTAS,
                                                     offset_symm_mem, row_range)):
