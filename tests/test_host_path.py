@@ -65,3 +65,17 @@ def test_a_replaced_forward_of_the_class_is_called(layer, monkeypatch, owner, na
     assert layer(x) == "replaced" and calls == [layer]
     fused(layer)
     assert calls == [layer, layer]
+
+
+@pytest.mark.parametrize("of_the_class", [True, False])
+def test_a_replaced_apply_inplace_is_called(layer, monkeypatch, of_the_class):
+    lin = tw.RowParallelLinear(8, 8, bias=False)
+    x, out = (torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(2))
+    calls = []
+
+    def replaced(*args, **kwargs):
+        calls.append(kwargs["max_cus"])
+        return "replaced"
+    assert lin(x, out, is_tokenweave=True, gemm_cus=3) == (out, None) and calls == []
+    monkeypatch.setattr(type(lin.quant_method) if of_the_class else lin.quant_method, "apply_inplace", replaced)
+    assert lin(x, out, is_tokenweave=True, gemm_cus=3) == ("replaced", None) and calls == [3]

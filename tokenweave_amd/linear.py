@@ -15,7 +15,7 @@ the reference, is available only where that all-reduce is the identity.
 """
 from __future__ import annotations
 
-from typing import Optional, Tuple
+from typing import Any, Optional, Tuple
 
 import torch
 import torch.nn as nn
@@ -42,6 +42,16 @@ class UnquantizedLinearMethod:
         out2 = output if output.dim() == 2 else output.view(-1, output.shape[-1])
         ops.gemm_bf16_nt(out2, x2, w, max_cus, None if bias is None else bias.data)
         return output
+
+
+_APPLY_INPLACE = UnquantizedLinearMethod.apply_inplace
+
+
+def _is_unquantized(method: Any) -> bool:
+    """Whether `method.apply_inplace` is the one above: of that very class, replaced neither on it nor on
+    the instance."""
+    return (type(method) is UnquantizedLinearMethod and UnquantizedLinearMethod.apply_inplace is _APPLY_INPLACE
+            and "apply_inplace" not in method.__dict__)
 
 
 class RowParallelLinear(nn.Module):
@@ -90,7 +100,7 @@ class RowParallelLinear(nn.Module):
     def forward(self, input_: torch.Tensor, output_: Optional[torch.Tensor] = None,
                 is_tokenweave: Optional[bool] = False, gemm_cus: Optional[int] = None
                 ) -> Tuple[torch.Tensor, Optional[Parameter]]:
-        if (is_tokenweave and ops._fast is not None and type(self.quant_method) is UnquantizedLinearMethod
+        if (is_tokenweave and ops._fast is not None and _is_unquantized(self.quant_method)
                 and ops._fast.row_parallel_inplace(self, input_, output_, gemm_cus)):
             if not self.return_bias:
                 return output_
