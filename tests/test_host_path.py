@@ -79,3 +79,32 @@ def test_a_replaced_apply_inplace_is_called(layer, monkeypatch, of_the_class):
     assert lin(x, out, is_tokenweave=True, gemm_cus=3) == (out, None) and calls == []
     monkeypatch.setattr(type(lin.quant_method) if of_the_class else lin.quant_method, "apply_inplace", replaced)
     assert lin(x, out, is_tokenweave=True, gemm_cus=3) == ("replaced", None) and calls == [3]
+
+
+class NotUnderTracing:
+    def __getattr__(self, name):
+        raise AssertionError(f"the direct call {name} was made while tracing")
+
+
+def test_no_direct_call_while_dynamo_traces(monkeypatch):
+    """On CPU tensors every ordinary route ends in its own error."""
+    monkeypatch.setattr(ops, "_fast", NotUnderTracing())
+    monkeypatch.setattr(ops, "_tracing", lambda: True)
+    x, out = (torch.zeros(4, 8, dtype=torch.bfloat16) for _ in range(2))
+    w, scale = torch.ones(8, dtype=torch.bfloat16), torch.ones(1)
+    layer, lin = tw.RMSNorm(8, dtype=torch.bfloat16), tw.RowParallelLinear(8, 8, bias=False)
+    code = torch.empty(4, 8, dtype=torch.float8_e4m3fn)
+    for call in (lambda: layer(x), lambda: layer(x, out), lambda: fused(layer),
+                 lambda: lin(x, out, is_tokenweave=True),
+                 lambda: ops.gemm_bf16_nt(out, x, lin.weight.data),
+                 lambda: ops.gemm_bf16_nt_partials([out], [x], [lin.weight.data]),
+                 lambda: ops.rms_norm(out, x, w, 1e-6), lambda: ops.rms_norm_inplace(out, x, w, 1e-6),
+                 lambda: ops.fused_add_rms_norm(x, out, w, 1e-6),
+                 lambda: ops.fused_add_rms_norm_cta(x, out, w, 0, 1e-6),
+                 lambda: ops.fused_rs_ln_cta(x, out, w, 0, 0, 0, 1, 0, 1e-6),
+                 lambda: ops.fused_rs_ln_ag_cta(x, out, w, 0, 0, 0, 1, 0, 1e-6),
+                 lambda: ops.rms_norm_static_fp8_quant(code, x, w, scale, 1e-6),
+                 lambda: ops.fused_add_rms_norm_static_fp8_quant(code, x, out, w, scale, 1e-6),
+                 lambda: ops.rms_norm_dynamic_per_token_quant(x, w, 1e-6, torch.int8)):
+        with pytest.raises(RuntimeError, match="on the GPU only"):
+            call()

@@ -58,7 +58,8 @@ if COMPILED_BINDING:
     except ImportError as e:
         warnings.warn(f"the direct calls could not be loaded ({e}); tokenweave_amd calls its ops through "
                       "torch.ops instead", RuntimeWarning)
-# Under torch.compile the registered op must be traced, not the direct call.
+# Under torch.compile the ordinary routes are traced, not the direct calls: dynamo warns of a native
+# function that it does not know, and breaks the graph there.
 _tracing = torch.compiler.is_dynamo_compiling
 
 # Message of the reference's launchers (csrc/tokenweave_fused_kernels.cu:259).
@@ -711,7 +712,7 @@ def gemm_bf16_nt(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor,
     reference does it (on the rounded product, rounded again).  `out` may be a row slice of
     a wider buffer (row stride >= N).  The in-place row-parallel linear of
     vllm/model_executor/layers/linear.py:203-228."""
-    if _fast is None or not _fast.gemm_bf16_nt(out, a, b, max_cus, bias):
+    if _fast is None or _tracing() or not _fast.gemm_bf16_nt(out, a, b, max_cus, bias):
         BoundOp(*_prepare_gemm_bf16_nt(out, a, b, max_cus, bias))()
 
 
@@ -756,7 +757,7 @@ def gemm_bf16_nt_partials(outs: Sequence[torch.Tensor], a: Sequence[torch.Tensor
     rank's staging rows (`outs[p]` = `PartialsBuffer.slot(p)[first_row:first_row + M]`).  The
     producer side of the fused op: vllm/model_executor/layers/linear.py:203-228, 1310-1321
     (only rank 0 adds its bias, :1306-1308: pass it as biases[0], None elsewhere)."""
-    if _fast is None or not _fast.gemm_bf16_nt_partials(outs, a, b, max_cus, biases):
+    if _fast is None or _tracing() or not _fast.gemm_bf16_nt_partials(outs, a, b, max_cus, biases):
         BoundOp(*_prepare_gemm_bf16_nt_partials(outs, a, b, max_cus, biases))()
 
 

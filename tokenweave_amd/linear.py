@@ -101,7 +101,7 @@ class RowParallelLinear(nn.Module):
                 is_tokenweave: Optional[bool] = False, gemm_cus: Optional[int] = None
                 ) -> Tuple[torch.Tensor, Optional[Parameter]]:
         if (is_tokenweave and ops._fast is not None and _is_unquantized(self.quant_method)
-                and ops._fast.row_parallel_inplace(self, input_, output_, gemm_cus)):
+                and not ops._tracing() and ops._fast.row_parallel_inplace(self, input_, output_, gemm_cus)):
             if not self.return_bias:
                 return output_
             return output_, (self.bias if self.skip_bias_add else None)
