@@ -1,5 +1,7 @@
 """Host-side mirror of the reference's Python interface for the path: schema
 strings, argument validation, row sharding, split arithmetic.  CPU only."""
+import contextlib
+
 import pytest
 import torch
 
@@ -255,6 +257,37 @@ def test_fuse_only_schedule_calls_in_reference_order():
     ]
     with pytest.raises(AssertionError, match="mlp_fn"):
         tw.tokenweave_with_fuse_only(Layer(), None, hs, res, object(), 1, nearest_multiple_of_world_size=16)
+
+
+@pytest.mark.parametrize("gemm_cus,mlp_gemm_cus,attn_cap,mlp_cap", [
+    (6, 5, 3, 2), (0, None, 0, 0), (6, 0, 3, 0), (0, 5, 0, 2), (6, None, 3, 2)])
+def test_overlap_caps_the_norm_only_beside_a_projection_with_a_budget(monkeypatch, gemm_cus, mlp_gemm_cus, attn_cap,
+                                                                      mlp_cap):
+    """A projection without a budget takes every compute unit; the norm then has the GPU to itself."""
+    caps, budgets = [], []
+
+    class Stream:
+        def record_event(self):
+            pass
+        wait_event = wait_stream = lambda self, other: None
+
+    class Layer:
+        def self_attn(self, positions, hidden_states, gemm_cus=0, **kw):
+            budgets.append(gemm_cus)
+
+    def norm(x, residual=None, **kw):
+        caps.append(kw["MAX_CTAS"])
+    Layer.input_layernorm = Layer.post_attention_layernorm = staticmethod(norm)
+    monkeypatch.setattr(torch.cuda, "stream", contextlib.nullcontext)
+    hs = torch.zeros(16, 8, dtype=torch.bfloat16)
+    tw.tokenweave_overlap(Layer(), torch.arange(16), hs, torch.zeros_like(hs), object(), 1, end_layer=3, rank=0,
+                          world_size=1, current_stream=Stream(), copy_stream=Stream(), next_layer_norm=norm, split_size=8,
+                          actual_tokens=16, num_tokens_padded=16, MAX_CTAS_ATTN=3, MAX_CTAS_MLP=2,
+                          mlp_fn=lambda x, gemm_cus=0: budgets.append(gemm_cus), gemm_cus=gemm_cus,
+                          mlp_gemm_cus=mlp_gemm_cus)
+    assert caps == [attn_cap] * 2 + [mlp_cap] * 2
+    mlp = gemm_cus if mlp_gemm_cus is None else mlp_gemm_cus
+    assert budgets == [gemm_cus] * 2 + [mlp] * 2
 
 
 def test_weave_plan_honours_measured_no_overlap_entries():
