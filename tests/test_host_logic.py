@@ -210,6 +210,14 @@ def test_every_reference_model_has_a_tuned_table(name):
     assert cfg[65536]["overlap"] == 1, "long prefill chunks overlap on MI355X"
 
 
+@pytest.mark.parametrize("name", ["llama_config_4", "llama_config_8", "mixtral_config_8", "qwen2_config_4",
+                                  "qwen2_config_8"])
+def test_every_woven_entry_has_budgets(name):
+    """Without one a projection leaves the norm beside it no compute unit: nothing overlaps."""
+    for n, e in tw.load_config(f"tokenweave_configs/{name}.json").items():
+        assert not e["overlap"] or (e["gemm_cus"] > 0 and e["mlp_gemm_cus"] > 0), n
+
+
 def test_bind_checks_arguments_at_bind_time():
     import tokenweave_amd._custom_ops as ops
     x = torch.zeros(4, 64, dtype=torch.bfloat16)
