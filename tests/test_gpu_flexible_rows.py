@@ -81,3 +81,12 @@ def test_every_output_kind_equals_the_plain_result(dtype, H):
     rb = r.clone()
     ops.fused_add_rms_norm_static_fp8_quant(code, x, rb, w, scale, EPS)
     assert torch.equal(code.view(torch.uint8), quantised(xa)) and torch.equal(ra, rb)
+
+
+@pytest.mark.parametrize("dtype,H", [(torch.bfloat16, 127), (torch.bfloat16, 129), (torch.float16, 127),
+                                     (torch.float16, 129), (torch.float32, 64), (torch.float32, 65)])
+def test_rows_at_the_line_to_the_element_wise_kernel(dtype, H):
+    """Up to 16 vectors of 16 bytes an element a lane, from 17 on a vector a lane."""
+    for shift in (0, 1):
+        test_add_norm(dtype, H, 3, shift)
+    test_every_output_kind_equals_the_plain_result(dtype, H)

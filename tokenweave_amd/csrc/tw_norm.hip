@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
 // ---------------------------------------------------------------------------
 // Element-wise kernel: any hidden size, any alignment, bf16 / fp16 / fp32, any number of
 // partials: the rows that are too long for the registers of a workgroup (more than 32768 16-bit or
-// 16384 fp32 elements).  Two passes over the row; the second re-reads the rounded residual (or the
+// 16384 fp32 elements), and those of at most 16 vectors (launch_flex).  Two passes over the row; the second re-reads the rounded residual (or the
 // input when there is none), like the reference's generic kernel
 // (csrc/layernorm_kernels.cu:122-158).
 // ---------------------------------------------------------------------------
@@ -1404,13 +1404,17 @@ static void launch_elem(const RowNormArgs& a) {
 #undef TW_LAUNCH
 }
 
-// The flexible vector kernel, or false where its registers do not hold a row: at most 4096 vectors
-// (64 chunk sums), two per lane while 1024 lanes hold the row (like the P = 1 kernels above), else four.
+// The flexible vector kernel, or false where the element-wise one is to run: at most 4096 vectors
+// (64 chunk sums: what its registers hold), two per lane while 1024 lanes hold the row (like the P = 1
+// kernels above), else four.  Rows of up to 16 vectors leave three quarters of its one wave without work,
+// where an element a lane keeps it busy: 16384 rows of 33 / 100 bf16 12.4 / 17.2 against 8.2 / 12.0 us
+// (add + norm), of 64 fp32 7.0 against 6.3; from 17 vectors on it is the faster one (129 bf16: 12.9
+// against 16.3, 100 fp32: 8.7 against 10.6).
 template <typename T>
 static bool launch_flex(const RowNormArgs& a) {
   constexpr int NE = 16 / (int)sizeof(T);
   const int64_t V = (a.H + NE - 1) / NE;
-  if (a.np != 1 || V > 64 * kMaxChunks) return false;
+  if (a.np != 1 || V <= 16 || V > 64 * kMaxChunks) return false;
   const int vpt = V <= 2048 ? 2 : 4;
   const int nt = (int)((V + vpt * 64 - 1) / (vpt * 64)) * 64;
   dim3 g(a.grid), b(nt);
