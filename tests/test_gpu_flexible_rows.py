@@ -90,3 +90,12 @@ def test_rows_at_the_line_to_the_element_wise_kernel(dtype, H):
     for shift in (0, 1):
         test_add_norm(dtype, H, 3, shift)
     test_every_output_kind_equals_the_plain_result(dtype, H)
+
+
+@pytest.mark.parametrize("dtype,H", [(d, 264 + tail) for d in (torch.bfloat16, torch.float16) for tail in range(1, 8)]
+                         + [(torch.float32, 132 + tail) for tail in range(1, 4)])
+def test_every_partial_last_vector(dtype, H):
+    """Read with the 16 bytes that end with the row, written in at most three pieces, in place too."""
+    for shift in (0, 1):
+        test_add_norm(dtype, H, 4, shift)
+    test_every_output_kind_equals_the_plain_result(dtype, H)

@@ -839,9 +839,11 @@ __global__ __launch_bounds__(256) void row_norm_mixed_kernel(
 // registers between the reduction and the store, every byte read once and written once.  Vector i
 // of a row begins 16 i bytes behind the row's first element, wherever that lies: global memory
 // accesses need no alignment on this GPU, and of an unaligned wave access only the first and last line
-// are shared with the neighbours.  The elements past the last whole vector are moved one by one,
-// by the lane whose vector they would begin.  The chunk sums are row_sum_chunks', so a row's bits do
-// not depend on the workgroup shape.
+// are shared with the neighbours.  The up to seven 16-bit elements past the last whole vector are read with
+// one access too, the 16 bytes that end with the row, of which the lane drops its neighbour's part, and
+// written with at most three (add + norm of 16384 rows, moved one by one -> so: 150 bf16 21.8 -> 12.5 us, 1006:
+// 33.1 -> 26.7, 8199: 278 -> 220); the up to three of fp32 go one by one (read so, 5123 fp32 elements took
+// 4 % longer).  The chunk sums are row_sum_chunks', so a row's bits do not depend on the workgroup shape.
 //
 // In place of the element-wise kernel (4 bytes per lane, two passes over the row): fp32
 // [4096, 5120] add + norm 78.7 -> 56.5 us (4.3 -> 5.9 TB/s); with the default cache policy 62 us.
@@ -857,9 +859,6 @@ template <> struct FlexVec<float> {
   static __device__ __forceinline__ u32x4_t pack(const float (&f)[4]) {
     return u32x4_t{__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
   }
-  static __device__ __forceinline__ uint32_t get(const float* p) { return __float_as_uint(*p); }
-  static __device__ __forceinline__ void put(u32x4_t& v, int e, uint32_t bits) { v[e] = bits; }
-  static __device__ __forceinline__ uint32_t take(const u32x4_t& v, int e) { return v[e]; }
 };
 template <typename E> struct FlexVec16 {
   static constexpr int NE = 8;
@@ -870,59 +869,100 @@ template <typename E> struct FlexVec16 {
   static __device__ __forceinline__ u32x4_t pack(const float (&f)[8]) {
     return u32x4_t{Pk<E>::pack(f[0], f[1]), Pk<E>::pack(f[2], f[3]), Pk<E>::pack(f[4], f[5]), Pk<E>::pack(f[6], f[7])};
   }
-  static __device__ __forceinline__ uint32_t get(const E* p) { return *reinterpret_cast<const uint16_t*>(p); }
-  static __device__ __forceinline__ void put(u32x4_t& v, int e, uint32_t bits) { v[e >> 1] |= bits << ((e & 1) * 16); }
-  static __device__ __forceinline__ uint32_t take(const u32x4_t& v, int e) {
-    return (v[e >> 1] >> ((e & 1) * 16)) & 0xffffu;
-  }
 };
 template <> struct FlexVec<__bf16> : FlexVec16<__bf16> {};
 template <> struct FlexVec<_Float16> : FlexVec16<_Float16> {};
 
-// The vector of `n` elements (NE: whole) at p; elements past n are zeros.
+// The vector of `n` elements (NE: whole) that begins at element `first` of a row.  Of a partial one, which ends
+// a row of at least NE elements: the 16 bytes that end with it, for flex_trim; the up to three of fp32 one by one.
 template <typename T, bool STREAM>
-__device__ __forceinline__ u32x4_t flex_load(const T* p, int n) {
+__device__ __forceinline__ u32x4_t flex_load(const T* row, int first, int n) {
   typedef FlexVec<T> F;
   u32x4_t v = {0, 0, 0, 0};
-  if (n == F::NE) {
-    if (STREAM) v = __builtin_nontemporal_load(reinterpret_cast<const typename F::Mem*>(p));
-    else v = *reinterpret_cast<const typename F::Mem*>(p);
-  } else if (n > 0) {
+  const T* p = row + first;
+  if (sizeof(T) == 2 ? n > 0 : n == F::NE) {
+    const typename F::Mem* m = reinterpret_cast<const typename F::Mem*>(sizeof(T) == 2 ? p + (n - F::NE) : p);
+    if (STREAM) v = __builtin_nontemporal_load(m);
+    else v = *m;
+  } else if (sizeof(T) == 4 && n > 0) {
 #pragma unroll
     for (int e = 0; e < F::NE - 1; ++e)
-      if (e < n) F::put(v, e, F::get(p + e));
+      if (e < n) v[e] = __float_as_uint((float)p[e]);
   }
   return v;
 }
 
+// ... and the partial one's `tail` elements moved to the front, zeros behind them.  (After all loads: the
+// lane that holds it waits once.)
+template <typename T, int VPT>
+__device__ __forceinline__ void flex_trim(u32x4_t (&v)[VPT], const int (&n)[VPT], int tail) {
+  if (sizeof(T) == 4 || tail == 0) return;
+  const int drop = (8 - tail) * 16;
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    if (n[k] == tail) {
+      const uint64_t lo = (uint64_t)v[k].y << 32 | v[k].x, hi = (uint64_t)v[k].w << 32 | v[k].z;
+      const uint64_t l = drop < 64 ? lo >> drop | hi << (64 - drop) : hi >> (drop - 64), h = drop < 64 ? hi >> drop : 0;
+      v[k] = u32x4_t{(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
+    }
+  }
+}
+
 template <typename T>
-__device__ __forceinline__ void flex_store(T* p, const u32x4_t& v, int n) {
+__device__ __forceinline__ void flex_store(T* row, int first, u32x4_t v, int n) {
   typedef FlexVec<T> F;
+  typedef u32x2_t Mem2 __attribute__((aligned(2)));
+  typedef uint32_t Mem1 __attribute__((aligned(2)));
+  T* p = row + first;
   if (n == F::NE) {
     __builtin_nontemporal_store(v, reinterpret_cast<typename F::Mem*>(p));
+  } else if (sizeof(T) == 2) {  // four, two and one of the elements, whichever there are
+    if (n & 4) {
+      *reinterpret_cast<Mem2*>(p) = u32x2_t{v.x, v.y};
+      p += 4;
+      v.x = v.z;
+      v.y = v.w;
+    }
+    if (n & 2) {
+      *reinterpret_cast<Mem1*>(p) = v.x;
+      p += 2;
+      v.x = v.y;
+    }
+    if (n & 1) *reinterpret_cast<uint16_t*>(p) = (uint16_t)v.x;
   } else if (n > 0) {
 #pragma unroll
-    for (int e = 0; e < F::NE - 1; ++e) {
-      if (e < n) {
-        if constexpr (sizeof(T) == 4) *reinterpret_cast<uint32_t*>(p + e) = F::take(v, e);
-        else *reinterpret_cast<uint16_t*>(p + e) = (uint16_t)F::take(v, e);
-      }
-    }
+    for (int e = 0; e < F::NE - 1; ++e)
+      if (e < n) reinterpret_cast<uint32_t*>(p)[e] = v[e];
   }
 }
 
 // The codes of one vector, four to a word.
 template <int NE>
-__device__ __forceinline__ void flex_store_codes(uint8_t* p, const uint32_t (&c)[NE / 4], int n) {
+__device__ __forceinline__ void flex_store_codes(uint8_t* row, int first, const uint32_t (&c)[NE / 4], int n) {
   typedef u32x2_t Mem2 __attribute__((aligned(1)));
   typedef uint32_t Mem1 __attribute__((aligned(1)));
+  typedef uint16_t MemHalf __attribute__((aligned(1)));
+  uint8_t* p = row + first;
   if (n == NE) {
     if constexpr (NE == 8) __builtin_nontemporal_store(u32x2_t{c[0], c[1]}, reinterpret_cast<Mem2*>(p));
     else __builtin_nontemporal_store(c[0], reinterpret_cast<Mem1*>(p));
+  } else if (NE == 8) {
+    uint32_t w = c[0];
+    if (n & 4) {
+      *reinterpret_cast<Mem1*>(p) = w;
+      p += 4;
+      w = c[NE / 4 - 1];
+    }
+    if (n & 2) {
+      *reinterpret_cast<MemHalf*>(p) = (uint16_t)w;
+      p += 2;
+      w >>= 16;
+    }
+    if (n & 1) *p = (uint8_t)w;
   } else if (n > 0) {
 #pragma unroll
     for (int e = 0; e < NE - 1; ++e)
-      if (e < n) p[e] = (uint8_t)(c[e >> 2] >> ((e & 3) * 8));
+      if (e < n) p[e] = (uint8_t)(c[0] >> (e * 8));
   }
 }
 
@@ -937,6 +977,7 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
   __shared__ float max_slots[2][16];
   const int nwaves = nt >> 6;
   const int nchunks = ((hidden_size + NE - 1) / NE + 63) >> 6;
+  const int tail = hidden_size % NE;
   int first[VPT], n[VPT];  // this lane's vectors: first element, elements inside the row
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
@@ -951,25 +992,28 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
     const size_t base = (size_t)row * hidden_size;
     u32x4_t raw[VPT], res[VPT], wv[VPT];
 #pragma unroll
-    for (int k = 0; k < VPT; ++k) raw[k] = flex_load<T, true>(x + base + first[k], n[k]);
+    for (int k = 0; k < VPT; ++k) raw[k] = flex_load<T, true>(x + base, first[k], n[k]);
     if (HAS_RES) {
 #pragma unroll
-      for (int k = 0; k < VPT; ++k) res[k] = flex_load<T, true>(residual + base + first[k], n[k]);
+      for (int k = 0; k < VPT; ++k) res[k] = flex_load<T, true>(residual + base, first[k], n[k]);
     }
 #pragma unroll
-    for (int k = 0; k < VPT; ++k) wv[k] = flex_load<T, false>(weight + first[k], n[k]);
+    for (int k = 0; k < VPT; ++k) wv[k] = flex_load<T, false>(weight, first[k], n[k]);
+    flex_trim<T>(raw, n, tail);
+    if (HAS_RES) flex_trim<T>(res, n, tail);
+    flex_trim<T>(wv, n, tail);
     float s[VPT][NE], ss[VPT];
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       F::unpack(raw[k], s[k]);
-      if (COPY) flex_store<T>(copy_out + base + first[k], raw[k], n[k]);
+      if (COPY) flex_store<T>(copy_out + base, first[k], raw[k], n[k]);
       if (HAS_RES) {
         float r[NE];
         F::unpack(res[k], r);
 #pragma unroll
         for (int e = 0; e < NE; ++e) s[k][e] += r[e];
         res[k] = F::pack(s[k]);
-        flex_store<T>(residual + base + first[k], res[k], n[k]);
+        flex_store<T>(residual + base, first[k], res[k], n[k]);
       }
       ss[k] = 0.0f;
 #pragma unroll
@@ -1008,7 +1052,7 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
                  : plain        ? quant4_fp8_plain(v[0], v[1], v[2], v[3], scale, sinv)
                                 : quant4_fp8_div(v[0], v[1], v[2], v[3], scale);
         }
-        flex_store_codes<NE>(static_cast<uint8_t*>(y_out) + base + first[k], c, n[k]);
+        flex_store_codes<NE>(static_cast<uint8_t*>(y_out) + base, first[k], c, n[k]);
       }
     } else {
       const float scale_inv = 1.0f / qparam;
@@ -1026,9 +1070,9 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
 #pragma unroll
           for (int g = 0; g < NE / 4; ++g)
             c[g] = quant4_fp8(r[4 * g], r[4 * g + 1], r[4 * g + 2], r[4 * g + 3], scale_inv);
-          flex_store_codes<NE>(static_cast<uint8_t*>(y_out) + base + first[k], c, n[k]);
+          flex_store_codes<NE>(static_cast<uint8_t*>(y_out) + base, first[k], c, n[k]);
         } else {
-          flex_store<T>(static_cast<T*>(y_out) + base + first[k], o, n[k]);
+          flex_store<T>(static_cast<T*>(y_out) + base, first[k], o, n[k]);
         }
       }
     }
