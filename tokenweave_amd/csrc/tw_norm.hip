@@ -1451,9 +1451,9 @@ static void launch_elem(const RowNormArgs& a) {
 // The flexible vector kernel, or false where the element-wise one is to run: at most 4096 vectors
 // (64 chunk sums: what its registers hold), two per lane while 1024 lanes hold the row (like the P = 1
 // kernels above), else four.  Rows of up to 16 vectors leave three quarters of its one wave without work,
-// where an element a lane keeps it busy: 16384 rows of 33 / 100 bf16 12.4 / 17.2 against 8.2 / 12.0 us
-// (add + norm), of 64 fp32 7.0 against 6.3; from 17 vectors on it is the faster one (129 bf16: 12.9
-// against 16.3, 100 fp32: 8.7 against 10.6).
+// where an element a lane keeps it busy.  16384 rows, this kernel against the element-wise one: add + norm of
+// 33 bf16 12.2 / 8.1 us, 100: 12.0 / 12.2 (static fp8: 9.8 / 8.5), 64 fp32 6.7 / 6.2 (dynamic fp8: 8.9 / 6.0); past
+// the line 129 bf16 11.8 / 16.4, 65 fp32 8.6 / 10.7.  (flex_load, too, needs a row of a whole vector.)
 template <typename T>
 static bool launch_flex(const RowNormArgs& a) {
   constexpr int NE = 16 / (int)sizeof(T);
