@@ -73,3 +73,9 @@ def test_inner_dimension_beyond_the_tile_descriptors():
     ops.gemm_bf16_nt(out, a, b)
     torch.cuda.synchronize()
     assert_product(out, a, b, "large K")
+
+
+@pytest.mark.parametrize("M", [65, 300])
+@pytest.mark.parametrize("N", [32, 36])
+def test_few_columns_and_more_than_64_rows(M, N):
+    test_tile_edges(M, N, 328)

@@ -746,11 +746,12 @@ static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N
 }
 
 // The rule looks at M, N and K alone: a product has the same bits under every grid cap and in
-// every batch.
+// every batch.  Up to 32 columns a second column half would be empty LDS and idle MFMAs: 256 rows x 16
+// columns 4.6 -> 4.1 us at K = 128, 13.7 -> 9.5 at 4096.
 static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
                              int max_cus, hipStream_t hs) {
   if (M <= 32) return launch_ksplit<1, 1>(batch, count, M, N, K, ldc, max_cus, hs);
-  if (M <= 64) return launch_ksplit<2, 1>(batch, count, M, N, K, ldc, max_cus, hs);
+  if (M <= 64 || N <= 32) return launch_ksplit<2, 1>(batch, count, M, N, K, ldc, max_cus, hs);
   return launch_ksplit<2, 2>(batch, count, M, N, K, ldc, max_cus, hs);
 }
 
