@@ -79,7 +79,6 @@ def bench_lib():
         L.twb_trace_reduce_add_rms_norm.argtypes = [ctypes.POINTER(vp), ci, vp, vp, vp, i64, i64, ci, f32, vp, vp]
         L.twb_gemm_loop.argtypes = [ci, ci, i64, vp, vp, vp, ci, vp]
         L.twb_lds_read_rate.argtypes = [ci, ci, ci, vp, vp, vp, ci, vp]
-        L.twb_gemm_bf16_nt_tile.argtypes = [vp, vp, vp, i64, i64, i64, i64, ci, ci, vp]
         L.twb_last_error.restype = ctypes.c_char_p
         _BENCH_LIB = L
     return _BENCH_LIB
@@ -106,7 +105,7 @@ def parse_args():
                     help="time the GEMM's k loop assembled from its parts (MFMAs, LDS fragment reads, operand "
                          "slabs global -> LDS) on L2-resident operands, and the LDS read rate, and print them")
     ap.add_argument("--gemm-scaling", action="store_true",
-                    help="time the big GEMM kernel's 320 x 256 tile, one tile per compute unit, on 32 .. 256 "
+                    help="time the tile GEMM's 256 x 256 tile, one tile per compute unit, on 32 .. 256 "
                          "compute units (K = 1024 and 8192) with the shader clock rocm-smi reports meanwhile")
     ap.add_argument("--weave-only", action="store_true",
                     help="time only the GEMM + norm weave of config 5 and print its figures (for profiling)")
@@ -966,8 +965,8 @@ def time_gemm_limits(device):
 
 
 def time_gemm_scaling(device, seconds=2.0):
-    """How the big GEMM kernel's speed per compute unit depends on how many compute units run it.
-    [320 c / 32, K] x [8192, K]^T with the grid capped at c workgroups is c tiles of 320 x 256, one per
+    """How the tile GEMM's speed per compute unit depends on how many compute units run it.
+    [256 c / 32, K] x [8192, K]^T with the grid capped at c workgroups is c tiles of 256 x 256, one per
     compute unit, a single round — the same work per compute unit for every c.  Each point runs for
     `seconds` of back-to-back launches (HIP events, median) while a thread samples `rocm-smi
     --showclocks`; sclk is the median shader clock it reported.  Per compute unit the nominal peak is
@@ -994,12 +993,12 @@ def time_gemm_scaling(device, seconds=2.0):
             return None
         return None
 
-    out = {"definitions": "one 320 x 256 tile per compute unit on `cus` compute units (grid cap), N = 8192; "
+    out = {"definitions": "one 256 x 256 tile per compute unit on `cus` compute units (grid cap), N = 8192; "
                           "tflops_per_cu against a nominal 9.77; sclk_mhz = median of rocm-smi samples during the run"}
     for K in (1024, 8192):
         rows = []
         for cus in (32, 64, 128, 192, 224, 256):
-            M = 320 * cus // 32
+            M = 256 * cus // 32
             g = wl.make_gemm_inputs(M, 8192, K, device)
             outs = [torch.zeros((M, 8192), dtype=torch.bfloat16, device=device) for _ in range(4)]
             calls = [ops.bind_gemm_bf16_nt(o, g.a, g.b, cus) for o in outs]
@@ -1062,15 +1061,12 @@ def time_weave_power(device, seconds=2.5):
     socket power, shader clock and memory-controller activity (medians of `rocm-smi
     --showmetrics` samples during the leg), the stage time (HIP events), and their product,
     the energy one stage takes.  Legs per form (one rank's GEMM / all eight partial sums):
-    GEMM alone, norm alone, both on one stream, the two-stream stage at the GEMM budgets
-    128 and 240 compute units; for one rank's GEMM also the big kernel forced to its 192 x 256
-    and 128 x 256 tiles (164 and 124 registers per lane: a norm workgroup fits beside two of
-    its waves on every SIMD) alone and beside the uncapped norm on the second stream."""
+    GEMM alone, norm alone, both on one stream, the GEMM alone and the two-stream stage at the
+    GEMM budgets 128 and 240 compute units."""
     import threading
     import torch
     from tokenweave_amd import _custom_ops as ops
     from tokenweave_amd import workloads as wl
-    BL = bench_lib()
     cfg = wl.C5_NORM
     inps = [wl.make_norm_inputs(cfg, device, seed_offset=i) for i in range(8)]
     norms = [ops.bind_reduce_add_rms_norm(inp.partials, inp.partials[0], inp.residual, inp.weight, cfg.eps, None)
@@ -1144,14 +1140,6 @@ def time_weave_power(device, seconds=2.5):
         for cap in (128, 240):
             legs[f"gemm/{cap}"] = (lambda c: lambda i: gemms[c][i % R](main_s))(cap)
             legs[f"weave/{cap}"] = two_streams((lambda c: lambda i, s: gemms[c][i % R](s))(cap))
-        if P == 1:
-            for tm in (3, 2):
-                def forced(i, stream, tm=tm):
-                    bench_check(BL.twb_gemm_bf16_nt_tile(stages[i % R][0].data_ptr(), gs[0].a.data_ptr(),
-                                                         gs[0].b.data_ptr(), Ta, N, K, N, tm, 2,
-                                                         stream.cuda_stream))
-                legs[f"gemm_tile{64 * tm}x256"] = (lambda f: lambda i: f(i, main_s))(forced)
-                legs[f"same_units/tile{64 * tm}x256"] = two_streams(forced)
         rows = {}
         for name, fn in legs.items():
             rows[name] = run_leg(fn)
