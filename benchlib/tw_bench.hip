@@ -537,14 +537,14 @@ TWB_API int twb_reduce_add_rms_norm_split_spread(const void* const* partials, in
   return tw::finish_launch(what);
 }
 
-// tw_gemm_bf16_nt with the tile kernel's shape forced to (64 tm) x (128 tn), without a
-// compute-unit budget, instead of the one the library's cost model picks.  Same operand rules as
-// the library call; the shape must fit the tile kernel.
-TWB_API int twb_gemm_bf16_nt_tile(void* out, const void* a, const void* b, int64_t M, int64_t N, int64_t K,
-                                  int64_t ldc, int tm, int tn, void* stream) {
+// tw_gemm_bf16_nt_bias with the tile kernel's shape forced to (32 tm) x (32 tn), one of the shapes
+// of tw::kTiles, instead of the one the library's cost model picks; any M, N and K that the library
+// call takes and the tile kernel's offsets hold.
+TWB_API int twb_gemm_bf16_nt_tile(void* out, const void* a, const void* b, const void* bias, int64_t M, int64_t N,
+                                  int64_t K, int64_t ldc, int tm, int tn, int max_cus, void* stream) {
   const char* what = "gemm_bf16_nt_tile";
   if (int rc = tw::check_gemm_shape(what, M, N, K, ldc)) return rc;
-  if (int rc = tw::check_gemm_pointers(what, out, a, b, nullptr)) return rc;
+  if (int rc = tw::check_gemm_pointers(what, out, a, b, bias)) return rc;
   if (M == 0) return TW_OK;
   if (K > tw::TILE_MAX_K || ldc > tw::TILE_MAX_LDC)
     return tw::set_error(TW_ERR_INVALID_ARGUMENT, "%s: shape outside the tile kernel", what);
@@ -552,12 +552,17 @@ TWB_API int twb_gemm_bf16_nt_tile(void* out, const void* a, const void* b, int64
   batch.out[0] = static_cast<uint16_t*>(out);
   batch.a[0] = static_cast<const uint16_t*>(a);
   batch.b[0] = static_cast<const uint16_t*>(b);
-  hipStream_t hs = static_cast<hipStream_t>(stream);
-  bool known = false;
-  for (const tw::TileChoice& t : tw::kTiles) known = known || (t.tm == 2 * tm && t.tn == 4 * tn);
-  if (!known) return tw::set_error(TW_ERR_INVALID_ARGUMENT, "%s: no %d x %d tile", what, 64 * tm, 128 * tn);
-  const int rc = tw::launch_tile_shape(2 * tm, 4 * tn, batch, 1, M, N, K, ldc, 0, hs);
+  batch.bias[0] = static_cast<const uint16_t*>(bias);
+  const int rc = tw::launch_tile_shape(tm, tn, batch, 1, M, N, K, ldc, max_cus, static_cast<hipStream_t>(stream));
   return rc ? rc : tw::finish_launch(what);
+}
+
+// Shape `index` of tw::kTiles in units of 32 rows and 32 columns; 0 past the last one.
+TWB_API int twb_gemm_tile_shape(int index, int* tm, int* tn) {
+  if (index < 0 || index >= (int)(sizeof(tw::kTiles) / sizeof(tw::kTiles[0]))) return 0;
+  *tm = tw::kTiles[index].tm;
+  *tn = tw::kTiles[index].tn;
+  return 1;
 }
 
 static int bench_lds_limit(const void* fn, int bytes) {

@@ -77,8 +77,8 @@ def test_gemm_output_with_wide_row_stride():
     (300, 384, 128, 388, 0),    # row stride % 8 != 0: 8-byte stores
     (300, 384, 128, 384, 4),    # out 8-byte but not 16-byte aligned: 8-byte stores
     (645, 520, 192, 520, 0),    # ragged tile edges in both directions, 16-byte stores
-    (2048, 10240, 128, 10240, 0),   # 8 x 27 tiles of 256 x 384 fit one round of 256 compute units
-    (2000, 10004, 128, 10004, 0),   # the same tile with ragged edges and 8-byte stores
+    (2048, 10240, 128, 10240, 0),   # more tiles than compute units, whole ones, 16-byte stores
+    (2000, 10004, 128, 10004, 0),   # ... with ragged edges and 8-byte stores
     (2040, 10000, 192, 10008, 0),   # ... and with 16-byte stores into a wider buffer
 ])
 def test_gemm_large_tile_kernel_store_paths(M, N, K, ldc, shift):
@@ -95,10 +95,10 @@ def test_gemm_large_tile_kernel_store_paths(M, N, K, ldc, shift):
 
 
 @pytest.mark.parametrize("P,M,N,K,first_row,rows", [
-    (8, 300, 512, 128, 0, 300),       # small: every tile kind of the big kernel's edges
+    (8, 300, 512, 128, 0, 300),       # small: partial tiles of the tile kernel in M
     (8, 333, 8192, 1024, 200, 600),   # ragged M, the split starts at a non-zero staging row
     (3, 645, 520, 192, 7, 700),       # odd P, ragged tiles in both directions
-    (2, 100, 128, 64, 5, 128),        # too small for the big kernel: one launch per product
+    (2, 100, 128, 64, 5, 128),        # at most 128 rows: the K-split kernel
 ])
 def test_partials_producer_writes_every_rank_slot(P, M, N, K, first_row, rows):
     """tw_gemm_bf16_nt_partials: the P partial sums of a token split land in rows
@@ -258,13 +258,13 @@ def reference_linear_inplace(a, b, bias):
 
 
 @pytest.mark.parametrize("M,N,K,ldc,shift", [
-    (100, 128, 64, 128, 0),          # fallback kernel
-    (129, 256, 72, 256, 0),          # fallback kernel, K % 64 != 0
-    (300, 384, 128, 384, 0),         # big kernel, 16-byte stores
-    (300, 388, 128, 388, 0),         # big kernel, 8-byte stores (N % 8 != 0)
-    (300, 384, 128, 384, 4),         # big kernel, out not 16-byte aligned
+    (100, 128, 64, 128, 0),          # K-split kernel
+    (129, 256, 72, 256, 0),          # tile kernel, K % 64 != 0
+    (300, 384, 128, 384, 0),         # tile kernel, 16-byte stores
+    (300, 388, 128, 388, 0),         # tile kernel, 8-byte stores (N % 8 != 0)
+    (300, 384, 128, 384, 4),         # tile kernel, out not 16-byte aligned
     (2458, 8192, 1024, 8192, 0),     # config 5's shape
-    (2048, 10240, 128, 10240, 0),    # 256 x 384 tiles
+    (2048, 10240, 128, 10240, 0),    # 320 tiles of 256 x 256
 ])
 def test_gemm_bias_matches_the_reference_two_step_arithmetic(M, N, K, ldc, shift):
     """out = bf16(bf16(a b^T) + bias): against fp32 CPU arithmetic within the path's
