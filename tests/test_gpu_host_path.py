@@ -131,6 +131,20 @@ def test_hooks_autograd_and_dispatch_modes_take_the_ordinary_route(counted):
     assert counted["rms_norm"] == 1
 
 
+def test_a_tensor_that_wants_its_gradient_takes_the_ordinary_route(counted):
+    x, r, layer = tensors()
+    w = layer.weight.data
+    want, got = torch.empty_like(x), torch.empty_like(x)
+    ops.rms_norm(want, x, w, 1e-6)
+    assert counted.pop("rms_norm") == 1
+    leaf = x.clone().requires_grad_()
+    ops.rms_norm(got, leaf, w, 1e-6)
+    assert counted == {} and torch.equal(got.detach(), want)
+    with torch.no_grad():
+        ops.rms_norm(torch.empty_like(x), leaf, w, 1e-6)
+    assert counted == {"rms_norm": 1}
+
+
 def test_a_lazily_negated_tensor_is_read_with_its_sign(counted):
     """`torch._neg_view` only marks a tensor as negated; the dispatcher resolves the mark before an op
     sees the storage, so such a tensor takes that route, whichever argument it is."""
