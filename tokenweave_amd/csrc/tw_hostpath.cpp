@@ -33,7 +33,7 @@ using at::Tensor;
 
 // Interned attribute names and torch.nn's global hook tables, looked up once.
 PyObject *s_parameters, *s_weight, *s_bias, *s_epsilon, *s_var_override, *s_forward, *s_compiled, *s_multicast,
-    *s_signal_pads, *s_hooks[4], *s_tp_rank, *s_skip_bias, *s_input_parallel, *s_residual, *s_out;
+    *s_signal_pads, *s_call, *s_hooks[4], *s_tp_rank, *s_skip_bias, *s_input_parallel, *s_residual, *s_out;
 PyObject* g_global_hooks[4];
 
 bool direct_allowed() {
@@ -279,6 +279,31 @@ bool plain_module(PyObject* dict) {
   return (!compiled || compiled == Py_None) && !PyDict_GetItem(dict, s_forward);
 }
 
+// The norm's class and torch.nn.Module with the functions that a call of a norm runs, as the package
+// defined them.
+PyTypeObject *g_norm, *g_module_class;
+PyObject *g_norm_forward, *g_norm_call, *g_module_call;
+
+// (RMSNorm, torch.nn.Module), once when the class is defined.
+PyObject* remember_rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 2 || !PyType_Check(a[0]) || !PyType_Check(a[1])) Py_RETURN_FALSE;
+  for (Py_ssize_t i = 0; i < n; ++i) Py_INCREF(a[i]);
+  g_norm = (PyTypeObject*)a[0];
+  g_module_class = (PyTypeObject*)a[1];
+  Py_XINCREF(g_norm_forward = _PyType_Lookup(g_norm, s_forward));
+  Py_XINCREF(g_norm_call = _PyType_Lookup(g_norm, s_call));
+  Py_XINCREF(g_module_call = _PyType_Lookup(g_module_class, s_call));
+  return yes_no(g_norm_forward && g_norm_call && g_module_call);
+}
+
+// Whether calling this object runs the package's RMSNorm: neither a subclass nor a class whose forward
+// or __call__ somebody has replaced (`plain_module` looks at the instance).  Looked up by type in 35 ns
+// where the reads in Python took 170.
+PyObject* runs_rms_norm(PyObject*, PyObject* o) {
+  return yes_no(g_norm && Py_TYPE(o) == g_norm && _PyType_Lookup(g_norm, s_forward) == g_norm_forward &&
+                _PyType_Lookup(g_norm, s_call) == g_norm_call && _PyType_Lookup(g_module_class, s_call) == g_module_call);
+}
+
 // A parameter, or what the class keeps as a plain tensor attribute in its place.
 const Tensor* module_tensor(PyObject* dict, PyObject* name) {
   PyObject* params = PyDict_GetItem(dict, s_parameters);
@@ -444,6 +469,8 @@ PyMethodDef g_methods[] = {
     TW_FAST_RESULT("rms_norm_call", rms_norm_call),
     TW_FAST("fused_allreduce_layernorm", fused_allreduce_layernorm),
     TW_FAST("row_parallel_inplace", row_parallel_inplace),
+    TW_FAST("remember_rms_norm", remember_rms_norm),
+    {"runs_rms_norm", runs_rms_norm, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_hostpath", "direct calls of the ops (see tw_hostpath.cpp)", -1, g_methods};
@@ -451,7 +478,7 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_hostpath", "direct calls of the
 bool init_names() {
   const struct { PyObject** at; const char* name; } names[] = {
       {&s_parameters, "_parameters"}, {&s_weight, "weight"}, {&s_bias, "bias"}, {&s_epsilon, "variance_epsilon"},
-      {&s_var_override, "variance_size_override"}, {&s_forward, "forward"}, {&s_compiled, "_compiled_call_impl"},
+      {&s_var_override, "variance_size_override"}, {&s_forward, "forward"}, {&s_call, "__call__"}, {&s_compiled, "_compiled_call_impl"},
       {&s_multicast, "multicast_ptr"}, {&s_signal_pads, "signal_pad_ptrs_dev"}, {&s_hooks[0], "_forward_hooks"},
       {&s_hooks[1], "_forward_pre_hooks"}, {&s_hooks[2], "_backward_hooks"}, {&s_hooks[3], "_backward_pre_hooks"}, {&s_tp_rank, "tp_rank"},
       {&s_skip_bias, "skip_bias_add"}, {&s_input_parallel, "input_is_parallel"},
