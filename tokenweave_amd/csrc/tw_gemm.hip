@@ -415,8 +415,8 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
 // (112 against 107 us, 8192 x 8192 x 1024).
 //
 // Measured against the 8-wave kernel this replaces, same box: 8192^3 874 -> 714 us (1 253 -> 1 539
-// TFLOP/s; matrix cores busy 65 -> 84 % of the cycles while the clock, under the board's power limit,
-// falls from 1.91 to 1.84 GHz), 8192 x 8192 x 3584 406 -> 325, 8192 x 8192 x 1024 127 -> 107,
+// TFLOP/s; matrix cores now busy 86 % of the cycles in which a unit has work, at a clock of 1.82 GHz and
+// less under the board's power limit), 8192 x 8192 x 3584 406 -> 325, 8192 x 8192 x 1024 127 -> 107,
 // 1024 x 8192 x 3712 59 -> 48, 512 x 8192 x 3584 49 -> 28 us.
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
