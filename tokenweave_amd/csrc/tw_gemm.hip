@@ -790,6 +790,10 @@ static int launch_tile(const GemmBatch& batch, int count, int64_t M, int64_t N, 
 // (M = 2458: 512 tiles) and the 192-wide ones for N = 6144, whose 24 columns of 256 leave a quarter
 // of the units idle; the small ones for M <= 512 at N = 8192 (64 x 128, 96 x 128, 128 x 128: 256
 // tiles for 256, 384 and 512 rows).
+// One column of costs serves every K: of the twelve shapes timed one by one, the picked one is the
+// fastest at 114 of 120 points (15 row counts from 129 to 4096; 8192 columns with K = 1024, 2048, 3584,
+// 3696, 7168, 7392 and 6144 columns with K = 768, 2048), 0.1 % from it on average and 5 % at worst
+// (640 rows, K = 7392: 82 us, 96 x 256 tiles 78).
 struct TileChoice { int tm, tn; double cost; };
 #define TW_TILES(X)                                                                                            \
   X(8, 8, 1.0) X(6, 8, 0.79) X(8, 6, 0.77) X(5, 8, 0.69) X(6, 6, 0.65) X(4, 8, 0.58) X(3, 8, 0.48) X(4, 6, 0.46) \
