@@ -99,3 +99,50 @@ def test_every_partial_last_vector(dtype, H):
     for shift in (0, 1):
         test_add_norm(dtype, H, 4, shift)
     test_every_output_kind_equals_the_plain_result(dtype, H)
+
+
+def element_order_inv_rms(v):
+    """1 / rms of the rows of `v` (fp32 on the CPU, values of bf16 tensors) with the element-wise kernel's order of
+    additions: lane t adds the squares t, t + lanes, ... by fused multiply-adds (the squares are exact in fp32,
+    the sums in fp64: one rounding each), 64 lanes as a tree in groups of 16, the rest one after the other."""
+    T, H = v.shape
+    lanes = (H + 63) // 64 * 64 if H < 1024 else 1024
+    squares = torch.zeros(T, (H + lanes - 1) // lanes * lanes, dtype=torch.float64)
+    squares[:, :H] = v.double().square()
+    acc = torch.zeros(T, lanes)
+    for step in squares.view(T, -1, lanes).unbind(1):
+        acc = (acc.double() + step).float()
+    acc = acc.view(T, -1, 4, 16)
+    while acc.shape[-1] > 1:
+        acc = acc[..., 0::2] + acc[..., 1::2]
+    acc = acc[..., 0]
+    waves = ((acc[:, :, 0] + acc[:, :, 1]) + acc[:, :, 2]) + acc[:, :, 3]
+    total = waves[:, 0]
+    for w in range(1, waves.shape[1]):
+        total = total + waves[:, w]
+    return 1.0 / torch.sqrt(total / torch.full_like(total, H) + torch.full_like(total, EPS))
+
+
+@pytest.mark.parametrize("dtype,H", [(torch.bfloat16, h) for h in (129, 777, 1000, 1025, 6663, 8199, 15865, 15873, 16383,
+                                                                   16385, 32767)]
+                         + [(torch.float32, h) for h in (65, 1490, 5120, 8193, 15873, 16384)])
+def test_sum_is_the_element_wise_kernels(dtype, H):
+    """The same norm to the last bit as rows that take the element-wise kernel, and so the same codes."""
+    T = 100 if H > 8192 else 300
+    print(f"[case] flex order {dtype} T={T} H={H}", flush=True)
+    g = torch.Generator().manual_seed(H)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    w = torch.randn(H, generator=g).to(torch.bfloat16)
+    v = x.float()
+    want = (v * element_order_inv_rms(v)[:, None] * w.float()).to(dtype)
+    xd = torch.empty(T * H + 1, device=DEV, dtype=dtype)[1:].view(T, H)  # unaligned: never the aligned kernels
+    xd.copy_(x)
+    wd, y = w.to(DEV, dtype), torch.empty(T, H, device=DEV, dtype=dtype)
+    ops.rms_norm(y, xd, wd, EPS)
+    assert torch.equal(y.cpu(), want)
+    if dtype == torch.bfloat16:
+        scale = torch.tensor([0.03])
+        code = torch.empty(T, H, device=DEV, dtype=torch.float8_e4m3fn)
+        ops.rms_norm_static_fp8_quant(code, xd, wd, scale.to(DEV), EPS)
+        q = (want.float() * (1.0 / scale)).clamp(-448, 448).to(torch.float8_e4m3fn)
+        assert torch.equal(code.cpu().view(torch.uint8), q.view(torch.uint8))

@@ -843,7 +843,13 @@ __global__ __launch_bounds__(256) void row_norm_mixed_kernel(
 // one access too, the 16 bytes that end with the row, of which the lane drops its neighbour's part, and
 // written with at most three (add + norm of 16384 rows, moved one by one -> so: 150 bf16 21.8 -> 12.5 us, 1006:
 // 33.1 -> 26.7, 8199: 278 -> 220); the up to three of fp32 go one by one (read so, 5123 fp32 elements took
-// 4 % longer).  The chunk sums are row_sum_chunks', so a row's bits do not depend on the workgroup shape.
+// 4 % longer).
+//
+// The sum of squares is the element-wise kernel's, addition by addition (elem_order_sum): the two share the
+// rows of an op by size and by number of partials, and a last-bit difference of the norm moves about one fp8 or
+// int8 code in a million.  It goes through LDS.  Against sums of whole vectors in registers, us: 2000 x 6663 bf16 to
+// dynamic fp8 32.7 -> 24.7 and static 27.7 -> 23.3, add + norm of 16384 x 8199 bf16 280 -> 246 and 4096 x 5120 fp32
+// 55.5 -> 56.1, but norm of 4096 x 5120 fp32 29.7 -> 33.4 and 100 x 3868 to dynamic fp8 5.8 -> 6.1.
 //
 // In place of the element-wise kernel (4 bytes per lane, two passes over the row): fp32
 // [4096, 5120] add + norm 78.7 -> 56.5 us (4.3 -> 5.9 TB/s); with the default cache policy 62 us.
@@ -966,6 +972,28 @@ __device__ __forceinline__ void flex_store_codes(uint8_t* row, int first, const 
   }
 }
 
+// Lanes of the element-wise kernel for a row.
+__host__ __device__ constexpr int elem_lanes(int hidden) { return hidden < 1024 ? (hidden + 63) / 64 * 64 : 1024; }
+
+// Sum of squares of the `hidden` values in `row` (LDS) as the element-wise kernel adds them: its lane t takes
+// the elements t, t + lanes, ... in order, then block_sum.  The workgroup's waves take those of its waves in turn.
+// The caller writes `row` before, and again only behind the last barrier in here; `slots` holds 16.
+__device__ __forceinline__ float elem_order_sum(const float* row, int hidden, float* slots, int nwaves) {
+  const int lanes = elem_lanes(hidden);
+  const int lane = threadIdx.x & 63;
+  __syncthreads();
+  for (int w = threadIdx.x >> 6; w < lanes >> 6; w += nwaves) {
+    float ss = 0.0f;
+    for (int j = w * 64 + lane; j < hidden; j += lanes) ss += row[j] * row[j];
+    ss = wave_sum(ss);
+    if (lane == 0) slots[w] = ss;
+  }
+  __syncthreads();
+  float total = slots[0];
+  for (int i = 1; i < lanes >> 6; ++i) total += slots[i];
+  return total;
+}
+
 template <typename T, int VPT, bool HAS_RES, bool COPY, int Q>
 __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
     const T* x, void* y_out, T* residual, T* copy_out, const T* __restrict__ weight,
@@ -973,10 +1001,10 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
     int nt, int grid) {
   typedef FlexVec<T> F;
   constexpr int NE = F::NE;
-  __shared__ float slots[2][kMaxChunks];
+  extern __shared__ __attribute__((aligned(16))) float lds_row[];  // the row's whole and partial vectors
+  __shared__ float slots[2][16];
   __shared__ float max_slots[2][16];
   const int nwaves = nt >> 6;
-  const int nchunks = ((hidden_size + NE - 1) / NE + 63) >> 6;
   const int tail = hidden_size % NE;
   int first[VPT], n[VPT];  // this lane's vectors: first element, elements inside the row
 #pragma unroll
@@ -1002,7 +1030,7 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
     flex_trim<T>(raw, n, tail);
     if (HAS_RES) flex_trim<T>(res, n, tail);
     flex_trim<T>(wv, n, tail);
-    float s[VPT][NE], ss[VPT];
+    float s[VPT][NE];
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       F::unpack(raw[k], s[k]);
@@ -1015,11 +1043,12 @@ __global__ __launch_bounds__(1024) void row_norm_flex_kernel(
         res[k] = F::pack(s[k]);
         flex_store<T>(residual + base, first[k], res[k], n[k]);
       }
-      ss[k] = 0.0f;
+      if (n[k] > 0) {
 #pragma unroll
-      for (int e = 0; e < NE; ++e) ss[k] += s[k][e] * s[k][e];
+        for (int e = 0; e < NE; ++e) lds_row[first[k] + e] = s[k][e];
+      }
     }
-    const float inv = inv_rms(row_sum_chunks<VPT>(ss, slots[phase], nwaves, nchunks), (float)hidden_size, eps);
+    const float inv = inv_rms(elem_order_sum(lds_row, hidden_size, slots[phase], nwaves), (float)hidden_size, eps);
     if (Q == kQDynFp8 || Q == kQDynInt8) {
       float amax = 0.0f;
 #pragma unroll
@@ -1425,7 +1454,7 @@ static int launch_vec_mode(const RowNormArgs& a) {
 
 template <typename T>
 static void launch_elem(const RowNormArgs& a) {
-  int nt = a.H < 1024 ? (int)((a.H + 63) / 64) * 64 : 1024;
+  int nt = elem_lanes((int)a.H);
   dim3 g(a.grid), b(nt);
 #define TW_LAUNCH(HAS_RES, COPY, FP8)                                                            \
   launch_kernel(row_norm_elem_kernel<T, HAS_RES, COPY, FP8>, g, b, 0, a.stream, a.parts,         \
@@ -1448,6 +1477,23 @@ static void launch_elem(const RowNormArgs& a) {
 #undef TW_LAUNCH
 }
 
+// More than 64 KiB of dynamic LDS must be allowed once per kernel and device.
+template <typename T, int VPT, bool HAS_RES, bool COPY, int Q>
+static bool flex_lds_allowed(size_t bytes) {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<bool> allowed[kMaxDevices];
+  if (bytes + 1024 <= 64 * 1024) return true;  // (1024: more than the kernel's static part)
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
+  if (!allowed[dev].load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(row_norm_flex_kernel<T, VPT, HAS_RES, COPY, Q>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 64 * kMaxChunks * 32) != hipSuccess)
+      return false;
+    allowed[dev].store(true, std::memory_order_release);
+  }
+  return true;
+}
+
 // The flexible vector kernel, or false where the element-wise one is to run: at most 4096 vectors
 // (64 chunk sums: what its registers hold), two per lane while 1024 lanes hold the row (like the P = 1
 // kernels above), else four.  Rows of up to 16 vectors leave three quarters of its one wave without work,
@@ -1461,12 +1507,16 @@ static bool launch_flex(const RowNormArgs& a) {
   if (a.np != 1 || V <= 16 || V > 64 * kMaxChunks) return false;
   const int vpt = V <= 2048 ? 2 : 4;
   const int nt = (int)((V + vpt * 64 - 1) / (vpt * 64)) * 64;
+  const size_t lds = (size_t)V * NE * sizeof(float);
   dim3 g(a.grid), b(nt);
-#define TW_LAUNCH_FLEX(VPT, HAS_RES, COPY, Q)                                                              \
-  launch_kernel(row_norm_flex_kernel<T, VPT, HAS_RES, COPY, Q>, g, b, 0, a.stream,                         \
-                static_cast<const T*>(a.parts.p[0]), a.y, static_cast<T*>(a.residual),                     \
-                static_cast<T*>(a.copy_out), static_cast<const T*>(a.weight), a.quant_scale, a.row_scales, \
-                a.eps, (int)a.T, (int)a.H, nt, a.grid)
+#define TW_LAUNCH_FLEX(VPT, HAS_RES, COPY, Q)                                                                \
+  do {                                                                                                       \
+    if (!flex_lds_allowed<T, VPT, HAS_RES, COPY, Q>(lds)) return false;                                      \
+    launch_kernel(row_norm_flex_kernel<T, VPT, HAS_RES, COPY, Q>, g, b, lds, a.stream,                       \
+                  static_cast<const T*>(a.parts.p[0]), a.y, static_cast<T*>(a.residual),                     \
+                  static_cast<T*>(a.copy_out), static_cast<const T*>(a.weight), a.quant_scale, a.row_scales, \
+                  a.eps, (int)a.T, (int)a.H, nt, a.grid);                                                    \
+  } while (0)
 #define TW_LAUNCH_FLEX_Q(HAS_RES, Q)                                                                       \
   do {                                                                                                     \
     if (vpt == 2) TW_LAUNCH_FLEX(2, HAS_RES, false, Q);                                                    \
