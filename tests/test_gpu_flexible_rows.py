@@ -101,8 +101,8 @@ def test_every_partial_last_vector(dtype, H):
     test_every_output_kind_equals_the_plain_result(dtype, H)
 
 
-def element_order_inv_rms(v):
-    """1 / rms of the rows of `v` (fp32 on the CPU, values of bf16 tensors) with the element-wise kernel's order of
+def element_order_sum(v):
+    """Sums of the squares of the rows of `v` (fp32 on the CPU, values of bf16 tensors) with the element-wise kernel's order of
     additions: lane t adds the squares t, t + lanes, ... by fused multiply-adds (the squares are exact in fp32,
     the sums in fp64: one rounding each), 64 lanes as a tree in groups of 16, the rest one after the other."""
     T, H = v.shape
@@ -120,29 +120,45 @@ def element_order_inv_rms(v):
     total = waves[:, 0]
     for w in range(1, waves.shape[1]):
         total = total + waves[:, w]
-    return 1.0 / torch.sqrt(total / torch.full_like(total, H) + torch.full_like(total, EPS))
+    return total
 
 
-@pytest.mark.parametrize("dtype,H", [(torch.bfloat16, h) for h in (129, 777, 1000, 1025, 6663, 8199, 15865, 15873, 16383,
-                                                                   16385, 32767)]
-                         + [(torch.float32, h) for h in (65, 1490, 5120, 8193, 15873, 16384)])
-def test_sum_is_the_element_wise_kernels(dtype, H):
-    """The same norm to the last bit as rows that take the element-wise kernel, and so the same codes."""
+def norm_factors(rows, H):
+    """The kernel's 1 / rms of fp32 rows, read off element 2: 2^-60, whose square vanishes in any sum here."""
+    x = torch.zeros(len(rows) * H + 1, device=DEV)[1:].view(len(rows), H)  # unaligned: never the aligned kernels
+    x[:, :rows.shape[1]] = rows.to(DEV)
+    x[:, 2] = 2.0 ** -60
+    y = torch.empty(len(rows), H, device=DEV)
+    ops.rms_norm(y, x, torch.ones(H, device=DEV), EPS)
+    return (y[:, 2] * 2.0 ** 60).cpu()
+
+
+@pytest.mark.parametrize("H", [65, 129, 777, 1000, 1025, 1490, 5120, 6663, 8193, 8199, 15873, 16384, 16385, 32767])
+def test_sum_is_the_element_wise_kernels(H):
+    """The same sum to the last bit as rows that take the element-wise kernel, and so the same norm and codes: a row
+    has the factor of a row of two elements whose squares add up to the emulated sum.  (fp32 rows of more than
+    16384 elements are the element-wise kernel's own; bf16 rows must have the factors of the fp32 ones.)"""
     T = 100 if H > 8192 else 300
-    print(f"[case] flex order {dtype} T={T} H={H}", flush=True)
+    print(f"[case] flex order T={T} H={H}", flush=True)
     g = torch.Generator().manual_seed(H)
     x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    x[:, 2] = 2.0 ** -60
     w = torch.randn(H, generator=g).to(torch.bfloat16)
-    v = x.float()
-    want = (v * element_order_inv_rms(v)[:, None] * w.float()).to(dtype)
-    xd = torch.empty(T * H + 1, device=DEV, dtype=dtype)[1:].view(T, H)  # unaligned: never the aligned kernels
+    total = element_order_sum(x.float())
+    a = total.sqrt() * (1 - 2.0 ** -20)
+    b = (total - a * a).sqrt()
+    assert torch.equal(a * a + b * b, total)
+    inv = norm_factors(x.float(), H)
+    assert torch.equal(inv, norm_factors(torch.stack([a, b], 1), H))
+    if H < 129:
+        return
+    want = (x.float() * inv[:, None] * w.float()).to(torch.bfloat16)
+    xd = torch.empty(T * H + 1, device=DEV, dtype=torch.bfloat16)[1:].view(T, H)
     xd.copy_(x)
-    wd, y = w.to(DEV, dtype), torch.empty(T, H, device=DEV, dtype=dtype)
-    ops.rms_norm(y, xd, wd, EPS)
+    y, code = torch.empty_like(xd), torch.empty(T, H, device=DEV, dtype=torch.float8_e4m3fn)
+    ops.rms_norm(y, xd, w.to(DEV), EPS)
     assert torch.equal(y.cpu(), want)
-    if dtype == torch.bfloat16:
-        scale = torch.tensor([0.03])
-        code = torch.empty(T, H, device=DEV, dtype=torch.float8_e4m3fn)
-        ops.rms_norm_static_fp8_quant(code, xd, wd, scale.to(DEV), EPS)
-        q = (want.float() * (1.0 / scale)).clamp(-448, 448).to(torch.float8_e4m3fn)
-        assert torch.equal(code.cpu().view(torch.uint8), q.view(torch.uint8))
+    scale = torch.tensor([0.03])
+    ops.rms_norm_static_fp8_quant(code, xd, w.to(DEV), scale.to(DEV), EPS)
+    q = (want.float() * (1.0 / scale)).clamp(-448, 448).to(torch.float8_e4m3fn)
+    assert torch.equal(code.cpu().view(torch.uint8), q.view(torch.uint8))
