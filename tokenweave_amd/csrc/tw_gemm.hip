@@ -204,15 +204,21 @@ struct GemmBatch {
 // dimension: wave w takes the 64-wide k-slabs w, w + 4, ... .  Each wave brings its slabs of
 // both operands from global memory straight into LDS of its own, STAGES slabs deep, and
 // reads its fragments back from there: no barrier in the k loop, a wave only waits for its own
-// loads.  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
+// loads.  (Three stages up to 32 rows, 1-2 % ahead of two; four are no better: what a unit has under way is
+// bounded by its L1, not by LDS.)  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
 // Every load covers whole 128-byte lines of eight rows.  The sum of an output element does not
 // depend on the tile it lies in (nor on MT, NT, the grid or the number of products).
 //
 // The launcher makes the tiles just wide enough for one (or a whole number of) workgroups per
 // compute unit: 32 columns at N = 8192, 24 at N = 6144.  Measured on 256 units, operands
-// rotated through 2 GB / through three sets: [32, 3584] x [8192, 3584]^T 13.9 / 10.6 us
-// (59 MB: 4.3 / 5.6 TB/s) against 65 / 47 us with 64 workgroups of 128 x 128; K = 1024: 6.0 / 5.0 us
+// rotated through 0.5 GB / through three sets: [32, 3584] x [8192, 3584]^T 14.1 / 10.7 us
+// (59 MB: 4.2 / 5.6 TB/s) against 65 / 47 us with 64 workgroups of 128 x 128; K = 1024: 5.2 us
 // against 16 us; [128, 3584]: 21 / 15 us against 69 / 50 us.
+//
+// What is short is also bound by the way to the first load: with rows past 16 or 8 not fetched, the partial
+// last slab in an instantiation of its own, no division for one product of one row tile and every pointer
+// fetched at the start, three sets: [8, 1024] 5.7 -> 4.8 us, [32, 1024] 5.8 -> 5.2, [32, 3584] 11.2 -> 10.7,
+// [64, 1024] 6.6 -> 6.3, [96, 768] x [6144, 768]^T 6.0 -> 5.7.
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -228,39 +234,42 @@ constexpr int ks_lds_bytes(int mt, int nt, int stages) {
   return slabs > sums ? slabs : sums;
 }
 
-// One operand's share of a slab, 8 rows per wave instruction; `tail`: the last slab of an inner
-// dimension that is no multiple of 64, whose chunks past K must arrive as zeros (`even` / `odd`
+// One operand's share of a slab, 8 rows per wave instruction; `last`: the last slab of an inner
+// dimension that is no multiple of 64 (TAIL), whose chunks past K must arrive as zeros (`even` / `odd`
 // say whether this lane's chunk of an even / odd 8-row block is inside).
-template <int L>
-__device__ __forceinline__ void ks_issue(__amdgpu_buffer_rsrc_t d, const uint32_t (&v)[L], uint8_t* s, uint32_t koff,
-                                         bool tail, bool even, bool odd) {
-  if (tail) {
+template <int L, int AUX, bool TAIL, int LV>
+__device__ __forceinline__ void ks_issue(__amdgpu_buffer_rsrc_t d, const uint32_t (&v)[LV], uint8_t* s, uint32_t koff,
+                                         bool last, bool even, bool odd) {
+  if (TAIL && last) {
 #pragma unroll
     for (int j = 0; j < L; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_void_t*)(s + j * 1024), 16,
-                                               ((j & 1) ? odd : even) ? v[j] : KS_OUT_OF_RANGE, koff, 0, 0);
+                                               ((j & 1) ? odd : even) ? v[j] : KS_OUT_OF_RANGE, koff, 0, AUX);
   } else {
 #pragma unroll
     for (int j = 0; j < L; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_void_t*)(s + j * 1024), 16, v[j], koff, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_void_t*)(s + j * 1024), 16, v[j], koff, 0, AUX);
   }
 }
 
-template <int MT, int NT, int STAGES>
+// LA: 8-row blocks of a that are fetched: 4 MT, or with few rows only those that hold any (the tile's other
+// rows are then whatever LDS holds: they reach no output row but their own, which is not stored).
+// BAUX: cache policy of b's loads.
+template <int MT, int NT, int STAGES, int LA, int BAUX, bool TAIL>
 __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
     GemmBatch batch, int count, int M, int N, int K, int64_t ldc, int tiles_m, int tiles_n, int cols) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host pass only needs the stub, and cannot instantiate the device builtins
-  constexpr int RA = 32 * MT, RB = 32 * NT, LA = RA / 8, LB = RB / 8;
+  constexpr int RA = 32 * MT, RB = 32 * NT, LB = RB / 8;
   constexpr int STAGE = (RA + RB) * KS_ROWB;
-  static_assert(STAGES == 2, "the k loop waits for one slab beside the one in use");
+  static_assert(STAGES == 2 || STAGES == 3, "the k loop waits for at most two slabs beside the one in use");
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_ks[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, lhi = lane >> 5;
   const int nk = (K + BK - 1) / BK;
   const int tail_chunks = (K % BK) / 8;
-  const bool even = ((lane & 7) ^ (lane >> 4)) < tail_chunks;
-  const bool odd = ((lane & 7) ^ (lane >> 4) ^ 4) < tail_chunks;
+  const bool even = TAIL && ((lane & 7) ^ (lane >> 4)) < tail_chunks;
+  const bool odd = TAIL && ((lane & 7) ^ (lane >> 4) ^ 4) < tail_chunks;
   // Row r of a slab keeps its 16-byte chunk c at position c ^ ((r >> 1) & 7) (see the file
   // comment).  Offsets are inside the tile: its descriptors begin at its first row and end
   // behind its last one, so that rows past M, N or the tile's columns read as zeros.
@@ -284,13 +293,28 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
     int pid = t;
     const int per_xcd = num_tiles / 8;
     if (t < per_xcd * 8) pid = (t & 7) * per_xcd + (t >> 3);
-    const int product = pid / tiles_per_product;
-    pid -= product * tiles_per_product;
-    const int m0 = (pid % tiles_m) * RA, n0 = (pid / tiles_m) * cols;
+    // One product of one row tile, the usual call, needs no division and finds its pointers among the first
+    // arguments fetched; `out` and `bias` are asked for here, not behind the k loop.
+    const uint16_t *a = batch.a[0], *b = batch.b[0], *bias = batch.bias[0];
+    uint16_t* out = batch.out[0];
+    if (count > 1) {
+      const int product = pid / tiles_per_product;
+      pid -= product * tiles_per_product;
+      a = batch.a[product];
+      b = batch.b[product];
+      bias = batch.bias[product];
+      out = batch.out[product];
+    }
+    int m0 = 0, n0 = pid * cols;
+    if (tiles_m > 1) {
+      const int column = pid / tiles_m;
+      m0 = (pid - column * tiles_m) * RA;
+      n0 = column * cols;
+    }
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(batch.a[product]) + (size_t)m0 * K, 0, (uint32_t)min(M - m0, RA) * (uint32_t)K * 2u, 0x00020000);
+        const_cast<uint16_t*>(a) + (size_t)m0 * K, 0, (uint32_t)min(M - m0, RA) * (uint32_t)K * 2u, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(batch.b[product]) + (size_t)n0 * K, 0, (uint32_t)min(N - n0, cols) * (uint32_t)K * 2u, 0x00020000);
+        const_cast<uint16_t*>(b) + (size_t)n0 * K, 0, (uint32_t)min(N - n0, cols) * (uint32_t)K * 2u, 0x00020000);
 
     f32x16_t acc[MT][NT];
 #pragma unroll
@@ -300,25 +324,30 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    // slabs `wave`, wave + 4, ...; b first: it is the operand that comes from far
-    int slab = wave;
-    if (slab < nk) {
-      const bool tail = tail_chunks && slab == nk - 1;
-      ks_issue<LB>(db, vb, mine + RA * KS_ROWB, (uint32_t)slab * KS_ROWB, tail, even, odd);
-      ks_issue<LA>(da, va, mine, (uint32_t)slab * KS_ROWB, tail, even, odd);
-    }
-    for (int stage = 0; slab < nk; slab += KS_WAVES, stage ^= 1) {
-      const int next = slab + KS_WAVES;
-      if (next < nk) {
-        uint8_t* s = mine + (stage ^ 1) * STAGE;
-        const bool tail = tail_chunks && next == nk - 1;
-        ks_issue<LB>(db, vb, s + RA * KS_ROWB, (uint32_t)next * KS_ROWB, tail, even, odd);
-        ks_issue<LA>(da, va, s, (uint32_t)next * KS_ROWB, tail, even, odd);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + LB) : "memory");  // all but the loads just issued
+    // slabs `wave`, wave + 4, ..., STAGES - 1 ahead; b first: it is the operand that comes from far
+    int next = wave;
+    uint32_t fill = 0, use = 0;
+    auto issue = [&]() {
+      const bool last = next == nk - 1;
+      uint8_t* s = mine + fill;
+      ks_issue<LB, BAUX, TAIL>(db, vb, s + RA * KS_ROWB, (uint32_t)next * KS_ROWB, last, even, odd);
+      ks_issue<LA, 0, TAIL>(da, va, s, (uint32_t)next * KS_ROWB, last, even, odd);
+      next += KS_WAVES;
+      fill = fill == (STAGES - 1) * STAGE ? 0 : fill + STAGE;
+    };
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i)
+      if (next < nk) issue();
+    for (int slab = wave; slab < nk; slab += KS_WAVES, use = use == (STAGES - 1) * STAGE ? 0 : use + STAGE) {
+      if (next < nk) {  // wait for all but the slabs behind this one
+        issue();
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * (LA + LB)) : "memory");
+      } else if (STAGES == 3 && slab + KS_WAVES < nk) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + LB) : "memory");
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
-      const uint8_t* pa = mine + stage * STAGE;
+      const uint8_t* pa = mine + use;
       const uint8_t* pb = pa + RA * KS_ROWB;
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
@@ -353,8 +382,6 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
           *reinterpret_cast<f32x4_t*>(sums + (i * 32 + l32) * PITCH + (j * 32 + 8 * q + 4 * lhi) * 4) =
               f32x4_t{acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
     __syncthreads();
-    uint16_t* __restrict__ out = batch.out[product];
-    const uint16_t* __restrict__ bias = batch.bias[product];
     for (int g = tid; g < RA * RB / 4; g += KS_THREADS) {
       const int m = g / (RB / 4), c = (g % (RB / 4)) * 4;
       if (m0 + m < M && c < cols && n0 + c < N) {  // N and cols are multiples of 4
@@ -721,12 +748,12 @@ static int allow_lds(const void* kernel, std::atomic<bool>* ok, int max_devices,
 }
 constexpr int kMaxDevices = 64;
 
-template <int MT, int NT>
+template <int MT, int NT, int STAGES, int LA, int BAUX, bool TAIL>
 static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc, int max_cus,
                          hipStream_t hs) {
-  constexpr int STAGES = 2, LDS = ks_lds_bytes(MT, NT, STAGES);
+  constexpr int LDS = ks_lds_bytes(MT, NT, STAGES);
   static std::atomic<bool> lds_ok[kMaxDevices];
-  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES>), lds_ok, kMaxDevices,
+  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES, LA, BAUX, TAIL>), lds_ok, kMaxDevices,
                          LDS))
     return rc;
   int cus = device_compute_units();
@@ -740,19 +767,37 @@ static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N
   const int64_t tiles_n = (N + cols - 1) / cols;
   int64_t grid = count * tiles_m * tiles_n;
   if (max_cus > 0 && grid > max_cus) grid = max_cus;
-  launch_kernel(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES>, dim3((unsigned)grid), dim3(KS_THREADS), LDS, hs, batch, count,
+  launch_kernel(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES, LA, BAUX, TAIL>, dim3((unsigned)grid), dim3(KS_THREADS), LDS, hs, batch, count,
                 (int)M, (int)N, (int)K, ldc, (int)tiles_m, (int)tiles_n, cols);
   return TW_OK;
 }
 
+// b's loads carry the non-temporal bit (KS_STREAM) where a launch's weights are so large that the last-level
+// cache (256 MB) does not keep three of them: from memory b arrives 8-12 % faster that way, but past that cache
+// too.  [M, 7168] x [8192, 7168]^T (117 MB), three or four in turn: 8 rows 21.4 -> 18.9 us, 32: 24.6 -> 22.5, 64:
+// 31.1 -> 28.8; not beyond (128 rows: 37.4 / 37.6, the unit's outstanding lines are shared with a).  Four products
+// [20, 2048] (134 MB) 33.9 -> 28.8.  Below the line, from the cache: [32, 4160] (68 MB) 12.1 -> 14.2, eight products
+// [8, 768] x [6144, 768]^T (75 MB) 20.9 -> 22.0.  Not where rows of b are not whole lines: the line that two slabs
+// share would be fetched twice (8 rows, K = 3696: 11.1 -> 13.4).
+constexpr int KS_STREAM = 2;  // nt
+constexpr double KS_STREAM_BYTES = 96.0 * 1024 * 1024;
+
 // The rule looks at M, N and K alone: a product has the same bits under every grid cap and in
-// every batch.  Up to 32 columns a second column half would be empty LDS and idle MFMAs: 256 rows x 16
+// every batch (the policy of the loads changes none).  Up to 32 columns a second column half would be empty LDS and idle MFMAs: 256 rows x 16
 // columns 4.6 -> 4.1 us at K = 128, 13.7 -> 9.5 at 4096.
 static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
                              int max_cus, hipStream_t hs) {
-  if (M <= 32) return launch_ksplit<1, 1>(batch, count, M, N, K, ldc, max_cus, hs);
-  if (M <= 64 || N <= 32) return launch_ksplit<2, 1>(batch, count, M, N, K, ldc, max_cus, hs);
-  return launch_ksplit<2, 2>(batch, count, M, N, K, ldc, max_cus, hs);
+  const bool stream = M <= 64 && (double)count * N * K * 2 > KS_STREAM_BYTES;
+#define TW_KSPLIT(MT, NT, STAGES, LA)                                                                              \
+  return K % BK ? launch_ksplit<MT, NT, STAGES, LA, 0, true>(batch, count, M, N, K, ldc, max_cus, hs)              \
+         : stream ? launch_ksplit<MT, NT, STAGES, LA, KS_STREAM, false>(batch, count, M, N, K, ldc, max_cus, hs)   \
+                  : launch_ksplit<MT, NT, STAGES, LA, 0, false>(batch, count, M, N, K, ldc, max_cus, hs)
+  if (M <= 8) TW_KSPLIT(1, 1, 3, 1);
+  if (M <= 16) TW_KSPLIT(1, 1, 3, 2);
+  if (M <= 32) TW_KSPLIT(1, 1, 3, 4);
+  if (M <= 64 || N <= 32) TW_KSPLIT(2, 1, 2, 8);
+  TW_KSPLIT(2, 2, 2, 8);
+#undef TW_KSPLIT
 }
 
 template <int TM, int TN, bool TAIL>
