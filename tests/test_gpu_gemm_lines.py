@@ -1,0 +1,60 @@
+"""The tile GEMM kernel where it fetches whole lines of rows that are not whole lines (K a multiple of 16, not of
+64): every shape with room for it, one slab to more than the ring holds, several tiles per workgroup, operands
+that begin anywhere in a line with NaN on both sides of them, and products of a batch that begin differently.
+
+Zeros behind the last element of every row make the same product one of whole slabs, whose loads are others but
+whose sums are the same: no bit may differ.  That product is held against float64 as in test_gpu_gemm_ksplit.py."""
+import pytest
+import torch
+
+from test_gpu_gemm_ksplit import assert_product
+from test_gpu_gemm_tiles import forced  # noqa: F401 (fixture)
+from tokenweave_amd import _custom_ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+SHAPES = ((4, 8), (3, 8), (4, 6), (3, 6), (4, 4), (3, 4), (2, 4))
+
+
+def placed(rows, K, offset, g):
+    """[rows, K] that begins `offset` elements into a line, between NaNs."""
+    flat = torch.full((rows * K + offset + 128,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    t = flat[offset:offset + rows * K].view(rows, K)
+    return t.copy_(torch.randn(rows, K, generator=g, device=DEV))
+
+
+def padded(t):
+    return torch.nn.functional.pad(t, (0, -t.shape[1] % 64)).contiguous()
+
+
+@pytest.mark.parametrize("K", [16, 48, 80, 112, 208, 336, 1072])
+@pytest.mark.parametrize("tm,tn", SHAPES)
+def test_every_shape(forced, tm, tn, K):  # noqa: F811
+    M, N = 2 * 32 * tm + 17, 2 * 32 * tn + 24         # nine tiles, the last row and column of them partial
+    g = torch.Generator(device=DEV).manual_seed(100 * tm + 10 * tn + K)
+    for at_a, at_b in ((0, 0), (8, 48), (32, 56)):
+        a, b = placed(M, K, at_a, g), placed(N, K, at_b, g)
+        want = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+        forced(want, padded(a), padded(b), None, tm, tn, 0)
+        torch.cuda.synchronize()
+        assert_product(want, a, b, f"{tm} {tn} {K}")
+        for cus in (0, 1, 4):
+            print(f"[case] lines {32 * tm}x{32 * tn} K={K} at {at_a} {at_b} cus={cus}", flush=True)
+            out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+            forced(out, a, b, None, tm, tn, cus)
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), (at_a, at_b, cus)
+
+
+@pytest.mark.parametrize("cap", [None, 5])
+def test_a_batch_whose_products_begin_differently(cap):
+    P, M, N, K = 4, 150, 392, 176
+    g = torch.Generator(device=DEV).manual_seed(7)
+    a = [placed(M, K, 16 * p, g) for p in range(P)]
+    b = [placed(N, K, 8 * p + 8, g) for p in range(P)]
+    outs = [torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(P)]
+    ops.gemm_bf16_nt_partials(outs, a, b, cap)
+    for p in range(P):
+        want = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+        ops.gemm_bf16_nt(want, padded(a[p]), padded(b[p]))
+        assert torch.equal(outs[p], want), p

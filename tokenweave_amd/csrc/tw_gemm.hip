@@ -454,7 +454,8 @@ constexpr int64_t TILE_MAX_LDC = 1 << 21;
 [[maybe_unused]] constexpr uint32_t TILE_OUT_OF_RANGE = 0x80000000u;
 
 // How a tile shape uses LDS and where in a slab (slots: its 2 TM TN MFMAs) its loads go out.
-template <int TM, int TN>
+enum TileRows { kWholeSlabs, kPartialSlab, kLines };  // see the kernel
+template <int TM, int TN, TileRows ROWS = kWholeSlabs>
 struct TileShape {
   static constexpr int BM = 32 * TM, BN = 32 * TN, SLOTS = TM * TN;
   static constexpr int LA = TM, LB = TN, L = LA + LB;  // wave loads (8 rows each) per slab and operand
@@ -462,10 +463,14 @@ struct TileShape {
   static constexpr int STAGES = 160 * 1024 / (PA + PB);
   // Two whole stages only: a third a panel, so that a's loads can go out in the phase before the
   // barrier, b's in the one behind it.
-  static constexpr bool TIGHT = STAGES == 2;
+  static constexpr bool TAKES_LINES = 4 * PA + 3 * PB <= 160 * 1024;
+  static constexpr bool LINES = ROWS == kLines;
+  static_assert(!LINES || TAKES_LINES, "no room for the line behind the slab in use");
+  static constexpr bool TIGHT = LINES ? STAGES < 4 : STAGES == 2;
+  static constexpr int NEED = LINES ? 2 : 1;  // slabs behind the one in use that its barrier waits for
   // slabs ahead; three at most: with four or five the 64- to 128-row tiles take longer to start than they
   // gain ([256, 1024] x [8192, 1024]^T 8.3 -> 8.8 us, [160, 3584] x [8192, 3584]^T 18.2 -> 18.8)
-  static constexpr int D = TIGHT ? 2 : (STAGES - 1 < 3 ? STAGES - 1 : 3);
+  static constexpr int D = LINES ? (STAGES < 5 ? 3 : 4) : TIGHT ? 2 : (STAGES - 1 < 3 ? STAGES - 1 : 3);
   static constexpr int SA = D + 1, SB = TIGHT ? D : D + 1;
   static constexpr int LDS = SA * PA + SB * PB;
   static constexpr int SPREAD = 2 * SLOTS / L;
@@ -479,10 +484,10 @@ struct TileShape {
     return c;
   }
   static constexpr int EARLY = before(A0, A_STEP, LA) + before(B0, B_STEP, LB);
-  // may be outstanding at a slab's barrier: slabs 2 .. D - 1 ahead and the early part of slab D
-  static constexpr int IN_FLIGHT = (D - 2) * L + EARLY;
+  // may be outstanding at a slab's barrier: slabs NEED + 1 .. D - 1 ahead and the early part of slab D
+  static constexpr int IN_FLIGHT = (D - 1 - NEED) * L + EARLY;
   static constexpr int STORES = SLOTS / 2;
-  static_assert(SPREAD >= 1 && D >= 2 && LDS <= 160 * 1024 && IN_FLIGHT + STORES <= 63, "tile shape");
+  static_assert(SPREAD >= 1 && D > NEED && LDS <= 160 * 1024 && IN_FLIGHT + STORES <= 63, "tile shape");
   static_assert(A0 + (LA - 1) * A_STEP < 2 * SLOTS && B0 + (LB - 1) * B_STEP < 2 * SLOTS, "every load has a slot");
   static_assert((L - 1) * READ_STEP < SLOTS, "every fragment read has a slot");
 };
@@ -503,13 +508,13 @@ __device__ __forceinline__ uint32_t tile_pack2(float lo, float hi) {
 
 // One phase: acc += fb x fa, and between the MFMAs the next phase's fragments (na, nb from pa, pb)
 // and this half's share of the loads of the slab D ahead.
-template <int TM, int TN, bool FIRST, int HALF>
+template <int TM, int TN, TileRows ROWS, bool FIRST, int HALF>
 __device__ __forceinline__ void tile_phase(f32x4_t (&acc)[TM][TN], const bf16x8_t (&fa)[TM], const bf16x8_t (&fb)[TN],
                                            bf16x8_t (&na)[TM], bf16x8_t (&nb)[TN], const lds_u8_t* pa,
-                                           const lds_u8_t* pb, __amdgpu_buffer_rsrc_t da, __amdgpu_buffer_rsrc_t db,
-                                           const uint32_t (&va)[TM], const uint32_t (&vb)[TN], lds_u8_t* sa,
-                                           lds_u8_t* sb, uint32_t koff) {
-  using S = TileShape<TM, TN>;
+                                           const lds_u8_t* pb, __amdgpu_buffer_rsrc_t da,
+                                           __amdgpu_buffer_rsrc_t db, const uint32_t (&va)[TM],
+                                           const uint32_t (&vb)[TN], lds_u8_t* sa, lds_u8_t* sb, uint32_t koff) {
+  using S = TileShape<TM, TN, ROWS>;
 #pragma unroll
   for (int n = 0; n < S::SLOTS; ++n) {
     const int i = n / TN, j = n % TN, slot = n + HALF * S::SLOTS;
@@ -533,6 +538,22 @@ __device__ __forceinline__ void tile_phase(f32x4_t (&acc)[TM][TN], const bf16x8_
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+}
+
+// The loads of one half of a slab, where no MFMAs are to be had between them.
+template <int TM, int TN, TileRows ROWS, int HALF>
+__device__ __forceinline__ void tile_loads(__amdgpu_buffer_rsrc_t da, __amdgpu_buffer_rsrc_t db,
+                                           const uint32_t (&va)[TM], const uint32_t (&vb)[TN], lds_u8_t* sa,
+                                           lds_u8_t* sb, uint32_t koff) {
+  using S = TileShape<TM, TN, ROWS>;
+#pragma unroll
+  for (int l = 0; l < S::LA; ++l)
+    if ((S::A0 + l * S::A_STEP >= S::SLOTS) == (HALF == 1))
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(da, (lds_void_t*)(sa + l * 1024), 16, va[l], koff, 0, 0);
+#pragma unroll
+  for (int l = 0; l < S::LB; ++l)
+    if ((S::B0 + l * S::B_STEP >= S::SLOTS) == (HALF == 1))
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(db, (lds_void_t*)(sb + l * 1024), 16, vb[l], koff, 0, 0);
 }
 
 constexpr int kStoreThrough = 19;  // nt sc0 sc1
@@ -576,6 +597,9 @@ struct TilePlace {
   int product, m0, n0;
 };
 
+// Where in its 128-byte line a row begins, in 16-byte chunks.
+__device__ __forceinline__ int line_phase(const uint16_t* row) { return (int)(reinterpret_cast<uintptr_t>(row) >> 4) & 7; }
+
 template <int TM, int TN>
 __device__ __forceinline__ TilePlace tile_place(int t, int num_tiles, int tiles_m, int tiles_n) {
   using S = TileShape<TM, TN>;
@@ -595,31 +619,42 @@ __device__ __forceinline__ TilePlace tile_place(int t, int num_tiles, int tiles_
 }
 #endif
 
-// TAIL: the last slab is a partial one.  (Apart from the others because switching the offsets costs
+// kPartialSlab: the last slab is a partial one.  (Apart from the others because switching the offsets costs
 // the k loop a register move per load and slab: 341 against 324 us for 8192 x 8192 x 3584.  Zeroing the
-// fragments instead needs no moves and is no faster, 227 against 230 us for 16384 x 8192 x 1000: what such
-// a K costs is that its rows are not whole lines, 46 against 58 us for 1000 rows at K = 3584 and 3696.)
-template <int TM, int TN, bool TAIL>
+// fragments instead needs no moves and is no faster, 227 against 230 us for 16384 x 8192 x 1000.)
+//
+// kLines: rows of such a K are not whole lines, and a slab of a row mostly lies on two of them, which a compute
+// unit then requests twice: its L1 has about 126 requests under way whatever the kernel does, so it is the
+// number of requests that bounds such a product ([1000, 3696] x [8192, 3696]^T: 9.9 million requests of 357 cycles
+// in 108 thousand cycles of every L1, 1.73 a slab row).  Here a load fetches the lines themselves, one a row and
+// slab, and a fragment read finds the first part of its slab in the ring's panel of that slab and the rest
+// in the next one.  That wants one panel more in the ring, and K % 16 == 0: rows two apart then begin at the
+// same place of a line or half a line apart, which the swizzle takes care of.  Aligned 64 bytes have to stay with
+// groups of four lanes: rotated by other amounts the loads take half of the gain back.  Same bits.
+// One product with 8192 columns, K = 3696, kPartialSlab -> kLines, operands rotated through three sets: 200 rows 25.8 ->
+// 23.2 us, 256: 27.1 -> 23.6, 512: 37.5 -> 32.6, 1000: 54.8 -> 50.8; K = 7392: 200 rows 63 -> 49, 256: 72 -> 56, 400: 79 -> 70.
+template <int TM, int TN, TileRows ROWS>
 __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THREADS) void gemm_bf16_nt_tile_kernel(
     GemmBatch batch, int count, int M, int N, int K, int64_t ldc, int tiles_m, int tiles_n, int wide_store) {
 #ifdef __HIP_DEVICE_COMPILE__
-  using S = TileShape<TM, TN>;
+  using S = TileShape<TM, TN, ROWS>;
   constexpr int LA = S::LA, LB = S::LB, PA = S::PA, PB = S::PB, D = S::D;
+  constexpr uint32_t AHEAD = S::LINES ? 128 : 0;  // the loads' offsets begin a line ahead of the tile
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_tile[];
   lds_u8_t* const lds_a = (lds_u8_t*)lds_tile;
   lds_u8_t* const lds_b = lds_a + S::SA * PA;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, quad = lane >> 4;
-  const int nk = (K + BK - 1) / BK;
-  const int tail_chunks = TAIL ? (K % BK) / 8 : 8;  // 16-byte chunks of the last slab that lie inside K
+  const int nk = (K + BK - 1) / BK, nl = nk + (S::LINES ? 1 : 0);  // slabs; loads of a tile
+  const int tail_chunks = ROWS == kPartialSlab ? (K % BK) / 8 : 8;  // 16-byte chunks of the last slab that lie inside K
   const int num_tiles = count * tiles_m * tiles_n;
 
   // Reader: the two 32-wide halves of a slab.
   const uint32_t row_a = (wm * 16 * TM + r16) * 128, row_b = (wn * 16 * TN + (r16 >> 2) * 8 + (r16 & 3)) * 128;
   const uint32_t chunk0 = (quad ^ (r16 >> 1)) << 4, chunk1 = ((4 + quad) ^ (r16 >> 1)) << 4;
-  const lds_u8_t *const a0 = lds_a + row_a + chunk0, *const a1 = lds_a + row_a + chunk1;
-  const lds_u8_t *const b0 = lds_b + row_b + chunk0, *const b1 = lds_b + row_b + chunk1;
+  const lds_u8_t *a0 = lds_a + row_a + chunk0, *a1 = lds_a + row_a + chunk1;
+  const lds_u8_t *b0 = lds_b + row_b + chunk0, *b1 = lds_b + row_b + chunk1;
   // Loader: wave instruction l fills the 8-row block wave * L + l; lane l lands at row l / 8,
   // position l % 8 of it and fetches the chunk that belongs there.  Offsets are inside the tile,
   // whose descriptors end with the last row of the operand: rows past it read as zeros.
@@ -638,6 +673,24 @@ __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THR
       vb[l] = c < (chunks) ? (uint32_t)((blk * 8 + (lane >> 3)) * K + c * 8) * 2u : TILE_OUT_OF_RANGE;       \
     }                                                                                                        \
   } while (0)
+  // kLines: the same for line `line` of every row: lane position x holds the line's chunk x ^ key ^ flip, so
+  // that aligned groups of four lanes fetch aligned 64 bytes.  kc: the chunk of the row that this is.
+#define TW_TILE_LINE_OFFSET(v, blk, key, phase, line)                                                        \
+  do {                                                                                                       \
+    const int row = (blk)*8 + (lane >> 3), j = (lane & 7) ^ (key) ^ (flip & (row << 1));                     \
+    const int kc = (line)*8 + j - (((phase) + row * row_chunks) & 7);                                        \
+    v = kc >= 0 && kc < row_chunks ? (uint32_t)(row * K + (kc - (line)*8 + 8) * 8) * 2u : TILE_OUT_OF_RANGE; \
+  } while (0)
+#define TW_TILE_LINE_OFFSETS(line)                                                                           \
+  do {                                                                                                       \
+    _Pragma("unroll") for (int l = 0; l < LA; ++l)                                                           \
+        TW_TILE_LINE_OFFSET(va[l], wave * LA + l, (((wave * LA + l) & 1) << 2) | (lane >> 4), load_phase_a, line); \
+    _Pragma("unroll") for (int l = 0; l < LB; ++l) TW_TILE_LINE_OFFSET(                                      \
+        vb[l], wave * LB + l, ((lane >> 4) & 1) | (((wave * LB + l) & 3) << 1), load_phase_b, line);         \
+  } while (0)
+  const int row_chunks = K / 8;
+  const int flip = (row_chunks & 2) << 1;  // 4 where rows two apart begin half a line apart
+  int load_phase_a = 0, load_phase_b = 0;  // where in a line the product's first row begins, in chunks
   // Load cursor: slab lk of tile lt.  Past the last tile it stays at slab 0 of an empty descriptor:
   // its loads ask memory for nothing.  (The hardware compares with the extent less the slab's offset,
   // which for an extent of 0 must not go below 0.)
@@ -647,27 +700,33 @@ __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THR
   do {                                                                                                       \
     const bool in = lt < num_tiles;                                                                          \
     const TilePlace p = tile_place<TM, TN>(in ? lt : 0, num_tiles, tiles_m, tiles_n);                        \
-    da = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(batch.a[p.product]) + (size_t)p.m0 * K, 0,  \
-                                           in ? (uint32_t)min(M - p.m0, S::BM) * (uint32_t)K * 2u : 0u,      \
+    const uint16_t *pa = batch.a[p.product] + (size_t)p.m0 * K, *pb = batch.b[p.product] + (size_t)p.n0 * K; \
+    if (S::LINES) load_phase_a = line_phase(pa), load_phase_b = line_phase(pb);                              \
+    da = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pa) - (int)AHEAD / 2, 0,                         \
+                                           in ? (uint32_t)min(M - p.m0, S::BM) * (uint32_t)K * 2u + AHEAD : 0u, \
                                            0x00020000);                                                      \
-    db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(batch.b[p.product]) + (size_t)p.n0 * K, 0,  \
-                                           in ? (uint32_t)min(N - p.n0, S::BN) * (uint32_t)K * 2u : 0u,      \
+    db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pb) - (int)AHEAD / 2, 0,                         \
+                                           in ? (uint32_t)min(N - p.n0, S::BN) * (uint32_t)K * 2u + AHEAD : 0u, \
                                            0x00020000);                                                      \
   } while (0)
 #define TW_TILE_ADVANCE()                                                                                    \
   do {                                                                                                       \
     if (lt < num_tiles) ++lk;                                                                                \
-    if (lk == nk) {                                                                                          \
+    if (lk == nl) {                                                                                          \
       lk = 0;                                                                                                \
       lt += gridDim.x;                                                                                       \
       TW_TILE_DESCRIPTORS();                                                                                 \
-      if (TAIL) TW_TILE_OFFSETS(nk == 1 ? tail_chunks : 8);                                                  \
-    } else if (TAIL && lk == nk - 1) {                                                                       \
+      if (S::LINES) TW_TILE_LINE_OFFSETS(0);                                                                 \
+      else if (ROWS == kPartialSlab) TW_TILE_OFFSETS(nk == 1 ? tail_chunks : 8);                             \
+    } else if (S::LINES && (lk == 1 || lk >= nk - 1)) {                                                      \
+      if (lt < num_tiles) TW_TILE_LINE_OFFSETS(lk);                                                          \
+    } else if (ROWS == kPartialSlab && lk == nk - 1) {                                                       \
       TW_TILE_OFFSETS(tail_chunks);                                                                          \
     }                                                                                                        \
   } while (0)
   TW_TILE_DESCRIPTORS();
-  TW_TILE_OFFSETS(nk == 1 ? tail_chunks : 8);
+  if (S::LINES) TW_TILE_LINE_OFFSETS(0);
+  else TW_TILE_OFFSETS(nk == 1 ? tail_chunks : 8);
 #pragma unroll
   for (int s = 0; s < D; ++s) {
 #pragma unroll
@@ -678,36 +737,58 @@ __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THR
       __builtin_amdgcn_raw_ptr_buffer_load_lds(db, (lds_void_t*)(wb + s * PB + l * 1024), 16, vb[l], lk * 128u, 0, 0);
     TW_TILE_ADVANCE();
   }
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 1) * S::L) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - S::NEED) * S::L) : "memory");
   f32x4_t acc[TM][TN];
   bf16x8_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
-#pragma unroll
-  for (int r = 0; r < TN; ++r) fb0[r] = *(lds_frag_t*)(b0 + (r >> 1) * 4096 + (r & 1) * 512);
-#pragma unroll
-  for (int r = 0; r < TM; ++r) fa0[r] = *(lds_frag_t*)(a0 + r * 2048);
-
   // ring positions: the slab in use and the one being filled
   uint32_t use_a = 0, use_b = 0, fill_a = (D % S::SA) * PA, fill_b = (D % S::SB) * PB;
-#define TW_RING(x, panel, n) x = (x) + (panel) == (n) * (panel) ? 0u : (x) + (panel)
+#define TW_NEXT(x, panel, n) ((x) + (panel) == (n) * (panel) ? 0u : (x) + (panel))
+#define TW_RING(x, panel, n) x = TW_NEXT(x, panel, n)
+  // kLines: the chunks 8 - phase and up of a row's slab lie in the line behind it.  The fragments of a lane are rows
+  // that begin alike in their lines.
+  bool next_a0 = false, next_a1 = false, next_b0 = false, next_b1 = false;
+  auto place_reader = [&](int t) {
+    const TilePlace p = tile_place<TM, TN>(t, num_tiles, tiles_m, tiles_n);
+    const int pa = line_phase(batch.a[p.product]) + (r16 & 1) * row_chunks, fa = (pa & 7) ^ (flip & (r16 << 1));
+    const int pb = line_phase(batch.b[p.product]) + (r16 & 1) * row_chunks, fb = (pb & 7) ^ (flip & (r16 << 1));
+    next_a0 = quad + fa >= 8, next_a1 = 4 + quad + fa >= 8;
+    next_b0 = quad + fb >= 8, next_b1 = 4 + quad + fb >= 8;
+    a0 = lds_a + row_a + ((((quad + pa) & 7) ^ (r16 >> 1)) << 4);
+    a1 = lds_a + row_a + ((((4 + quad + pa) & 7) ^ (r16 >> 1)) << 4);
+    b0 = lds_b + row_b + ((((quad + pb) & 7) ^ (r16 >> 1)) << 4);
+    b1 = lds_b + row_b + ((((4 + quad + pb) & 7) ^ (r16 >> 1)) << 4);
+  };
+#define TW_AT(x, ptr, next, panel, n) ((ptr) + (S::LINES && (next) ? TW_NEXT(x, panel, n) : (x)))
+#define TW_TILE_READ_FIRST()                                                                                 \
+  do {                                                                                                       \
+    const lds_u8_t *const pb = TW_AT(use_b, b0, next_b0, PB, S::SB), *const pa = TW_AT(use_a, a0, next_a0, PA, S::SA); \
+    _Pragma("unroll") for (int r = 0; r < TN; ++r)                                                           \
+        fb0[r] = *(lds_frag_t*)(pb + (r >> 1) * 4096 + (r & 1) * 512);                                       \
+    _Pragma("unroll") for (int r = 0; r < TM; ++r) fa0[r] = *(lds_frag_t*)(pa + r * 2048);                   \
+  } while (0)
+  if (S::LINES) place_reader(blockIdx.x);
+  TW_TILE_READ_FIRST();
 #define TW_TILE_SLAB(FIRST, AFTER_STORE)                                                                         \
   do {                                                                                                       \
-    tile_phase<TM, TN, FIRST, 0>(acc, fa0, fb0, fa1, fb1, a1 + use_a, b1 + use_b, da, db, va, vb, wa + fill_a, \
-                                 wb + fill_b, lk * 128u);                                                    \
+    tile_phase<TM, TN, ROWS, FIRST, 0>(acc, fa0, fb0, fa1, fb1, TW_AT(use_a, a1, next_a1, PA, S::SA),          \
+                                       TW_AT(use_b, b1, next_b1, PB, S::SB), \
+                                       da, db, va, vb, wa + fill_a, wb + fill_b, lk * 128u);                 \
     if (AFTER_STORE)                                                                                         \
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S::IN_FLIGHT + S::STORES) : "memory"); \
     else                                                                                                     \
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S::IN_FLIGHT) : "memory");            \
     TW_RING(use_a, PA, S::SA);                                                                               \
     TW_RING(use_b, PB, S::SB);                                                                               \
-    tile_phase<TM, TN, false, 1>(acc, fa1, fb1, fa0, fb0, a0 + use_a, b0 + use_b, da, db, va, vb, wa + fill_a, \
-                                 wb + fill_b, lk * 128u);                                                    \
+    tile_phase<TM, TN, ROWS, false, 1>(acc, fa1, fb1, fa0, fb0, TW_AT(use_a, a0, next_a0, PA, S::SA),          \
+                                       TW_AT(use_b, b0, next_b0, PB, S::SB), \
+                                       da, db, va, vb, wa + fill_a, wb + fill_b, lk * 128u);                 \
     TW_TILE_ADVANCE();                                                                                       \
     TW_RING(fill_a, PA, S::SA);                                                                              \
     TW_RING(fill_b, PB, S::SB);                                                                              \
   } while (0)
 
   for (int t = blockIdx.x; t < num_tiles; t += gridDim.x) {
-    TW_TILE_SLAB(true, t != (int)blockIdx.x);
+    TW_TILE_SLAB(true, !S::LINES && t != (int)blockIdx.x);
     for (int kt = 1; kt < nk; ++kt) TW_TILE_SLAB(false, false);
 
     const TilePlace p = tile_place<TM, TN>(t, num_tiles, tiles_m, tiles_n);
@@ -725,11 +806,29 @@ __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THR
       if (wide_store) tile_store<TM, TN, true, false>(acc, dc, row_off, row_step, p.n0 + col, N, bias);
       else tile_store<TM, TN, false, false>(acc, dc, row_off, row_step, p.n0 + col, N, bias);
     }
+    // The tile's rows have one line more than slabs: a slab without products between this tile and the next.
+    if (S::LINES && t + (int)gridDim.x < num_tiles) {
+      tile_loads<TM, TN, ROWS, 0>(da, db, va, vb, wa + fill_a, wb + fill_b, lk * 128u);
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S::IN_FLIGHT + S::STORES) : "memory");
+      TW_RING(use_a, PA, S::SA);
+      TW_RING(use_b, PB, S::SB);
+      place_reader(t + gridDim.x);
+      TW_TILE_READ_FIRST();
+      tile_loads<TM, TN, ROWS, 1>(da, db, va, vb, wa + fill_a, wb + fill_b, lk * 128u);
+      TW_TILE_ADVANCE();
+      TW_RING(fill_a, PA, S::SA);
+      TW_RING(fill_b, PB, S::SB);
+    }
   }
 #undef TW_TILE_SLAB
+#undef TW_TILE_READ_FIRST
+#undef TW_AT
+#undef TW_NEXT
 #undef TW_RING
 #undef TW_TILE_ADVANCE
 #undef TW_TILE_DESCRIPTORS
+#undef TW_TILE_LINE_OFFSETS
+#undef TW_TILE_LINE_OFFSET
 #undef TW_TILE_OFFSETS
 #endif
 }
@@ -800,12 +899,12 @@ static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64
 #undef TW_KSPLIT
 }
 
-template <int TM, int TN, bool TAIL>
+template <int TM, int TN, TileRows ROWS>
 static int launch_tile_kernel(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
                        int max_cus, hipStream_t hs) {
-  using S = TileShape<TM, TN>;
+  using S = TileShape<TM, TN, ROWS>;
   static std::atomic<bool> lds_ok[kMaxDevices];
-  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<TM, TN, TAIL>), lds_ok, kMaxDevices,
+  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_tile_kernel<TM, TN, ROWS>), lds_ok, kMaxDevices,
                          S::LDS))
     return rc;
   const int tiles_m = (int)((M + S::BM - 1) / S::BM), tiles_n = (int)((N + S::BN - 1) / S::BN);
@@ -817,7 +916,7 @@ static int launch_tile_kernel(const GemmBatch& batch, int count, int64_t M, int6
   int wide_store = (N % 8 == 0 && ldc % 8 == 0) ? 1 : 0;
   for (int p = 0; p < count; ++p)
     if (reinterpret_cast<uintptr_t>(batch.out[p]) & 15u) wide_store = 0;
-  launch_kernel(gemm_bf16_nt_tile_kernel<TM, TN, TAIL>, dim3((unsigned)grid), dim3(TILE_THREADS), S::LDS, hs, batch, count,
+  launch_kernel(gemm_bf16_nt_tile_kernel<TM, TN, ROWS>, dim3((unsigned)grid), dim3(TILE_THREADS), S::LDS, hs, batch, count,
                 (int)M, (int)N, (int)K, ldc, tiles_m, tiles_n, wide_store);
   return TW_OK;
 }
@@ -825,8 +924,15 @@ static int launch_tile_kernel(const GemmBatch& batch, int count, int64_t M, int6
 template <int TM, int TN>
 static int launch_tile(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
                        int max_cus, hipStream_t hs) {
-  return K % BK ? launch_tile_kernel<TM, TN, true>(batch, count, M, N, K, ldc, max_cus, hs)
-                : launch_tile_kernel<TM, TN, false>(batch, count, M, N, K, ldc, max_cus, hs);
+  // Whole lines where the shape's ring has room for the panel more.  The shapes whose ring then is down to the
+  // least (TIGHT: 128 x 256 and 96 x 256) cover less of memory's latency and are taken only where more than half of
+  // the rows lie on two lines: K = 7392, 128 x 256, 800 and 1000 rows 122 / 138 us with kPartialSlab, 132 / 133 with kLines.
+  if constexpr (TileShape<TM, TN>::TAKES_LINES) {
+    if (K % BK && K % 16 == 0 && (!TileShape<TM, TN, kLines>::TIGHT || K % 32))
+      return launch_tile_kernel<TM, TN, kLines>(batch, count, M, N, K, ldc, max_cus, hs);
+  }
+  return K % BK ? launch_tile_kernel<TM, TN, kPartialSlab>(batch, count, M, N, K, ldc, max_cus, hs)
+                : launch_tile_kernel<TM, TN, kWholeSlabs>(batch, count, M, N, K, ldc, max_cus, hs);
 }
 
 // The tile shapes, in 32-row and 32-column units, with the time a round of them takes on all
