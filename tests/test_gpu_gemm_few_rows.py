@@ -56,3 +56,17 @@ def test_a_batch_whose_weights_are_large_together():
     for p, (a, b) in enumerate(made):
         assert torch.equal(outs[p], product(a, b)), p
     assert_product(outs[P - 1], *made[P - 1], "last product")
+
+
+@pytest.mark.parametrize("N,K", [(8192, 320), (1028, 840), (36, 264), (6144, 64)])
+def test_two_row_tiles_share_the_rows_evenly(N, K):
+    """Row m is the same in every batch of 33 to 128 rows, whose tiles are of 40, 48, 56 or 64 rows, also
+    behind a product that has left NaN in the local memory of the compute units."""
+    a, b = operands(128, N, K, N + K + 1)
+    poison = torch.full((128, K), float("nan"), dtype=torch.bfloat16, device=DEV)
+    whole = product(a, b)
+    assert_product(whole, a, b, f"N={N} K={K}")
+    for M in (33, 40, 41, 48, 49, 56, 57, 64, 65, 80, 81, 96, 97, 112, 113, 127):
+        print(f"[case] shared rows M={M} N={N} K={K}", flush=True)
+        product(poison, b)
+        assert torch.equal(product(a[:M].contiguous(), b), whole[:M]), M

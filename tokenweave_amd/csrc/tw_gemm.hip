@@ -252,14 +252,15 @@ __device__ __forceinline__ void ks_issue(__amdgpu_buffer_rsrc_t d, const uint32_
   }
 }
 
-// LA: 8-row blocks of a that are fetched: 4 MT, or with few rows only those that hold any (the tile's other
-// rows are then whatever LDS holds: they reach no output row but their own, which is not stored).
+// LA: the tile's 8-row blocks of a: 4 MT, or only as many as its share of the rows needs (the rest of its MFMA
+// blocks is then whatever LDS holds: it reaches no output row but its own, which is not stored).
 // BAUX: cache policy of b's loads.
 template <int MT, int NT, int STAGES, int LA, int BAUX, bool TAIL>
 __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
     GemmBatch batch, int count, int M, int N, int K, int64_t ldc, int tiles_m, int tiles_n, int cols) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host pass only needs the stub, and cannot instantiate the device builtins
-  constexpr int RA = 32 * MT, RB = 32 * NT, LB = RB / 8;
+  constexpr int RA = 32 * MT, RB = 32 * NT, LB = RB / 8, ROWS = 8 * LA;
+  static_assert(ROWS <= RA, "a tile's rows fit its MFMA blocks");
   constexpr int STAGE = (RA + RB) * KS_ROWB;
   static_assert(STAGES == 2 || STAGES == 3, "the k loop waits for at most two slabs beside the one in use");
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_ks[];
@@ -308,11 +309,11 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
     int m0 = 0, n0 = pid * cols;
     if (tiles_m > 1) {
       const int column = pid / tiles_m;
-      m0 = (pid - column * tiles_m) * RA;
+      m0 = (pid - column * tiles_m) * ROWS;
       n0 = column * cols;
     }
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(a) + (size_t)m0 * K, 0, (uint32_t)min(M - m0, RA) * (uint32_t)K * 2u, 0x00020000);
+        const_cast<uint16_t*>(a) + (size_t)m0 * K, 0, (uint32_t)min(M - m0, ROWS) * (uint32_t)K * 2u, 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(b) + (size_t)n0 * K, 0, (uint32_t)min(N - n0, cols) * (uint32_t)K * 2u, 0x00020000);
 
@@ -382,7 +383,7 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
           *reinterpret_cast<f32x4_t*>(sums + (i * 32 + l32) * PITCH + (j * 32 + 8 * q + 4 * lhi) * 4) =
               f32x4_t{acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
     __syncthreads();
-    for (int g = tid; g < RA * RB / 4; g += KS_THREADS) {
+    for (int g = tid; g < ROWS * RB / 4; g += KS_THREADS) {
       const int m = g / (RB / 4), c = (g % (RB / 4)) * 4;
       if (m0 + m < M && c < cols && n0 + c < N) {  // N and cols are multiples of 4
         const uint8_t* p = lds_ks + m * PITCH + c * 4;
@@ -859,7 +860,7 @@ static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N
   if (cus <= 0) cus = 256;
   // Columns per workgroup: as few rounds of one workgroup per unit as full-width tiles need, and
   // then tiles no wider than that many rounds require, so that every unit streams its share of b.
-  const int64_t tiles_m = (M + 32 * MT - 1) / (32 * MT), full = (N + 32 * NT - 1) / (32 * NT);
+  const int64_t tiles_m = (M + 8 * LA - 1) / (8 * LA), full = (N + 32 * NT - 1) / (32 * NT);
   const int64_t rounds = (tiles_m * full + cus - 1) / cus;
   const int64_t per_row_tile = std::max(full, cus * rounds / tiles_m);  // column tiles those rounds have room for
   const int cols = (int)std::min<int64_t>(32 * NT, ((N + per_row_tile - 1) / per_row_tile + 3) / 4 * 4);
@@ -881,21 +882,44 @@ static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N
 constexpr int KS_STREAM = 2;  // nt
 constexpr double KS_STREAM_BYTES = 96.0 * 1024 * 1024;
 
+// Rows of a tile.  What a unit can have under way is bounded by its L1, so a short tile fetches only the 8-row
+// blocks that it has, and two row tiles take even shares of 65 to 96 rows instead of 64 and the rest: the launch
+// ends with its longest workgroup.  us, weights of three or four sets in turn, 64-row tiles / this rule:
+// [40, 1024] x [8192, 1024]^T 5.77 / 5.52, [40, 3584] 11.67 / 11.37, [40, 3696] 13.50 / 12.91, [33, 7168] 23.9 / 22.9,
+// [48, 2048] x [6144, 2048]^T 7.41 / 7.18; [72, 768] x [6144, 768]^T 6.03 / 5.59, [72, 1024] x [8192, 1024]^T 7.05 / 6.64,
+// [72, 3584] 13.53 / 12.52, [96, 1024] 7.14 / 6.93.  Even shares gain while the longest workgroup is the bound; where
+// the L2s and the memory are, they lose: weights past KS_EVEN_BYTES ([80, 7168] 32.6 / 33.0), and past half of it for
+// 48-row tiles ([96, 3584] 13.4 / 13.6), or rows of b that are not whole lines ([80, 3696] 16.0 / 16.5; 48 rows
+// there: 14.2 / 14.5).  56-row tiles are within 1 % either way and are not built.
+constexpr double KS_EVEN_BYTES = 64.0 * 1024 * 1024;
+
 // The rule looks at M, N and K alone: a product has the same bits under every grid cap and in
 // every batch (the policy of the loads changes none).  Up to 32 columns a second column half would be empty LDS and idle MFMAs: 256 rows x 16
 // columns 4.6 -> 4.1 us at K = 128, 13.7 -> 9.5 at 4096.
 static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
                              int max_cus, hipStream_t hs) {
-  const bool stream = M <= 64 && (double)count * N * K * 2 > KS_STREAM_BYTES;
-#define TW_KSPLIT(MT, NT, STAGES, LA)                                                                              \
-  return K % BK ? launch_ksplit<MT, NT, STAGES, LA, 0, true>(batch, count, M, N, K, ldc, max_cus, hs)              \
-         : stream ? launch_ksplit<MT, NT, STAGES, LA, KS_STREAM, false>(batch, count, M, N, K, ldc, max_cus, hs)   \
-                  : launch_ksplit<MT, NT, STAGES, LA, 0, false>(batch, count, M, N, K, ldc, max_cus, hs)
-  if (M <= 8) TW_KSPLIT(1, 1, 3, 1);
-  if (M <= 16) TW_KSPLIT(1, 1, 3, 2);
-  if (M <= 32) TW_KSPLIT(1, 1, 3, 4);
-  if (M <= 64 || N <= 32) TW_KSPLIT(2, 1, 2, 8);
-  TW_KSPLIT(2, 2, 2, 8);
+  const double b_bytes = (double)count * N * K * 2;
+  const bool whole = K % BK == 0, stream = whole && M <= 64 && b_bytes > KS_STREAM_BYTES;
+#define TW_KSPLIT(MT, NT, STAGES, LA, AUX, TAIL) \
+  return launch_ksplit<MT, NT, STAGES, LA, AUX, TAIL>(batch, count, M, N, K, ldc, max_cus, hs)
+#define TW_KSPLIT_ONE(MT, STAGES, LA)                    \
+  do {                                                   \
+    if (stream) TW_KSPLIT(MT, 1, STAGES, LA, KS_STREAM, false); \
+    if (whole) TW_KSPLIT(MT, 1, STAGES, LA, 0, false);   \
+    TW_KSPLIT(MT, 1, STAGES, LA, 0, true);               \
+  } while (0)
+  if (M <= 8) TW_KSPLIT_ONE(1, 3, 1);
+  if (M <= 16) TW_KSPLIT_ONE(1, 3, 2);
+  if (M <= 32) TW_KSPLIT_ONE(1, 3, 4);
+  if (M <= 40) TW_KSPLIT_ONE(2, 2, 5);
+  if (M <= 48 && stream) TW_KSPLIT(2, 1, 2, 6, KS_STREAM, false);
+  if (M <= 48 && whole) TW_KSPLIT(2, 1, 2, 6, 0, false);
+  if (M <= 64 || N <= 32) TW_KSPLIT_ONE(2, 2, 8);
+  if (M <= 80 && whole && b_bytes <= KS_EVEN_BYTES) TW_KSPLIT(2, 2, 2, 5, 0, false);
+  if (M <= 96 && whole && b_bytes < KS_EVEN_BYTES / 2) TW_KSPLIT(2, 2, 2, 6, 0, false);
+  if (whole) TW_KSPLIT(2, 2, 2, 8, 0, false);
+  TW_KSPLIT(2, 2, 2, 8, 0, true);
+#undef TW_KSPLIT_ONE
 #undef TW_KSPLIT
 }
 
