@@ -204,8 +204,10 @@ struct GemmBatch {
 // dimension: wave w takes the 64-wide k-slabs w, w + 4, ... .  Each wave brings its slabs of
 // both operands from global memory straight into LDS of its own, STAGES slabs deep, and
 // reads its fragments back from there: no barrier in the k loop, a wave only waits for its own
-// loads.  (Three stages up to 32 rows, 1-2 % ahead of two; four are no better: what a unit has under way is
-// bounded by its L1, not by LDS.)  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
+// loads.  (Three stages up to 32 rows, 1-2 % ahead of two, and up to 40 where rows are whole lines: [36, 768] x
+// [6144, 768]^T 4.89 -> 4.68 us, [36, 2048] 7.10 -> 6.76, [36, 3584] x [8192, 3584]^T 11.3 -> 11.2, but [36, 3696]
+// 12.6 -> 12.7 and [64, 3584] 12.6 -> 12.9; four are no better: what a unit has under way is bounded by its L1, not by
+// LDS.)  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
 // Every load covers whole 128-byte lines of eight rows.  The sum of an output element does not
 // depend on the tile it lies in (nor on MT, NT, the grid or the number of products).
 //
@@ -911,7 +913,9 @@ static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64
   if (M <= 8) TW_KSPLIT_ONE(1, 3, 1);
   if (M <= 16) TW_KSPLIT_ONE(1, 3, 2);
   if (M <= 32) TW_KSPLIT_ONE(1, 3, 4);
-  if (M <= 40) TW_KSPLIT_ONE(2, 2, 5);
+  if (M <= 40 && stream) TW_KSPLIT(2, 1, 3, 5, KS_STREAM, false);
+  if (M <= 40 && whole) TW_KSPLIT(2, 1, 3, 5, 0, false);
+  if (M <= 40) TW_KSPLIT(2, 1, 2, 5, 0, true);
   if (M <= 48 && stream) TW_KSPLIT(2, 1, 2, 6, KS_STREAM, false);
   if (M <= 48 && whole) TW_KSPLIT(2, 1, 2, 6, 0, false);
   if (M <= 64 || N <= 32) TW_KSPLIT_ONE(2, 2, 8);
