@@ -557,6 +557,22 @@ TWB_API int twb_gemm_bf16_nt_tile(void* out, const void* a, const void* b, const
   return rc ? rc : tw::finish_launch(what);
 }
 
+// How the K-split kernel would run a launch on `cus` units (host only): rows and columns of its widest tile, slabs
+// in LDS, whether b streams past the caches, LDS bytes, workgroups.  1, or 0 where no kernel is built for the form.
+TWB_API int twb_gemm_ksplit_form(int64_t M, int64_t N, int64_t K, int count, int max_cus, int cus, int64_t form[6]) {
+  const tw::KsForm f = tw::ksplit_form(M, N, K, count, max_cus, cus);
+  const tw::KsTiles tiles = tw::ksplit_tiles(M, N, 8 * f.la, 32 * f.nt, cus);
+  const int64_t groups = count * tiles.m * tiles.n;
+  const int64_t made[6] = {8 * f.la, tiles.cols, f.stages, f.stream, tw::ks_lds_bytes(f.mt, f.nt, f.stages),
+                           max_cus > 0 ? std::min<int64_t>(groups, max_cus) : groups};
+  std::copy(made, made + 6, form);
+#define TWB_FORM(MT, NT, STAGES, LA, STREAM, TAIL)                                                            \
+  if (f.mt == MT && f.nt == NT && f.stages == STAGES && f.la == LA && f.stream == STREAM && f.tail == TAIL) return 1;
+  TW_KSPLIT_FORMS(TWB_FORM)
+#undef TWB_FORM
+  return 0;
+}
+
 // Shape `index` of tw::kTiles in units of 32 rows and 32 columns; 0 past the last one.
 TWB_API int twb_gemm_tile_shape(int index, int* tm, int* tn) {
   if (index < 0 || index >= (int)(sizeof(tw::kTiles) / sizeof(tw::kTiles[0]))) return 0;

@@ -1,0 +1,49 @@
+"""Which form of a GEMM kernel a launch takes.  The rules are host code and run here without a GPU, on 256 units and
+on fewer; the forms' results are compared in the test_gpu_gemm_* files."""
+import ctypes
+
+import pytest
+
+from helpers import bench_lib
+
+LDS_OF_A_UNIT = 160 * 1024
+WIDTHS = (4, 32, 36, 256, 1028, 6144, 8192, 8452, 28672)
+
+
+@pytest.fixture(scope="module")
+def few_rows():
+    lib = bench_lib()
+    lib.twb_gemm_ksplit_form.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 3 + [ctypes.POINTER(ctypes.c_int64)]
+
+    def form(M, N, K, count=1, cap=0, cus=256):
+        f = (ctypes.c_int64 * 6)()
+        assert lib.twb_gemm_ksplit_form(M, N, K, count, cap, cus, f) == 1, (M, N, K, count, cap, cus)
+        return dict(zip(("rows", "cols", "stages", "stream", "lds", "groups"), f))
+
+    return form
+
+
+@pytest.mark.parametrize("cus", [256, 80])
+@pytest.mark.parametrize("K", [8, 64, 200, 1024, 3584, 3696, 7168])
+def test_every_launch_of_few_rows_has_a_kernel(few_rows, K, cus):
+    for M in (*range(1, 130), 1000):
+        for N in WIDTHS:
+            for count, cap in ((1, 0), (8, 0), (1, 7), (3, 160)):
+                f = few_rows(M, N, K, count, cap, cus)
+                assert f["lds"] <= LDS_OF_A_UNIT and f["cols"] % 4 == 0 and f["rows"] * -(-M // f["rows"]) >= M
+                assert not cap or f["groups"] <= cap
+
+
+@pytest.mark.parametrize("cus", [256, 80])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
+def test_units_with_several_tiles_hold_two_workgroups(few_rows, M, cus):
+    """Up to 32 rows: a third slab in LDS only where no unit has a second tile to fill its waits with."""
+    for K in (128, 1024, 3584, 3696):
+        for N in WIDTHS:
+            for count, cap in ((1, 0), (4, 0), (8, 0), (1, 16), (2, 200)):
+                f = few_rows(M, N, K, count, cap, cus)
+                tiles = count * -(-N // f["cols"])
+                if tiles > (min(cap, cus) if cap else cus):
+                    assert 2 * f["lds"] <= LDS_OF_A_UNIT, (N, K, count, cap)
+                else:
+                    assert f["stages"] == 3, (N, K, count, cap)

@@ -70,3 +70,21 @@ def test_two_row_tiles_share_the_rows_evenly(N, K):
         print(f"[case] shared rows M={M} N={N} K={K}", flush=True)
         product(poison, b)
         assert torch.equal(product(a[:M].contiguous(), b), whole[:M]), M
+
+
+@pytest.mark.parametrize("K", [8, 64, 320, 328])
+def test_more_tiles_than_units(K):
+    """Launches that give units a second tile keep one slab less in local memory.  Same bits as launches that do
+    not, also under a grid cap, where workgroups walk several tiles."""
+    N = 8452                                      # 423 tiles of 20 columns for 256 units, the last one partial
+    a, b = operands(32, N, K, K)
+    for M in (1, 8, 9, 16, 17, 32):
+        print(f"[case] more tiles than units M={M} K={K}", flush=True)
+        rows = a[:M].contiguous()
+        out = product(rows, b)
+        assert torch.equal(out[:, :4096], product(rows, b[:4096].contiguous())), M
+        assert torch.equal(out[:, 4096:], product(rows, b[4096:].contiguous())), M
+        capped = torch.full_like(out, 3.0)
+        ops.gemm_bf16_nt(capped, rows, b, max_cus=100)
+        assert torch.equal(capped, out), M
+    assert_product(out, a, b, f"K={K}")

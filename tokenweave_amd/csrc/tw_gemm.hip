@@ -204,10 +204,10 @@ struct GemmBatch {
 // dimension: wave w takes the 64-wide k-slabs w, w + 4, ... .  Each wave brings its slabs of
 // both operands from global memory straight into LDS of its own, STAGES slabs deep, and
 // reads its fragments back from there: no barrier in the k loop, a wave only waits for its own
-// loads.  (Three stages up to 32 rows, 1-2 % ahead of two, and up to 40 where rows are whole lines: [36, 768] x
-// [6144, 768]^T 4.89 -> 4.68 us, [36, 2048] 7.10 -> 6.76, [36, 3584] x [8192, 3584]^T 11.3 -> 11.2, but [36, 3696]
-// 12.6 -> 12.7 and [64, 3584] 12.6 -> 12.9; four are no better: what a unit has under way is bounded by its L1, not by
-// LDS.)  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
+// loads.  (Three stages up to 32 rows where no unit has a second tile, see ksplit_form, and up to 40 where rows are
+// whole lines: [36, 768] x [6144, 768]^T 4.89 -> 4.68 us, [36, 2048] 7.10 -> 6.76, [36, 3584] x [8192, 3584]^T
+// 11.3 -> 11.2, but [36, 3696] 12.6 -> 12.7 and [64, 3584] 12.6 -> 12.9; four are no better: what a unit has under way
+// is bounded by its L1, not by LDS.)  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
 // Every load covers whole 128-byte lines of eight rows.  The sum of an output element does not
 // depend on the tile it lies in (nor on MT, NT, the grid or the number of products).
 //
@@ -850,27 +850,29 @@ static int allow_lds(const void* kernel, std::atomic<bool>* ok, int max_devices,
 }
 constexpr int kMaxDevices = 64;
 
-template <int MT, int NT, int STAGES, int LA, int BAUX, bool TAIL>
-static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc, int max_cus,
-                         hipStream_t hs) {
-  constexpr int LDS = ks_lds_bytes(MT, NT, STAGES);
-  static std::atomic<bool> lds_ok[kMaxDevices];
-  if (int rc = allow_lds(reinterpret_cast<const void*>(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES, LA, BAUX, TAIL>), lds_ok, kMaxDevices,
-                         LDS))
-    return rc;
-  int cus = device_compute_units();
-  if (cus <= 0) cus = 256;
-  // Columns per workgroup: as few rounds of one workgroup per unit as full-width tiles need, and
-  // then tiles no wider than that many rounds require, so that every unit streams its share of b.
-  const int64_t tiles_m = (M + 8 * LA - 1) / (8 * LA), full = (N + 32 * NT - 1) / (32 * NT);
+// A K-split launch's tiles: as few rounds of one workgroup per unit as full-width tiles need, and then tiles no
+// wider than that many rounds require, so that every unit streams its share of b.
+struct KsTiles { int64_t m, n; int cols; };
+static KsTiles ksplit_tiles(int64_t M, int64_t N, int rows, int most_cols, int cus) {
+  const int64_t tiles_m = (M + rows - 1) / rows, full = (N + most_cols - 1) / most_cols;
   const int64_t rounds = (tiles_m * full + cus - 1) / cus;
   const int64_t per_row_tile = std::max(full, cus * rounds / tiles_m);  // column tiles those rounds have room for
-  const int cols = (int)std::min<int64_t>(32 * NT, ((N + per_row_tile - 1) / per_row_tile + 3) / 4 * 4);
-  const int64_t tiles_n = (N + cols - 1) / cols;
-  int64_t grid = count * tiles_m * tiles_n;
+  const int cols = (int)std::min<int64_t>(most_cols, ((N + per_row_tile - 1) / per_row_tile + 3) / 4 * 4);
+  return {tiles_m, (N + cols - 1) / cols, cols};
+}
+
+template <int MT, int NT, int STAGES, int LA, int BAUX, bool TAIL>
+static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc, int max_cus,
+                         int cus, hipStream_t hs) {
+  constexpr int LDS = ks_lds_bytes(MT, NT, STAGES);
+  static std::atomic<bool> lds_ok[kMaxDevices];
+  const auto kernel = gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES, LA, BAUX, TAIL>;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), lds_ok, kMaxDevices, LDS)) return rc;
+  const KsTiles tiles = ksplit_tiles(M, N, 8 * LA, 32 * NT, cus);
+  int64_t grid = count * tiles.m * tiles.n;
   if (max_cus > 0 && grid > max_cus) grid = max_cus;
-  launch_kernel(gemm_bf16_nt_ksplit_kernel<MT, NT, STAGES, LA, BAUX, TAIL>, dim3((unsigned)grid), dim3(KS_THREADS), LDS, hs, batch, count,
-                (int)M, (int)N, (int)K, ldc, (int)tiles_m, (int)tiles_n, cols);
+  launch_kernel(kernel, dim3((unsigned)grid), dim3(KS_THREADS), LDS, hs, batch, count, (int)M, (int)N, (int)K, ldc,
+                (int)tiles.m, (int)tiles.n, tiles.cols);
   return TW_OK;
 }
 
@@ -895,36 +897,54 @@ constexpr double KS_STREAM_BYTES = 96.0 * 1024 * 1024;
 // there: 14.2 / 14.5).  56-row tiles are within 1 % either way and are not built.
 constexpr double KS_EVEN_BYTES = 64.0 * 1024 * 1024;
 
-// The rule looks at M, N and K alone: a product has the same bits under every grid cap and in
-// every batch (the policy of the loads changes none).  Up to 32 columns a second column half would be empty LDS and idle MFMAs: 256 rows x 16
-// columns 4.6 -> 4.1 us at K = 128, 13.7 -> 9.5 at 4096.
-static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
-                             int max_cus, hipStream_t hs) {
+// The instantiations: MT, NT, STAGES, LA, stream, tail.
+#define TW_KSPLIT_ROWS_32(X, LA) \
+  X(1, 1, 2, LA, true, false) X(1, 1, 2, LA, false, false) X(1, 1, 2, LA, false, true) \
+  X(1, 1, 3, LA, true, false) X(1, 1, 3, LA, false, false) X(1, 1, 3, LA, false, true)
+#define TW_KSPLIT_FORMS(X)                                                                                   \
+  TW_KSPLIT_ROWS_32(X, 1) TW_KSPLIT_ROWS_32(X, 2) TW_KSPLIT_ROWS_32(X, 4)                                      \
+  X(2, 1, 3, 5, true, false) X(2, 1, 3, 5, false, false) X(2, 1, 2, 5, false, true)                            \
+  X(2, 1, 2, 6, true, false) X(2, 1, 2, 6, false, false)                                                       \
+  X(2, 1, 2, 8, true, false) X(2, 1, 2, 8, false, false) X(2, 1, 2, 8, false, true)                            \
+  X(2, 2, 2, 5, false, false) X(2, 2, 2, 6, false, false) X(2, 2, 2, 8, false, false) X(2, 2, 2, 8, false, true)
+struct KsForm { int mt, nt, stages, la; bool stream, tail; };
+
+// No form changes a result bit (see the kernel), so a product has the same bits under every grid cap and in every
+// batch, although both are part of the rule.  Up to 32 columns a second column half would be empty LDS and idle
+// MFMAs: 256 rows x 16 columns 4.6 -> 4.1 us at K = 128, 13.7 -> 9.5 at 4096.
+//
+// Up to 32 rows the third stage's 96 KiB leave a compute unit room for one workgroup, two stages for two.  So three
+// stages only where no unit has a second tile; us, two / three stages, cold weights: [8, 1024] x [8192, 1024]^T
+// 5.52 / 5.39, [32, 4096] x [4096, 4096]^T 10.9 / 10.4, but [32, 1024] x [16384, 1024]^T 9.0 / 10.1, x
+// [28672, 1024]^T 14.7 / 17.8, eight products [32, 1024] x [8192, 1024]^T 27.0 / 34.0, [32, 128] 10.5 / 16.4.
+static KsForm ksplit_form(int64_t M, int64_t N, int64_t K, int count, int max_cus, int cus) {
   const double b_bytes = (double)count * N * K * 2;
   const bool whole = K % BK == 0, stream = whole && M <= 64 && b_bytes > KS_STREAM_BYTES;
-#define TW_KSPLIT(MT, NT, STAGES, LA, AUX, TAIL) \
-  return launch_ksplit<MT, NT, STAGES, LA, AUX, TAIL>(batch, count, M, N, K, ldc, max_cus, hs)
-#define TW_KSPLIT_ONE(MT, STAGES, LA)                    \
-  do {                                                   \
-    if (stream) TW_KSPLIT(MT, 1, STAGES, LA, KS_STREAM, false); \
-    if (whole) TW_KSPLIT(MT, 1, STAGES, LA, 0, false);   \
-    TW_KSPLIT(MT, 1, STAGES, LA, 0, true);               \
-  } while (0)
-  if (M <= 8) TW_KSPLIT_ONE(1, 3, 1);
-  if (M <= 16) TW_KSPLIT_ONE(1, 3, 2);
-  if (M <= 32) TW_KSPLIT_ONE(1, 3, 4);
-  if (M <= 40 && stream) TW_KSPLIT(2, 1, 3, 5, KS_STREAM, false);
-  if (M <= 40 && whole) TW_KSPLIT(2, 1, 3, 5, 0, false);
-  if (M <= 40) TW_KSPLIT(2, 1, 2, 5, 0, true);
-  if (M <= 48 && stream) TW_KSPLIT(2, 1, 2, 6, KS_STREAM, false);
-  if (M <= 48 && whole) TW_KSPLIT(2, 1, 2, 6, 0, false);
-  if (M <= 64 || N <= 32) TW_KSPLIT_ONE(2, 2, 8);
-  if (M <= 80 && whole && b_bytes <= KS_EVEN_BYTES) TW_KSPLIT(2, 2, 2, 5, 0, false);
-  if (M <= 96 && whole && b_bytes < KS_EVEN_BYTES / 2) TW_KSPLIT(2, 2, 2, 6, 0, false);
-  if (whole) TW_KSPLIT(2, 2, 2, 8, 0, false);
-  TW_KSPLIT(2, 2, 2, 8, 0, true);
-#undef TW_KSPLIT_ONE
-#undef TW_KSPLIT
+  if (M <= 32) {
+    const int la = M <= 8 ? 1 : M <= 16 ? 2 : 4;
+    const KsTiles tiles = ksplit_tiles(M, N, 8 * la, 32, cus);
+    const bool one_each = count * tiles.m * tiles.n <= (max_cus > 0 ? std::min(max_cus, cus) : cus);
+    return {1, 1, one_each ? 3 : 2, la, stream, !whole};
+  }
+  if (M <= 40) return {2, 1, whole ? 3 : 2, 5, stream, !whole};
+  if (M <= 48 && whole) return {2, 1, 2, 6, stream, false};
+  if (M <= 64 || N <= 32) return {2, 1, 2, 8, stream, !whole};
+  if (M <= 80 && whole && b_bytes <= KS_EVEN_BYTES) return {2, 2, 2, 5, false, false};
+  if (M <= 96 && whole && b_bytes < KS_EVEN_BYTES / 2) return {2, 2, 2, 6, false, false};
+  return {2, 2, 2, 8, false, !whole};
+}
+
+static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
+                             int max_cus, hipStream_t hs) {
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  const KsForm f = ksplit_form(M, N, K, count, max_cus, cus);
+#define TW_KSPLIT_LAUNCH(MT, NT, STAGES, LA, STREAM, TAIL)                                                     \
+  if (f.mt == MT && f.nt == NT && f.stages == STAGES && f.la == LA && f.stream == STREAM && f.tail == TAIL)      \
+    return launch_ksplit<MT, NT, STAGES, LA, STREAM ? KS_STREAM : 0, TAIL>(batch, count, M, N, K, ldc, max_cus, cus, hs);
+  TW_KSPLIT_FORMS(TW_KSPLIT_LAUNCH)
+#undef TW_KSPLIT_LAUNCH
+  return set_error(TW_ERR_INVALID_ARGUMENT, "gemm_bf16_nt: no kernel for %d rows", (int)M);
 }
 
 template <int TM, int TN, TileRows ROWS>
