@@ -37,7 +37,8 @@ def test_every_launch_of_few_rows_has_a_kernel(few_rows, K, cus):
 @pytest.mark.parametrize("cus", [256, 80])
 @pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
 def test_units_with_several_tiles_hold_two_workgroups(few_rows, M, cus):
-    """Up to 32 rows: a third slab in LDS only where no unit has a second tile to fill its waits with."""
+    """Up to 32 rows: a third slab in LDS only where no unit has a second tile to fill its waits with, and past 16
+    rows only where rows of b are whole lines."""
     for K in (128, 1024, 3584, 3696):
         for N in WIDTHS:
             for count, cap in ((1, 0), (4, 0), (8, 0), (1, 16), (2, 200)):
@@ -46,4 +47,5 @@ def test_units_with_several_tiles_hold_two_workgroups(few_rows, M, cus):
                 if tiles > (min(cap, cus) if cap else cus):
                     assert 2 * f["lds"] <= LDS_OF_A_UNIT, (N, K, count, cap)
                 else:
-                    assert f["stages"] == 3, (N, K, count, cap)
+                    whole_lines = K % 64 == 0
+                    assert f["stages"] == (3 if whole_lines or M <= 16 else 2), (N, K, count, cap)

@@ -917,6 +917,8 @@ struct KsForm { int mt, nt, stages, la; bool stream, tail; };
 // stages only where no unit has a second tile; us, two / three stages, cold weights: [8, 1024] x [8192, 1024]^T
 // 5.52 / 5.39, [32, 4096] x [4096, 4096]^T 10.9 / 10.4, but [32, 1024] x [16384, 1024]^T 9.0 / 10.1, x
 // [28672, 1024]^T 14.7 / 17.8, eight products [32, 1024] x [8192, 1024]^T 27.0 / 34.0, [32, 128] 10.5 / 16.4.
+// Nor past 16 rows where rows of b are not whole lines, two / three stages, cold weights: [24, 2000] x [8192, 2000]^T
+// 9.8 / 10.2, [28, 2000] x [6144, 2000]^T 8.8 / 9.3, [17, 3696] x [8192, 3696]^T 14.7 / 15.2.
 static KsForm ksplit_form(int64_t M, int64_t N, int64_t K, int count, int max_cus, int cus) {
   const double b_bytes = (double)count * N * K * 2;
   const bool whole = K % BK == 0, stream = whole && M <= 64 && b_bytes > KS_STREAM_BYTES;
@@ -924,7 +926,7 @@ static KsForm ksplit_form(int64_t M, int64_t N, int64_t K, int count, int max_cu
     const int la = M <= 8 ? 1 : M <= 16 ? 2 : 4;
     const KsTiles tiles = ksplit_tiles(M, N, 8 * la, 32, cus);
     const bool one_each = count * tiles.m * tiles.n <= (max_cus > 0 ? std::min(max_cus, cus) : cus);
-    return {1, 1, one_each ? 3 : 2, la, stream, !whole};
+    return {1, 1, one_each && (whole || M <= 16) ? 3 : 2, la, stream, !whole};
   }
   if (M <= 40) return {2, 1, whole ? 3 : 2, 5, stream, !whole};
   if (M <= 48 && whole) return {2, 1, 2, 6, stream, false};
