@@ -49,3 +49,12 @@ def test_units_with_several_tiles_hold_two_workgroups(few_rows, M, cus):
                 else:
                     whole_lines = K % 64 == 0
                     assert f["stages"] == (3 if whole_lines or M <= 16 else 2), (N, K, count, cap)
+
+
+@pytest.mark.parametrize("M,rows", [(65, 40), (80, 40), (88, 48), (96, 48), (97, 64)])
+def test_even_shares_of_two_row_tiles(few_rows, M, rows):
+    """Not where a grid cap makes workgroups of long inner dimensions walk several tiles."""
+    for N, K in ((4096, 2048), (6144, 2048), (4096, 2112), (1024, 3584)):
+        for cap in (0, 16, 160, 255, 256, 1000):
+            f = few_rows(M, N, K, 1, cap)
+            assert f["rows"] == (64 if K > 2048 and 0 < cap < 256 else rows), (N, K, cap)

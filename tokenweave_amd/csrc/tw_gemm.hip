@@ -895,7 +895,13 @@ constexpr double KS_STREAM_BYTES = 96.0 * 1024 * 1024;
 // the L2s and the memory are, they lose: weights past KS_EVEN_BYTES ([80, 7168] 32.6 / 33.0), and past half of it for
 // 48-row tiles ([96, 3584] 13.4 / 13.6), or rows of b that are not whole lines ([80, 3696] 16.0 / 16.5; 48 rows
 // there: 14.2 / 14.5).  56-row tiles are within 1 % either way and are not built.
+//
+// Under a grid cap workgroups walk several tiles and the longest one counts for less: from cold weights, 64-row tiles /
+// even shares, cap 64: [72, 2048] x [8192, 2048]^T 35.5 / 34.9 us, [80, 2048] 35.9 / 36.0, but [80, 2560] 46.2 / 47.5,
+// [80, 3072] 50.1 / 51.8, [80, 2560] x [6144, 2560]^T 41.1 / 41.8; cap 160: [80, 3584] 30.5 / 31.2.  So not past
+// KS_EVEN_CAPPED_K there.
 constexpr double KS_EVEN_BYTES = 64.0 * 1024 * 1024;
+constexpr int64_t KS_EVEN_CAPPED_K = 2048;
 
 // The instantiations: MT, NT, STAGES, LA, stream, tail.
 #define TW_KSPLIT_ROWS_32(X, LA) \
@@ -931,8 +937,9 @@ static KsForm ksplit_form(int64_t M, int64_t N, int64_t K, int count, int max_cu
   if (M <= 40) return {2, 1, whole ? 3 : 2, 5, stream, !whole};
   if (M <= 48 && whole) return {2, 1, 2, 6, stream, false};
   if (M <= 64 || N <= 32) return {2, 1, 2, 8, stream, !whole};
-  if (M <= 80 && whole && b_bytes <= KS_EVEN_BYTES) return {2, 2, 2, 5, false, false};
-  if (M <= 96 && whole && b_bytes < KS_EVEN_BYTES / 2) return {2, 2, 2, 6, false, false};
+  const bool even = whole && (K <= KS_EVEN_CAPPED_K || max_cus <= 0 || max_cus >= cus);
+  if (M <= 80 && even && b_bytes <= KS_EVEN_BYTES) return {2, 2, 2, 5, false, false};
+  if (M <= 96 && even && b_bytes < KS_EVEN_BYTES / 2) return {2, 2, 2, 6, false, false};
   return {2, 2, 2, 8, false, !whole};
 }
 
