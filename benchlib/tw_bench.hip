@@ -573,6 +573,23 @@ TWB_API int twb_gemm_ksplit_form(int64_t M, int64_t N, int64_t K, int count, int
   return 0;
 }
 
+// How the tile kernel's (32 tm) x (32 tn) shape fetches rows of K elements (host only): 0 whole slabs, 1 a partial last
+// slab, 2 whole lines; -1 where there is no such shape.
+TWB_API int twb_gemm_tile_rows(int tm, int tn, int64_t K) {
+#define TWB_ROWS(TM, TN, COST) \
+  if (tm == TM && tn == TN) return tw::tile_rows<TM, TN>(K);
+  TW_TILES(TWB_ROWS)
+#undef TWB_ROWS
+  return -1;
+}
+
+// The shape that tw::pick_tile takes for `cus` units (host only).
+TWB_API void twb_gemm_pick_tile(int64_t M, int64_t N, int count, int cus, int* tm, int* tn) {
+  const tw::TileChoice& t = tw::pick_tile(M, N, count, cus);
+  *tm = t.tm;
+  *tn = t.tn;
+}
+
 // Shape `index` of tw::kTiles in units of 32 rows and 32 columns; 0 past the last one.
 TWB_API int twb_gemm_tile_shape(int index, int* tm, int* tn) {
   if (index < 0 || index >= (int)(sizeof(tw::kTiles) / sizeof(tw::kTiles[0]))) return 0;

@@ -7,6 +7,7 @@ import pytest
 from helpers import bench_lib
 
 LDS_OF_A_UNIT = 160 * 1024
+TILES = ((8, 8), (6, 8), (8, 6), (5, 8), (6, 6), (4, 8), (3, 8), (4, 6), (3, 6), (4, 4), (3, 4), (2, 4))
 WIDTHS = (4, 32, 36, 256, 1028, 6144, 8192, 8452, 28672)
 
 
@@ -58,3 +59,15 @@ def test_even_shares_of_two_row_tiles(few_rows, M, rows):
         for cap in (0, 16, 160, 255, 256, 1000):
             f = few_rows(M, N, K, 1, cap)
             assert f["rows"] == (64 if K > 2048 and 0 < cap < 256 else rows), (N, K, cap)
+
+
+@pytest.mark.parametrize("K", [16, 80, 208, 336, 528, 544, 784, 1040, 1056, 1264, 1312, 1952, 2016, 72, 328, 1000, 7384])
+def test_short_rows_are_fetched_by_slabs(K):
+    """Whole lines cost a tile more than they give there; rows that are no multiple of 16 never take them."""
+    assert [bench_lib().twb_gemm_tile_rows(*s, ctypes.c_int64(K)) for s in TILES] == [1] * len(TILES)
+
+
+@pytest.mark.parametrize("K,lines", [(1296, 7), (3696, 7), (2080, 5), (7392, 5), (64, 0), (1024, 0), (3584, 0)])
+def test_long_rows_are_fetched_by_lines_where_the_ring_has_room(K, lines):
+    kinds = [bench_lib().twb_gemm_tile_rows(*s, ctypes.c_int64(K)) for s in TILES]
+    assert kinds.count(2) == lines and kinds.count(0 if K % 64 == 0 else 1) == len(TILES) - lines

@@ -1,9 +1,12 @@
-"""The tile GEMM kernel where it fetches whole lines of rows that are not whole lines (K a multiple of 16, not of
-64): every shape with room for it, one slab to more than the ring holds, several tiles per workgroup, operands
-that begin anywhere in a line with NaN on both sides of them, and products of a batch that begin differently.
+"""The tile GEMM kernel where rows are not whole lines (K a multiple of 16, not of 64): every shape with room for
+fetching whole lines of them, from the K on where it does so and below, where it fetches slabs, several tiles per
+workgroup, operands that begin anywhere in a line with NaN on both sides of them, and products of a batch that begin
+differently.
 
 Zeros behind the last element of every row make the same product one of whole slabs, whose loads are others but
 whose sums are the same: no bit may differ.  That product is held against float64 as in test_gpu_gemm_ksplit.py."""
+import ctypes
+
 import pytest
 import torch
 
@@ -13,6 +16,7 @@ from tokenweave_amd import _custom_ops as ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+LEAST_RING = ((4, 8), (3, 8))   # lines only where most rows lie on two of them
 SHAPES = ((4, 8), (3, 8), (4, 6), (3, 6), (4, 4), (3, 4), (2, 4))
 
 
@@ -23,14 +27,20 @@ def placed(rows, K, offset, g):
     return t.copy_(torch.randn(rows, K, generator=g, device=DEV))
 
 
+def takes_lines(lib, tm, tn, K):
+    return lib.twb_gemm_tile_rows(tm, tn, ctypes.c_int64(K)) == 2
+
+
 def padded(t):
     return torch.nn.functional.pad(t, (0, -t.shape[1] % 64)).contiguous()
 
 
-@pytest.mark.parametrize("K", [16, 48, 80, 112, 208, 336, 1072])
+# From 1296 on whole lines: rows begin 2, 6 and 4 chunks of 16 bytes after one another in their lines.
+@pytest.mark.parametrize("K", [16, 48, 80, 112, 208, 336, 1072, 1296, 1328, 2080, 2144])
 @pytest.mark.parametrize("tm,tn", SHAPES)
 def test_every_shape(forced, tm, tn, K):  # noqa: F811
     M, N = 2 * 32 * tm + 17, 2 * 32 * tn + 24         # nine tiles, the last row and column of them partial
+    assert takes_lines(forced.lib, tm, tn, K) == (K > 1280 and (K % 32 == 16 or (tm, tn) not in LEAST_RING))
     g = torch.Generator(device=DEV).manual_seed(100 * tm + 10 * tn + K)
     for at_a, at_b in ((0, 0), (8, 48), (32, 56)):
         a, b = placed(M, K, at_a, g), placed(N, K, at_b, g)

@@ -978,18 +978,36 @@ static int launch_tile_kernel(const GemmBatch& batch, int count, int64_t M, int6
   return TW_OK;
 }
 
+// Whole lines where the shape's ring has room for the panel more and rows are long: a tile costs 0.8 to 1 us more
+// (one line more to fetch and every row's place in its lines).  us, kPartialSlab / kLines, 8192 columns, weights from
+// memory: [200, 208] 6.1 / 6.9, [200, 528] 8.6 / 8.6, [200, 1040] 12.8 / 11.6, [200, 1552] 17.3 / 14.7; K a multiple of 32,
+// where half as many rows lie on two lines: [200, 544] 8.2 / 8.7, [200, 1056] 11.9 / 11.6, [200, 2080] 19.6 / 17.7.
+// The same weights again and again, from the last-level cache, gain later, and the lines are drawn between the two:
+// [200, 1040] 10.7 / 10.8, [200, 1552] 13.7 / 13.3, [200, 2080] 15.5 / 15.9, [200, 4128] 28.0 / 26.5.  (What the L2s
+// hold is not bound by requests: [129, 2064] x [1024, 2064]^T 11.5 / 14.9; from memory 19.9 / 16.7.)
+constexpr int64_t LINES_FROM_K = 1280, LINES_FROM_K_32 = 2048;
+
+// The shapes whose ring then is down to the least (TIGHT: 128 x 256 and 96 x 256) cover less of memory's latency and are
+// taken only where more than half of the rows lie on two lines: K = 7392, 128 x 256, 800 and 1000 rows 122 / 138 us with
+// kPartialSlab, 132 / 133 with kLines.
+template <int TM, int TN>
+static TileRows tile_rows(int64_t K) {
+  if (K % BK == 0) return kWholeSlabs;
+  if constexpr (TileShape<TM, TN>::TAKES_LINES) {
+    if (K % 32 == 16 && K >= LINES_FROM_K) return kLines;
+    if (K % 32 == 0 && K >= LINES_FROM_K_32 && !TileShape<TM, TN, kLines>::TIGHT) return kLines;
+  }
+  return kPartialSlab;
+}
+
 template <int TM, int TN>
 static int launch_tile(const GemmBatch& batch, int count, int64_t M, int64_t N, int64_t K, int64_t ldc,
                        int max_cus, hipStream_t hs) {
-  // Whole lines where the shape's ring has room for the panel more.  The shapes whose ring then is down to the
-  // least (TIGHT: 128 x 256 and 96 x 256) cover less of memory's latency and are taken only where more than half of
-  // the rows lie on two lines: K = 7392, 128 x 256, 800 and 1000 rows 122 / 138 us with kPartialSlab, 132 / 133 with kLines.
-  if constexpr (TileShape<TM, TN>::TAKES_LINES) {
-    if (K % BK && K % 16 == 0 && (!TileShape<TM, TN, kLines>::TIGHT || K % 32))
-      return launch_tile_kernel<TM, TN, kLines>(batch, count, M, N, K, ldc, max_cus, hs);
-  }
-  return K % BK ? launch_tile_kernel<TM, TN, kPartialSlab>(batch, count, M, N, K, ldc, max_cus, hs)
-                : launch_tile_kernel<TM, TN, kWholeSlabs>(batch, count, M, N, K, ldc, max_cus, hs);
+  const TileRows rows = tile_rows<TM, TN>(K);
+  if (rows == kWholeSlabs) return launch_tile_kernel<TM, TN, kWholeSlabs>(batch, count, M, N, K, ldc, max_cus, hs);
+  if constexpr (TileShape<TM, TN>::TAKES_LINES)
+    if (rows == kLines) return launch_tile_kernel<TM, TN, kLines>(batch, count, M, N, K, ldc, max_cus, hs);
+  return launch_tile_kernel<TM, TN, kPartialSlab>(batch, count, M, N, K, ldc, max_cus, hs);
 }
 
 // The tile shapes, in 32-row and 32-column units, with the time a round of them takes on all
