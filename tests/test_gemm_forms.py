@@ -71,3 +71,10 @@ def test_short_rows_are_fetched_by_slabs(K):
 def test_long_rows_are_fetched_by_lines_where_the_ring_has_room(K, lines):
     kinds = [bench_lib().twb_gemm_tile_rows(*s, ctypes.c_int64(K)) for s in TILES]
     assert kinds.count(2) == lines and kinds.count(0 if K % 64 == 0 else 1) == len(TILES) - lines
+
+
+@pytest.mark.parametrize("M,most_mib", [(65, 64), (72, 64), (73, 56), (80, 56), (81, 31), (96, 31)])
+def test_large_weights_keep_tiles_of_64_rows(few_rows, M, most_mib):
+    for mib in (8, 16, 31, 33, 40, 56, 57, 64, 65, 112):
+        f = few_rows(M, 8192, 64 * mib)           # 8192 columns: a MiB per 64 of K
+        assert (f["rows"] < 64) == (mib <= most_mib), mib

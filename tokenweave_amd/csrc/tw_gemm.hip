@@ -892,7 +892,8 @@ constexpr double KS_STREAM_BYTES = 96.0 * 1024 * 1024;
 // [40, 1024] x [8192, 1024]^T 5.77 / 5.52, [40, 3584] 11.67 / 11.37, [40, 3696] 13.50 / 12.91, [33, 7168] 23.9 / 22.9,
 // [48, 2048] x [6144, 2048]^T 7.41 / 7.18; [72, 768] x [6144, 768]^T 6.03 / 5.59, [72, 1024] x [8192, 1024]^T 7.05 / 6.64,
 // [72, 3584] 13.53 / 12.52, [96, 1024] 7.14 / 6.93.  Even shares gain while the longest workgroup is the bound; where
-// the L2s and the memory are, they lose: weights past KS_EVEN_BYTES ([80, 7168] 32.6 / 33.0), and past half of it for
+// the L2s and the memory are, they lose: weights past KS_EVEN_BYTES ([80, 7168] 32.6 / 33.0, [72, 5120] 24.5 / 25.3),
+// past 7/8 of it from 73 rows on ([80, 4096] 19.9 / 20.3, weights from memory; [72, 4096] 19.7 / 19.5), past half of it for
 // 48-row tiles ([96, 3584] 13.4 / 13.6), or rows of b that are not whole lines ([80, 3696] 16.0 / 16.5; 48 rows
 // there: 14.2 / 14.5).  56-row tiles are within 1 % either way and are not built.
 //
@@ -938,7 +939,7 @@ static KsForm ksplit_form(int64_t M, int64_t N, int64_t K, int count, int max_cu
   if (M <= 48 && whole) return {2, 1, 2, 6, stream, false};
   if (M <= 64 || N <= 32) return {2, 1, 2, 8, stream, !whole};
   const bool even = whole && (K <= KS_EVEN_CAPPED_K || max_cus <= 0 || max_cus >= cus);
-  if (M <= 80 && even && b_bytes <= KS_EVEN_BYTES) return {2, 2, 2, 5, false, false};
+  if (M <= 80 && even && b_bytes <= KS_EVEN_BYTES * (M <= 72 ? 1.0 : 0.875)) return {2, 2, 2, 5, false, false};
   if (M <= 96 && even && b_bytes < KS_EVEN_BYTES / 2) return {2, 2, 2, 6, false, false};
   return {2, 2, 2, 8, false, !whole};
 }
