@@ -38,7 +38,7 @@ def test_rows_that_are_not_fetched_reach_no_result(N, K):
         assert torch.equal(product(a[:M].contiguous(), b), whole[:M]), M
 
 
-@pytest.mark.parametrize("M", [8, 16, 17, 64, 65])
+@pytest.mark.parametrize("M", [8, 16, 17, 33, 40, 41, 48, 64, 65])
 def test_large_weights(M):
     N, K = 6208, 8128                             # 100.9 MB: the streaming form up to 64 rows
     a, b = operands(M, N, K, M)
@@ -58,9 +58,20 @@ def test_a_batch_whose_weights_are_large_together():
     assert_product(outs[P - 1], *made[P - 1], "last product")
 
 
+@pytest.mark.parametrize("M", [65, 72, 80, 88, 96])
+def test_a_batch_of_64_row_tiles_has_the_bits_of_products_that_share_rows(M):
+    P, N, K = 4, 8192, 1088                       # 71 MB together: tiles of 64 rows; each one alone of 40 or 48
+    made = [operands(M, N, K, 70 + p) for p in range(P)]
+    outs = [torch.full((M, N), 3.0, dtype=torch.bfloat16, device=DEV) for _ in range(P)]
+    ops.gemm_bf16_nt_partials(outs, [m[0] for m in made], [m[1] for m in made])
+    for p, (a, b) in enumerate(made):
+        assert torch.equal(outs[p], product(a, b)), p
+    assert_product(outs[0][:, :512], made[0][0], made[0][1][:512], f"M={M}")
+
+
 @pytest.mark.parametrize("N,K", [(8192, 320), (1028, 840), (36, 264), (6144, 64)])
 def test_two_row_tiles_share_the_rows_evenly(N, K):
-    """Row m is the same in every batch of 33 to 128 rows, whose tiles are of 40, 48, 56 or 64 rows, also
+    """Row m is the same in every batch of 33 to 128 rows, whose tiles are of 40, 48 or 64 rows, also
     behind a product that has left NaN in the local memory of the compute units."""
     a, b = operands(128, N, K, N + K + 1)
     poison = torch.full((128, K), float("nan"), dtype=torch.bfloat16, device=DEV)

@@ -56,9 +56,33 @@ def test_every_shape(forced, tm, tn, K):  # noqa: F811
             assert torch.equal(out, want), (at_a, at_b, cus)
 
 
-@pytest.mark.parametrize("cap", [None, 5])
-def test_a_batch_whose_products_begin_differently(cap):
-    P, M, N, K = 4, 150, 392, 176
+@pytest.mark.parametrize("K", [1296, 2080])
+@pytest.mark.parametrize("tm,tn", SHAPES)
+def test_bias_and_both_stores(forced, tm, tn, K):  # noqa: F811
+    """The stores of a tile, 8 or 16 bytes wide, and its bias lie between the loads that the next tile waits for."""
+    M, N = 2 * 32 * tm + 17, 2 * 32 * tn + 24
+    g = torch.Generator(device=DEV).manual_seed(tm + 10 * tn + K)
+    a, b, bias = placed(M, K, 24, g), placed(N, K, 40, g), torch.randn(N, generator=g, device=DEV).to(torch.bfloat16)
+    want = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+    forced(want, padded(a), padded(b), None, tm, tn, 0)
+    for ld, cus, with_bias in ((N + 8, 1, False), (N + 4, 1, False), (N + 8, 4, True), (N + 4, 4, True), (N + 4, 1, True)):
+        print(f"[case] lines {32 * tm}x{32 * tn} K={K} ld={ld} cus={cus} bias={with_bias}", flush=True)
+        wide = torch.full((M + 2, ld), 7.0, dtype=torch.bfloat16, device=DEV)     # ld % 8: 16- or 8-byte stores
+        forced(wide[1:M + 1, :N], a, b, bias if with_bias else None, tm, tn, cus)
+        torch.cuda.synchronize()
+        assert torch.equal(wide[1:M + 1, :N], want + bias if with_bias else want), (ld, cus, with_bias)
+        assert bool((wide[0] == 7).all() and (wide[-1] == 7).all() and (wide[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("P,M,N,K,cap,tile", [(4, 150, 392, 176, None, None), (4, 150, 392, 176, 5, None),
+                                              (4, 150, 520, 1296, 8, (3, 6)), (3, 330, 520, 2080, 4, (4, 6))])
+def test_a_batch_whose_products_begin_differently(forced, P, M, N, K, cap, tile):  # noqa: F811
+    """With a tile: workgroups walk from one product to the next, whose rows begin elsewhere in their lines."""
+    if tile:
+        tm, tn = ctypes.c_int(), ctypes.c_int()
+        forced.lib.twb_gemm_pick_tile(ctypes.c_int64(M), ctypes.c_int64(N), P, cap, ctypes.byref(tm), ctypes.byref(tn))
+        tiles = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1]))
+        assert (tm.value, tn.value) == tile and takes_lines(forced.lib, *tile, K) and P * tiles >= 3 * cap
     g = torch.Generator(device=DEV).manual_seed(7)
     a = [placed(M, K, 16 * p, g) for p in range(P)]
     b = [placed(N, K, 8 * p + 8, g) for p in range(P)]
@@ -68,3 +92,15 @@ def test_a_batch_whose_products_begin_differently(cap):
         want = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
         ops.gemm_bf16_nt(want, padded(a[p]), padded(b[p]))
         assert torch.equal(outs[p], want), p
+    assert_product(outs[P - 1], a[P - 1], b[P - 1], "last product")
+
+
+@pytest.mark.parametrize("M,K", [(200, 7392), (640, 3696)])
+def test_long_rows_through_the_library(M, K):
+    N, g = 8192, torch.Generator(device=DEV).manual_seed(K)
+    a, b = placed(M, K, 16, g), placed(N, K, 8, g)
+    out, want = (torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.gemm_bf16_nt(out, a, b)
+    ops.gemm_bf16_nt(want, padded(a), padded(b))
+    assert torch.equal(out, want)
+    assert_product(out[:, -320:], a, b[-320:], f"M={M} K={K}")
