@@ -561,7 +561,7 @@ TWB_API int twb_gemm_bf16_nt_tile(void* out, const void* a, const void* b, const
 // in LDS, whether b streams past the caches, LDS bytes, workgroups.  1, or 0 where no kernel is built for the form.
 TWB_API int twb_gemm_ksplit_form(int64_t M, int64_t N, int64_t K, int count, int max_cus, int cus, int64_t form[6]) {
   const tw::KsForm f = tw::ksplit_form(M, N, K, count, max_cus, cus);
-  const tw::KsTiles tiles = tw::ksplit_tiles(M, N, 8 * f.la, 32 * f.nt, cus);
+  const tw::KsTiles tiles = tw::ksplit_tiles(M, N, count, 8 * f.la, 32 * f.nt, cus);
   const int64_t groups = count * tiles.m * tiles.n;
   const int64_t made[6] = {8 * f.la, tiles.cols, f.stages, f.stream, tw::ks_lds_bytes(f.mt, f.nt, f.stages),
                            max_cus > 0 ? std::min<int64_t>(groups, max_cus) : groups};

@@ -78,3 +78,14 @@ def test_large_weights_keep_tiles_of_64_rows(few_rows, M, most_mib):
     for mib in (8, 16, 31, 33, 40, 56, 57, 64, 65, 112):
         f = few_rows(M, 8192, 64 * mib)           # 8192 columns: a MiB per 64 of K
         assert (f["rows"] < 64) == (mib <= most_mib), mib
+
+
+@pytest.mark.parametrize("M", [8, 32, 64, 96, 128])
+def test_tiles_of_a_batch_are_no_narrower_than_its_rounds_need(few_rows, M):
+    for N in (264, 1024, 2048, 4096, 6144, 8192):
+        for count in (1, 2, 3, 8, 16):
+            f = few_rows(M, N, 1024, count)
+            row_tiles, widest = count * -(-M // f["rows"]), 64 if M > 64 else 32
+            full_width = row_tiles * -(-N // widest)
+            rounds = -(-full_width // 256)
+            assert f["groups"] <= max(full_width, 256 * rounds), (N, count)
