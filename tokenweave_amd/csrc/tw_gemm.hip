@@ -9,9 +9,9 @@
 // operand, which leaves every lane with 4 consecutive n per accumulator quad.
 //
 // Three kernels:
-//  * gemm_bf16_nt_ksplit_kernel<MT, NT> (at most 128 rows): (32 MT) x (32 NT) tiles whose four
-//    waves share the inner dimension;
-//  * gemm_bf16_nt_tile_kernel<TM, TN> (more rows): (32 TM) x (32 TN) tiles, 64 x 128 to 256 x 256,
+//  * gemm_bf16_nt_ksplit_kernel (at most 128 rows): tiles of 8 to 64 rows and at most 32 or 64 columns
+//    whose four waves share the inner dimension;
+//  * gemm_bf16_nt_tile_kernel<TM, TN, ROWS> (more rows): (32 TM) x (32 TN) tiles, 64 x 128 to 256 x 256,
 //    picked per problem so that the tile count wastes the fewest workgroup rounds;
 //  * gemm_bf16_nt_kernel (K > 2^24, where a tile's rows outgrow 32-bit offsets): 128 x 128 x 64
 //    tiles, 4 waves, register-staged loads into padded LDS, 64-bit addresses.
@@ -200,21 +200,20 @@ struct GemmBatch {
 // K-split kernel: few rows (a decode step, a short prefill chunk).  The product is bound by
 // reading b once, so what counts is how many compute units stream it and how evenly.
 //
-// A workgroup owns (32 MT) x (at most 32 NT) of the output and its four waves share the inner
-// dimension: wave w takes the 64-wide k-slabs w, w + 4, ... .  Each wave brings its slabs of
-// both operands from global memory straight into LDS of its own, STAGES slabs deep, and
-// reads its fragments back from there: no barrier in the k loop, a wave only waits for its own
-// loads.  (Three stages up to 32 rows where no unit has a second tile, see ksplit_form, and up to 40 where rows are
-// whole lines: [36, 768] x [6144, 768]^T 4.89 -> 4.68 us, [36, 2048] 7.10 -> 6.76, [36, 3584] x [8192, 3584]^T
-// 11.3 -> 11.2, but [36, 3696] 12.6 -> 12.7 and [64, 3584] 12.6 -> 12.9; four are no better: what a unit has under way
-// is bounded by its L1, not by LDS.)  The four partial tiles meet in LDS at the end and are added as ((w0+w1)+w2)+w3.
-// Every load covers whole 128-byte lines of eight rows.  The sum of an output element does not
-// depend on the tile it lies in (nor on MT, NT, the grid or the number of products).
+// A workgroup owns 8 LA rows (in MT blocks of 32) x at most 32 NT columns of the output and its four waves share the
+// inner dimension: wave w takes the 64-wide k-slabs w, w + 4, ... .  Each wave brings its slabs of both operands from
+// global memory straight into LDS of its own, STAGES slabs deep, and reads its fragments back from there: no barrier
+// in the k loop, a wave only waits for its own loads.  (Three stages up to 32 rows where no unit has a second tile,
+// see ksplit_form, and up to 40 where rows are whole lines: [36, 768] x [6144, 768]^T 4.89 -> 4.68 us, [36, 2048]
+// 7.10 -> 6.76, [36, 3584] x [8192, 3584]^T 11.3 -> 11.2, but [36, 3696] 12.6 -> 12.7 and [64, 3584] 12.6 -> 12.9;
+// four are no better: what a unit has under way is bounded by its L1, not by LDS.)  The four partial tiles meet in
+// LDS at the end and are added as ((w0+w1)+w2)+w3. Every load covers whole 128-byte lines of eight rows.  The sum of
+// an output element does not depend on the tile it lies in (nor on MT, NT, the grid or the number of products).
 //
 // The launcher makes the tiles just wide enough for one (or a whole number of) workgroups per
 // compute unit: 32 columns at N = 8192, 24 at N = 6144.  Measured on 256 units, operands
-// rotated through 0.5 GB / through three sets: [32, 3584] x [8192, 3584]^T 14.1 / 10.7 us
-// (59 MB: 4.2 / 5.6 TB/s) against 65 / 47 us with 64 workgroups of 128 x 128; K = 1024: 5.2 us
+// rotated through 1.25 GB / through three sets: [32, 3584] x [8192, 3584]^T 13.6 / 11.2 us
+// (59 MB: 4.4 / 5.3 TB/s) against 65 / 47 us with 64 workgroups of 128 x 128; K = 1024: 5.2 us
 // against 16 us; [128, 3584]: 21 / 15 us against 69 / 50 us.
 //
 // What is short is also bound by the way to the first load: with rows past 16 or 8 not fetched, the partial
@@ -429,7 +428,8 @@ __global__ __launch_bounds__(KS_THREADS) void gemm_bf16_nt_ksplit_kernel(
 //  * The slab sequence runs on across tiles: a workgroup keeps its compute unit and walks the tile
 //    list with stride gridDim.x, the first D slabs of the next tile are under way while the
 //    accumulators of the last one are stored, and its first barrier does not wait for those stores
-//    (vmcnt counts in order: they are younger than the loads it needs).
+//    (vmcnt counts in order: they are younger than the loads it needs).  Where whole lines are fetched, the slab
+//    without products between two tiles does not wait for them, the next tile's first slab does.
 //  * Results leave by 16-byte stores from the registers.  The columns a lane holds are made
 //    adjacent by the row order in which b's fragments are read: MFMA row r of the tile pair
 //    (2 p, 2 p + 1) is column 32 p + 8 (r / 4) + 4 (tile & 1) + r % 4 of the wave's columns.  They are
@@ -472,7 +472,8 @@ struct TileShape {
   static constexpr bool TIGHT = LINES ? STAGES < 4 : STAGES == 2;
   static constexpr int NEED = LINES ? 2 : 1;  // slabs behind the one in use that its barrier waits for
   // slabs ahead; three at most: with four or five the 64- to 128-row tiles take longer to start than they
-  // gain ([256, 1024] x [8192, 1024]^T 8.3 -> 8.8 us, [160, 3584] x [8192, 3584]^T 18.2 -> 18.8)
+  // gain ([256, 1024] x [8192, 1024]^T 8.3 -> 8.8 us, [160, 3584] x [8192, 3584]^T 18.2 -> 18.8).  Rows of
+  // whole lines end in the line behind their slab: one more there.
   static constexpr int D = LINES ? (STAGES < 5 ? 3 : 4) : TIGHT ? 2 : (STAGES - 1 < 3 ? STAGES - 1 : 3);
   static constexpr int SA = D + 1, SB = TIGHT ? D : D + 1;
   static constexpr int LDS = SA * PA + SB * PB;
@@ -601,7 +602,9 @@ struct TilePlace {
 };
 
 // Where in its 128-byte line a row begins, in 16-byte chunks.
-__device__ __forceinline__ int line_phase(const uint16_t* row) { return (int)(reinterpret_cast<uintptr_t>(row) >> 4) & 7; }
+__device__ __forceinline__ int line_phase(const uint16_t* row) {
+  return (int)(reinterpret_cast<uintptr_t>(row) >> 4) & 7;
+}
 
 template <int TM, int TN>
 __device__ __forceinline__ TilePlace tile_place(int t, int num_tiles, int tiles_m, int tiles_n) {
@@ -627,15 +630,17 @@ __device__ __forceinline__ TilePlace tile_place(int t, int num_tiles, int tiles_
 // fragments instead needs no moves and is no faster, 227 against 230 us for 16384 x 8192 x 1000.)
 //
 // kLines: rows of such a K are not whole lines, and a slab of a row mostly lies on two of them, which a compute
-// unit then requests twice: its L1 has about 126 requests under way whatever the kernel does, so it is the
-// number of requests that bounds such a product ([1000, 3696] x [8192, 3696]^T: 9.9 million requests of 357 cycles
-// in 108 thousand cycles of every L1, 1.73 a slab row).  Here a load fetches the lines themselves, one a row and
-// slab, and a fragment read finds the first part of its slab in the ring's panel of that slab and the rest
+// unit then requests twice ([1000, 3696] x [8192, 3696]^T: 9.9 million requests, 1.73 a slab row; its L1 has about 126
+// under way whatever the kernel does).  Here a load fetches the lines themselves, one a row and slab (5.7 million
+// requests, 1.01), and a fragment read finds the first part of its slab in the ring's panel of that slab and the rest
 // in the next one.  That wants one panel more in the ring, and K % 16 == 0: rows two apart then begin at the
 // same place of a line or half a line apart, which the swizzle takes care of.  Aligned 64 bytes have to stay with
 // groups of four lanes: rotated by other amounts the loads take half of the gain back.  Same bits.
-// One product with 8192 columns, K = 3696, kPartialSlab -> kLines, operands rotated through three sets: 200 rows 25.8 ->
-// 23.2 us, 256: 27.1 -> 23.6, 512: 37.5 -> 32.6, 1000: 54.8 -> 50.8; K = 7392: 200 rows 63 -> 49, 256: 72 -> 56, 400: 79 -> 70.
+// Requests that miss the L2s gain most.  One product with 8192 columns, kPartialSlab -> kLines, weights from memory /
+// three sets in turn, us: K = 3696, 200 rows 36.3 -> 27.4 / 26.2 -> 23.8, 256: 41.3 -> 30.8 / 27.5 -> 24.1, 512: 47.4
+// -> 40.4 / 37.0 -> 33.5, 640: 69.4 -> 49.7 / 48.9 -> 41.4, 800: 71.5 -> 70.7 / 49.7 -> 50.6, 1000: 77.0 -> 71.1 /
+// 55.0 -> 51.8; K = 7392 (both from memory), 200 rows 61 -> 50, 256: 72 -> 57, 512: 85 -> 77, 640: 122 -> 96.  On one
+// set again and again the units are busy 4 % fewer cycles at 1000 rows and 3 to 7 % more at 200.
 template <int TM, int TN, TileRows ROWS>
 __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THREADS) void gemm_bf16_nt_tile_kernel(
     GemmBatch batch, int count, int M, int N, int K, int64_t ldc, int tiles_m, int tiles_n, int wide_store) {
@@ -705,10 +710,10 @@ __global__ __attribute__((amdgpu_waves_per_eu(1, 1))) __launch_bounds__(TILE_THR
     const TilePlace p = tile_place<TM, TN>(in ? lt : 0, num_tiles, tiles_m, tiles_n);                        \
     const uint16_t *pa = batch.a[p.product] + (size_t)p.m0 * K, *pb = batch.b[p.product] + (size_t)p.n0 * K; \
     if (S::LINES) load_phase_a = line_phase(pa), load_phase_b = line_phase(pb);                              \
-    da = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pa) - (int)AHEAD / 2, 0,                         \
+    da = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pa) - (int)AHEAD / 2, 0,                    \
                                            in ? (uint32_t)min(M - p.m0, S::BM) * (uint32_t)K * 2u + AHEAD : 0u, \
                                            0x00020000);                                                      \
-    db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pb) - (int)AHEAD / 2, 0,                         \
+    db = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(pb) - (int)AHEAD / 2, 0,                    \
                                            in ? (uint32_t)min(N - p.n0, S::BN) * (uint32_t)K * 2u + AHEAD : 0u, \
                                            0x00020000);                                                      \
   } while (0)
@@ -851,10 +856,10 @@ static int allow_lds(const void* kernel, std::atomic<bool>* ok, int max_devices,
 constexpr int kMaxDevices = 64;
 
 // A K-split launch's tiles: as few rounds of one workgroup per unit as full-width tiles need, and then tiles no
-// wider than that many rounds require, so that every unit streams its share of b.  The rounds are the whole batch's: with
-// those of one product alone its tiles were up to `count` times too narrow, us: two products [32, 1024] x [2048, 1024]^T
-// 6.2 -> 5.0, eight 19.2 -> 9.2, eight [32, 1024] x [6144, 1024]^T 26.2 -> 23.1, four [64, 1024] x [4096, 1024]^T 20.1 -> 12.9
-// (weights from memory).
+// wider than that many rounds require, so that every unit streams its share of b.  The rounds are the whole batch's:
+// with those of one product alone its tiles were up to `count` times too narrow, us: two products [32, 1024] x [2048,
+// 1024]^T 6.2 -> 5.0, eight 19.2 -> 9.2, eight [32, 1024] x [6144, 1024]^T 26.2 -> 23.1, four [64, 1024] x [4096,
+// 1024]^T 20.1 -> 12.9 (weights from memory).
 struct KsTiles { int64_t m, n; int cols; };
 static KsTiles ksplit_tiles(int64_t M, int64_t N, int count, int rows, int most_cols, int cus) {
   const int64_t tiles_m = (M + rows - 1) / rows, full = (N + most_cols - 1) / most_cols;
@@ -880,12 +885,18 @@ static int launch_ksplit(const GemmBatch& batch, int count, int64_t M, int64_t N
 }
 
 // b's loads carry the non-temporal bit (KS_STREAM) where a launch's weights are so large that the last-level
-// cache (256 MB) does not keep three of them: from memory b arrives 8-12 % faster that way, but past that cache
-// too.  [M, 7168] x [8192, 7168]^T (117 MB), three or four in turn: 8 rows 21.4 -> 18.9 us, 32: 24.6 -> 22.5, 64:
-// 31.1 -> 28.8; not beyond (128 rows: 37.4 / 37.6, the unit's outstanding lines are shared with a).  Four products
-// [20, 2048] (134 MB) 33.9 -> 28.8.  Below the line, from the cache: [32, 4160] (68 MB) 12.1 -> 14.2, eight products
-// [8, 768] x [6144, 768]^T (75 MB) 20.9 -> 22.0.  Not where rows of b are not whole lines: the line that two slabs
-// share would be fetched twice (8 rows, K = 3696: 11.1 -> 13.4).
+// cache (256 MB) does not keep three of them.  Not beyond 64 rows (128 rows: 37.4 / 37.6, the unit's outstanding lines
+// are shared with a), and not where rows of b are not whole lines: the line that two slabs share would be fetched twice
+// (8 rows, K = 3696: 11.1 -> 13.4).
+// From memory b arrives faster that way at every size, and past the caches too.  us, default / streaming, N = 8192:
+//                    weights from memory                       three sets in turn            one set again and again
+//   K = 1024 (17 MB)  8 rows 5.43 / 5.11, 32: 5.96 / 5.64    5.22 / 4.65, 5.56 / 5.23      3.59 / 3.60, 3.94 / 3.95
+//   K = 2048 (34 MB)  8      8.69 / 7.71, 32: 9.37 / 8.66    7.50 / 7.25, 7.85 / 8.34      4.84 / 5.22, 6.23 / 6.84
+//   K = 3584 (59 MB)  8     12.20 / 10.87, 32: 13.63 / 12.65 10.78 / 10.48, 11.24 / 12.47  10.78 / 9.11, 11.19 / 11.49
+//   K = 5120 (84 MB)  8     16.30 / 14.76, 32: 19.60 / 18.42 14.06 / 14.37, 14.83 / 18.20  14.04 / 13.13, 14.78 / 17.47
+//   K = 7168 (117 MB) 8     21.72 / 19.15, 32: 24.95 / 22.63 21.64 / 18.87, 25.06 / 22.49  18.36 / 17.48, 18.92 / 21.83
+// So the line favours weights that are used again before they leave the cache, and costs products below it 5 to 12 %
+// where they are not; above it, one product repeated on the same weights pays (64 rows: 22.1 / 28.5).
 constexpr int KS_STREAM = 2;  // nt
 constexpr double KS_STREAM_BYTES = 96.0 * 1024 * 1024;
 
@@ -893,12 +904,12 @@ constexpr double KS_STREAM_BYTES = 96.0 * 1024 * 1024;
 // blocks that it has, and two row tiles take even shares of 65 to 96 rows instead of 64 and the rest: the launch
 // ends with its longest workgroup.  us, weights of three or four sets in turn, 64-row tiles / this rule:
 // [40, 1024] x [8192, 1024]^T 5.77 / 5.52, [40, 3584] 11.67 / 11.37, [40, 3696] 13.50 / 12.91, [33, 7168] 23.9 / 22.9,
-// [48, 2048] x [6144, 2048]^T 7.41 / 7.18; [72, 768] x [6144, 768]^T 6.03 / 5.59, [72, 1024] x [8192, 1024]^T 7.05 / 6.64,
-// [72, 3584] 13.53 / 12.52, [96, 1024] 7.14 / 6.93.  Even shares gain while the longest workgroup is the bound; where
-// the L2s and the memory are, they lose: weights past KS_EVEN_BYTES ([80, 7168] 32.6 / 33.0, [72, 5120] 24.5 / 25.3),
-// past 7/8 of it from 73 rows on ([80, 4096] 19.9 / 20.3, weights from memory; [72, 4096] 19.7 / 19.5), past half of it for
-// 48-row tiles ([96, 3584] 13.4 / 13.6), or rows of b that are not whole lines ([80, 3696] 16.0 / 16.5; 48 rows
-// there: 14.2 / 14.5).  56-row tiles are within 1 % either way and are not built.
+// [48, 2048] x [6144, 2048]^T 7.41 / 7.18; [72, 768] x [6144, 768]^T 6.03 / 5.59, [72, 1024] x [8192, 1024]^T 7.05 /
+// 6.64, [72, 3584] 13.53 / 12.52, [96, 1024] 7.14 / 6.93.  Even shares gain while the longest workgroup is the bound;
+// where the L2s and the memory are, they lose: weights past KS_EVEN_BYTES ([80, 7168] 32.6 / 33.0, [72, 5120] 24.5 /
+// 25.3), past 7/8 of it from 73 rows on ([80, 4096] 19.9 / 20.3, weights from memory; [72, 4096] 19.7 / 19.5), past
+// half of it for 48-row tiles ([96, 3584] 13.4 / 13.6), or rows of b that are not whole lines ([80, 3696] 16.0 /
+// 16.5; 48 rows there: 14.2 / 14.5).  56-row tiles are within 1 % either way and are not built.
 //
 // Under a grid cap workgroups walk several tiles and the longest one counts for less: from cold weights, 64-row tiles /
 // even shares, cap 64: [72, 2048] x [8192, 2048]^T 35.5 / 34.9 us, [80, 2048] 35.9 / 36.0, but [80, 2560] 46.2 / 47.5,
@@ -954,7 +965,8 @@ static int launch_ksplit_for(const GemmBatch& batch, int count, int64_t M, int64
   const KsForm f = ksplit_form(M, N, K, count, max_cus, cus);
 #define TW_KSPLIT_LAUNCH(MT, NT, STAGES, LA, STREAM, TAIL)                                                     \
   if (f.mt == MT && f.nt == NT && f.stages == STAGES && f.la == LA && f.stream == STREAM && f.tail == TAIL)      \
-    return launch_ksplit<MT, NT, STAGES, LA, STREAM ? KS_STREAM : 0, TAIL>(batch, count, M, N, K, ldc, max_cus, cus, hs);
+    return launch_ksplit<MT, NT, STAGES, LA, STREAM ? KS_STREAM : 0, TAIL>(batch, count, M, N, K, ldc, max_cus, cus, \
+                                                                           hs);
   TW_KSPLIT_FORMS(TW_KSPLIT_LAUNCH)
 #undef TW_KSPLIT_LAUNCH
   return set_error(TW_ERR_INVALID_ARGUMENT, "gemm_bf16_nt: no kernel for %d rows", (int)M);
@@ -977,23 +989,23 @@ static int launch_tile_kernel(const GemmBatch& batch, int count, int64_t M, int6
   int wide_store = (N % 8 == 0 && ldc % 8 == 0) ? 1 : 0;
   for (int p = 0; p < count; ++p)
     if (reinterpret_cast<uintptr_t>(batch.out[p]) & 15u) wide_store = 0;
-  launch_kernel(gemm_bf16_nt_tile_kernel<TM, TN, ROWS>, dim3((unsigned)grid), dim3(TILE_THREADS), S::LDS, hs, batch, count,
-                (int)M, (int)N, (int)K, ldc, tiles_m, tiles_n, wide_store);
+  launch_kernel(gemm_bf16_nt_tile_kernel<TM, TN, ROWS>, dim3((unsigned)grid), dim3(TILE_THREADS), S::LDS, hs, batch,
+                count, (int)M, (int)N, (int)K, ldc, tiles_m, tiles_n, wide_store);
   return TW_OK;
 }
 
 // Whole lines where the shape's ring has room for the panel more and rows are long: a tile costs 0.8 to 1 us more
 // (one line more to fetch and every row's place in its lines).  us, kPartialSlab / kLines, 8192 columns, weights from
-// memory: [200, 208] 6.1 / 6.9, [200, 528] 8.6 / 8.6, [200, 1040] 12.8 / 11.6, [200, 1552] 17.3 / 14.7; K a multiple of 32,
-// where half as many rows lie on two lines: [200, 544] 8.2 / 8.7, [200, 1056] 11.9 / 11.6, [200, 2080] 19.6 / 17.7.
-// The same weights again and again, from the last-level cache, gain later, and the lines are drawn between the two:
-// [200, 1040] 10.7 / 10.8, [200, 1552] 13.7 / 13.3, [200, 2080] 15.5 / 15.9, [200, 4128] 28.0 / 26.5.  (What the L2s
-// hold is not bound by requests: [129, 2064] x [1024, 2064]^T 11.5 / 14.9; from memory 19.9 / 16.7.)
+// memory: [200, 208] 6.1 / 6.9, [200, 528] 8.6 / 8.6, [200, 1040] 12.8 / 11.6, [200, 1552] 17.3 / 14.7; K a multiple
+// of 32, where half as many rows lie on two lines: [200, 544] 8.2 / 8.7, [200, 1056] 11.9 / 11.6, [200, 2080] 19.6 /
+// 17.7. The same weights again and again, from the last-level cache, gain later, and the lines are drawn between the
+// two: [200, 1040] 10.7 / 10.8, [200, 1552] 13.7 / 13.3, [200, 2080] 15.5 / 15.9, [200, 4128] 28.0 / 26.5.  (What the
+// L2s hold is not bound by requests: [129, 2064] x [1024, 2064]^T 11.5 / 14.9; from memory 19.9 / 16.7.)
 constexpr int64_t LINES_FROM_K = 1280, LINES_FROM_K_32 = 2048;
 
-// The shapes whose ring then is down to the least (TIGHT: 128 x 256 and 96 x 256) cover less of memory's latency and are
-// taken only where more than half of the rows lie on two lines: K = 7392, 128 x 256, 800 and 1000 rows 122 / 138 us with
-// kPartialSlab, 132 / 133 with kLines.
+// The shapes whose ring then is down to the least (TIGHT: 128 x 256 and 96 x 256) cover less of memory's latency and
+// are taken only where more than half of the rows lie on two lines: K = 7392, 128 x 256, 800 and 1000 rows 122 / 138
+// us with kPartialSlab, 132 / 133 with kLines.
 template <int TM, int TN>
 static TileRows tile_rows(int64_t K) {
   if (K % BK == 0) return kWholeSlabs;
@@ -1020,10 +1032,13 @@ static int launch_tile(const GemmBatch& batch, int count, int64_t M, int64_t N, 
 // (M = 2458: 512 tiles) and the 192-wide ones for N = 6144, whose 24 columns of 256 leave a quarter
 // of the units idle; the small ones for M <= 512 at N = 8192 (64 x 128, 96 x 128, 128 x 128: 256
 // tiles for 256, 384 and 512 rows).
-// One column of costs serves every K: of the twelve shapes timed one by one, the picked one is the
-// fastest at 114 of 120 points (15 row counts from 129 to 4096; 8192 columns with K = 1024, 2048, 3584,
-// 3696, 7168, 7392 and 6144 columns with K = 768, 2048), 0.1 % from it on average and 5 % at worst
-// (640 rows, K = 7392: 82 us, 96 x 256 tiles 78).
+// One column of costs serves every K and every way of fetching rows: of the twelve shapes timed one by one, the
+// picked one is the fastest at 112 of 120 points (15 row counts from 129 to 4096; 8192 columns with K = 1024, 2048,
+// 3584, 3696, 7168, 7392 and 6144 columns with K = 768, 2048; three sets of operands in turn), 0.3 % from it on
+// average and 15 % at worst (640 rows, 6144 columns, K = 768: 11.7 us, 96 x 192 tiles 10.2); with weights from memory
+// at 115 points, 0.1 % from it on average and 5 % at worst (2458 rows there: 29.6 us, 192 x 192 tiles 28.3).  At
+// K = 3696 and 7392 it misses at two: 800 rows from memory 70.7 us (128 x 128 tiles 67.9), 1000 rows 138 (160 x 256
+// 133).
 struct TileChoice { int tm, tn; double cost; };
 #define TW_TILES(X)                                                                                            \
   X(8, 8, 1.0) X(6, 8, 0.79) X(8, 6, 0.77) X(5, 8, 0.69) X(6, 6, 0.65) X(4, 8, 0.58) X(3, 8, 0.48) X(4, 6, 0.46) \
