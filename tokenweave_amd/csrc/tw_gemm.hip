@@ -921,9 +921,10 @@ constexpr int64_t KS_EVEN_CAPPED_K = 2048;
 // The instantiations: MT, NT, STAGES, LA, stream, tail.
 #define TW_KSPLIT_ROWS_32(X, LA) \
   X(1, 1, 2, LA, true, false) X(1, 1, 2, LA, false, false) X(1, 1, 2, LA, false, true) \
-  X(1, 1, 3, LA, true, false) X(1, 1, 3, LA, false, false) X(1, 1, 3, LA, false, true)
+  X(1, 1, 3, LA, true, false) X(1, 1, 3, LA, false, false)
 #define TW_KSPLIT_FORMS(X)                                                                                   \
   TW_KSPLIT_ROWS_32(X, 1) TW_KSPLIT_ROWS_32(X, 2) TW_KSPLIT_ROWS_32(X, 4)                                      \
+  X(1, 1, 3, 1, false, true) X(1, 1, 3, 2, false, true)                                                        \
   X(2, 1, 3, 5, true, false) X(2, 1, 3, 5, false, false) X(2, 1, 2, 5, false, true)                            \
   X(2, 1, 2, 6, true, false) X(2, 1, 2, 6, false, false)                                                       \
   X(2, 1, 2, 8, true, false) X(2, 1, 2, 8, false, false) X(2, 1, 2, 8, false, true)                            \
